@@ -735,14 +735,11 @@ __global__ __launch_bounds__(512) void k_grid_bwd(SubParams p, const float4* __r
         }
       }
     }
-    if (!covered) continue;
     // the recorded forward's node state before the update: (momentum / mass, mass)
-    const float4 pre = grid_pre[nid];
+    const float4 pre = covered ? grid_pre[nid] : make_float4(0.f, 0.f, 0.f, 0.f);
     const float mass = pre.w;
-    if (mass < 1e-10f) {
-      grid_adj[nid] = make_float4(0.f, 0.f, 0.f, 0.f);
-      continue;
-    }
+    const bool live = covered && !(mass < 1e-10f);
+    if (covered && !live) grid_adj[nid] = make_float4(0.f, 0.f, 0.f, 0.f);
     // forward recompute (shaders/mpm_grid_update.comp:17-101, mpm_nanovdb_bc.comp:23-54)
     const float u0x = pre.x, u0y = pre.y, u0z = pre.z;
     const float sp = len3(u0x, u0y, u0z);
@@ -751,8 +748,15 @@ __global__ __launch_bounds__(512) void k_grid_bwd(SubParams p, const float4* __r
     if (capped) { const float kk = 15.f / sp; vx *= kk; vy *= kk; vz *= kk; }
     // forces add constants with respect to the state: they pass the adjoint
     // through, but the flags below depend on the velocity they produce
-    apply_forces<NOISE>(vx, vy, vz, (float(nx) + 0.5f) * sg.h + sg.wmin[0], (float(ny) + 0.5f) * sg.h + sg.wmin[1],
-                        (float(nz) + 0.5f) * sg.h + sg.wmin[2], forces, p.force_count, p.dt);
+    if constexpr (NOISE) {
+      __shared__ NoiseLds s_noise;
+      if (!__syncthreads_or(live)) continue;
+      tile_forces(vx, vy, vz, (float(nx) + 0.5f) * sg.h + sg.wmin[0], (float(ny) + 0.5f) * sg.h + sg.wmin[1],
+                  (float(nz) + 0.5f) * sg.h + sg.wmin[2], live, forces, p.force_count, p.dt, s_noise);
+    } else {
+      apply_forces(vx, vy, vz, forces, p.force_count, p.dt);
+    }
+    if (!live) continue;
     const int Nx = sg.grid_res[0] - 1, Ny = sg.grid_res[1] - 1, Nz = sg.grid_res[2] - 1;
     bool wx = false, wy = false, wz = false;
     if (nx <= 1 && vx < 0.f) { vx = 0.f; wx = true; }

@@ -735,25 +735,24 @@ __device__ __forceinline__ bool sum_partials(const SceneGeo& g, int tx, int ty, 
 // in registers and in this order: the 15 m/s cap, the saved (pre-force)
 // velocity, forces, walls, analytic colliders, the dense-SDF BC
 // (shaders/mpm_grid_update.comp:30-110, shaders/mpm_nanovdb_bc.comp:23-54).
-// v enters as momentum / mass; o receives the saved velocity.
-template <bool NOISE>
-__device__ __forceinline__ void node_update(const SubParams& p, const SceneGeo& g, int nx, int ny, int nz,
-                                            float& vx, float& vy, float& vz, float& ox, float& oy, float& oz,
-                                            const float* __restrict__ sdf, const nb_collider* __restrict__ cols,
-                                            const nb_force* __restrict__ forces) {
-  {
-    const float sp = len3(vx, vy, vz);
-    const float vmax = 15.f;
-    if (sp > vmax) {
-      const float k = vmax / sp;
-      vx *= k; vy *= k; vz *= k;
-    }
+// v enters as momentum / mass; o receives the saved velocity.  node_update is
+// the whole of it for force lists without turbulence and noise.
+__device__ __forceinline__ void node_cap(float& vx, float& vy, float& vz) {
+  const float sp = len3(vx, vy, vz);
+  const float vmax = 15.f;
+  if (sp > vmax) {
+    const float k = vmax / sp;
+    vx *= k; vy *= k; vz *= k;
   }
-  ox = vx; oy = vy; oz = vz;
-  const float px = (float(nx) + 0.5f) * g.h + g.wmin[0];
-  const float py = (float(ny) + 0.5f) * g.h + g.wmin[1];
-  const float pz = (float(nz) + 0.5f) * g.h + g.wmin[2];
-  apply_forces<NOISE>(vx, vy, vz, px, py, pz, forces, p.force_count, p.dt);
+}
+__device__ __forceinline__ float3 node_pos(const SceneGeo& g, int nx, int ny, int nz) {
+  return make_float3((float(nx) + 0.5f) * g.h + g.wmin[0], (float(ny) + 0.5f) * g.h + g.wmin[1],
+                     (float(nz) + 0.5f) * g.h + g.wmin[2]);
+}
+// walls, analytic colliders and the dense SDF; (px, py, pz) is the node's position
+__device__ __forceinline__ void node_bc(const SubParams& p, const SceneGeo& g, int nx, int ny, int nz, float px,
+                                        float py, float pz, float& vx, float& vy, float& vz,
+                                        const float* __restrict__ sdf, const nb_collider* __restrict__ cols) {
   // separating walls on the two outer node layers (shaders/mpm_grid_update.comp:54-60)
   const int Nx = g.grid_res[0] - 1, Ny = g.grid_res[1] - 1, Nz = g.grid_res[2] - 1;
   if (nx <= 1 && vx < 0.f) vx = 0.f;
@@ -788,6 +787,16 @@ __device__ __forceinline__ void node_update(const SubParams& p, const SceneGeo& 
     }
   }
 }
+__device__ __forceinline__ void node_update(const SubParams& p, const SceneGeo& g, int nx, int ny, int nz, float& vx,
+                                            float& vy, float& vz, float& ox, float& oy, float& oz,
+                                            const float* __restrict__ sdf, const nb_collider* __restrict__ cols,
+                                            const nb_force* __restrict__ forces) {
+  node_cap(vx, vy, vz);
+  ox = vx; oy = vy; oz = vz;
+  const float3 x = node_pos(g, nx, ny, nz);
+  apply_forces(vx, vy, vz, forces, p.force_count, p.dt);
+  node_bc(p, g, nx, ny, nz, x.x, x.y, x.z, vx, vy, vz, sdf, cols);
+}
 
 template <bool FROM_PARTIALS, bool UPDATE, bool BATCH, bool NOISE>
 __global__ __launch_bounds__(512) void k_grid(SubParams p, const float4* __restrict__ partial,
@@ -807,26 +816,43 @@ __global__ __launch_bounds__(512) void k_grid(SubParams p, const float4* __restr
     tile_coords(g, N, tx, ty, tz);
     const int nx = tx * 8 + lx, ny = ty * 8 + ly, nz = tz * 8 + lz;
     const size_t nid = (size_t(N) << kTileBits) | threadIdx.x;
-    float mx, my, mz, mass;
+    float mx = 0.f, my = 0.f, mz = 0.f, mass = 0.f;
+    // A node outside every occupied tile's box receives nothing and lies in
+    // no particle's stencil: it is not written (readers treat it as empty).
+    bool covered = true;
     if (FROM_PARTIALS) {
-      // A node outside every occupied tile's box receives nothing and lies in
-      // no particle's stencil: it is not written (readers treat it as empty).
-      if (!sum_partials(g, tx, ty, tz, lx, ly, lz, tile_act, partial, mx, my, mz, mass)) continue;
+      covered = sum_partials(g, tx, ty, tz, lx, ly, lz, tile_act, partial, mx, my, mz, mass);
     } else {
       const float4 g4 = grid_node[nid];
       mx = g4.x; my = g4.y; mz = g4.z; mass = g4.w;
     }
-    if (grid_pre)
+    if (covered && grid_pre)
       grid_pre[nid] = mass < 1e-10f ? make_float4(0.f, 0.f, 0.f, mass) : make_float4(mx / mass, my / mass, mz / mass, mass);
-    if (!UPDATE || mass < 1e-10f) {
-      // massless nodes keep their momentum (shaders/mpm_grid_update.comp:109-110)
-      grid_node[nid] = make_float4(mx, my, mz, mass);
-      continue;
+    const bool live = covered && UPDATE && !(mass < 1e-10f);
+    // massless nodes keep their momentum (shaders/mpm_grid_update.comp:109-110)
+    if (covered && !live) grid_node[nid] = make_float4(mx, my, mz, mass);
+    if constexpr (NOISE) {
+      // the block's threads share the noise's lattice points (tile_forces)
+      __shared__ NoiseLds s_noise;
+      if (!__syncthreads_or(live)) continue;
+      float vx = 0.f, vy = 0.f, vz = 0.f;
+      if (live) {
+        vx = mx / mass; vy = my / mass; vz = mz / mass;
+        node_cap(vx, vy, vz);
+        if (p.write_old) grid_old[nid] = make_float4(vx, vy, vz, 0.f);
+      }
+      const float3 x = node_pos(g, nx, ny, nz);
+      tile_forces(vx, vy, vz, x.x, x.y, x.z, live, forces, p.force_count, p.dt, s_noise);
+      if (live) {
+        node_bc(p, g, nx, ny, nz, x.x, x.y, x.z, vx, vy, vz, sdf, cols);
+        grid_node[nid] = make_float4(vx, vy, vz, mass);
+      }
+    } else if (live) {
+      float vx = mx / mass, vy = my / mass, vz = mz / mass, ox, oy, oz;
+      node_update(p, g, nx, ny, nz, vx, vy, vz, ox, oy, oz, sdf, cols, forces);
+      if (p.write_old) grid_old[nid] = make_float4(ox, oy, oz, 0.f);
+      grid_node[nid] = make_float4(vx, vy, vz, mass);
     }
-    float vx = mx / mass, vy = my / mass, vz = mz / mass, ox, oy, oz;
-    node_update<NOISE>(p, g, nx, ny, nz, vx, vy, vz, ox, oy, oz, sdf, cols, forces);
-    if (p.write_old) grid_old[nid] = make_float4(ox, oy, oz, 0.f);
-    grid_node[nid] = make_float4(vx, vy, vz, mass);
   }
 }
 
@@ -1486,7 +1512,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         (void)sum_partials(g, ntx, nty, ntz, nx & 7, ny & 7, nz & 7, tile_act, partial, mx, my, mz, mass);
         if (mass >= 1e-10f) {
           float vx = mx / mass, vy = my / mass, vz = mz / mass, ox, oy, oz;
-          node_update<false>(p, g, nx, ny, nz, vx, vy, vz, ox, oy, oz, sdf, cols, forces);
+          node_update(p, g, nx, ny, nz, vx, vy, vz, ox, oy, oz, sdf, cols, forces);
           v = make_float4(vx, vy, vz, 1.f);
           o = make_float4(ox, oy, oz, 0.f);
         }
