@@ -482,7 +482,7 @@ int nb_mpm_active_tile_count(nb_mpm* h, uint32_t* tiles);
  * d_params.  The engine is left in the state the recorded run ended in (its
  * grid is not kept: nb_mpm_get_grid needs another substep first).
  * Memory: per particle of capacity (ceil(n/segment) + segment - 1) x 132 B
- * (records and bin keys of the kept states) + segment x 8 B (each substep's
+ * (records and bin keys of the kept states) + segment x 4 B (each substep's
  * sorted order) + 480 B; per grid node segment x 40 B (each substep's grid
  * and cell counts, kept so that the backward does not bin again or redo P2G
  * and the grid update) + 32 B. */

@@ -83,10 +83,14 @@ struct nb_mpm {
   // reference layout d.field.  rec_stale: the API wrote d.field since the
   // records were last filled.  ptr_exported: device pointers to d.field were
   // handed out, so the caller may write them between calls.  keys_valid: the
-  // last G2P wrote every live particle's cell key and nothing moved since.
+  // last G2P wrote every live particle's cell key and nothing moved since;
+  // counted: and counted them into their tiles.  counts_dirty: d.tile_cnt is
+  // not zero (counted, or counts of a state that was replaced).
   bool rec_stale = true;
   bool ptr_exported = false;
   bool keys_valid = false;
+  bool counted = false;
+  bool counts_dirty = false;
   GridMode grid_mode = GridMode::NONE;
   bool old_valid = false;
   std::vector<void*> allocs;
@@ -255,7 +259,7 @@ int sync_in(nb_mpm* h) {
   if ((h->rec_stale || h->ptr_exported) && h->n_live) {
     launch_soa_to_aos(h->d, h->n_live, h->stream);
     NB_HIP(hipGetLastError());
-    h->keys_valid = false;
+    h->keys_valid = h->counted = false;
   }
   h->rec_stale = false;
   return NB_OK;
@@ -270,6 +274,14 @@ int sync_out(nb_mpm* h) {
   return NB_OK;
 }
 
+// The bin of dv's records, from as much as the last G2P left of it.
+void bin(nb_mpm* h, const DevState& dv, const SubParams& p, Prof* pf) {
+  const BinFrom from = !h->keys_valid ? BinFrom::RECORDS : (h->counted ? BinFrom::COUNTED : BinFrom::KEYS);
+  if (from != BinFrom::COUNTED && h->counts_dirty) launch_clear_counts(dv, h->NT, h->stream);
+  launch_bin(dv, p, h->NT, from, h->stream, pf);
+  h->counted = h->counts_dirty = false;
+}
+
 // one substep on the records (the caller brackets a run of them with
 // sync_in / sync_out)
 // Where a recorded substep reads and writes: records and bin keys before
@@ -278,13 +290,9 @@ int sync_out(nb_mpm* h) {
 // stops after the grid update.
 // the bin buffers of dv replaced by those of b
 void use_bins(DevState& dv, const DevState& b) {
-  dv.rank = b.rank;
   dv.sorted = b.sorted;
   dv.cell_count = b.cell_count;
   dv.cell_end = b.cell_end;
-  dv.tile_flag = b.tile_flag;
-  dv.tile_mark = b.tile_mark;
-  dv.blk_cnt = b.blk_cnt;
   dv.tile_act = b.tile_act;
   dv.act_tiles = b.act_tiles;
   dv.node_tiles = b.node_tiles;
@@ -305,22 +313,27 @@ struct TapeIO {
   const DevState* bins = nullptr;  // bin buffers to use instead of the engine's
 };
 
-// One substep.  fused: the grid update runs inside G2P (k_g2p_tile) and the
+// One substep.  last: the call's last, so the FP64 fallback's queue is worked
+// off at its end (the next substep's bin does it otherwise); if the caller may
+// write the state before the next call, its particles are not counted for a
+// bin that would not use the counts.  fused: the grid update runs inside G2P (k_g2p_tile) and the
 // grid arrays are left unwritten; only for plain substeps with no tape, and
 // the same results bit for bit.
-int enqueue_substep(nb_mpm* h, float dt, Prof* pf, const TapeIO& io = TapeIO{}, bool fused = false) {
+int enqueue_substep(nb_mpm* h, float dt, Prof* pf, bool last, const TapeIO& io = TapeIO{},
+                    bool fused = false) {
   if (h->n_live == 0) return NB_OK;
   const bool flip = h->knobs.flip_ratio > 0.01f;
   SubParams p = h->params(dt, flip);
   DevState dv = h->dev();
   if (fused && p.noise_forces == 0 && !io.bins && !io.rec_in && !io.keys_in && !io.grid_node && !io.grid_pre &&
       io.g2p && !io.keys_out && !io.rec_out) {
-    launch_bin(dv, p, h->NT, h->keys_valid, h->stream, pf);
+    bin(h, dv, p, pf);
     launch_p2g(dv, p, h->NT, h->stream, pf);
     launch_g2p_fused(dv, p, h->NT, h->stream, pf);
+    if (last) launch_g2p_fb(dv, p, dv.rec, h->stream, pf);
     NB_HIP(hipGetLastError());
     h->bins_valid = true;
-    h->keys_valid = true;
+    h->keys_valid = h->counted = h->counts_dirty = true;
     h->grid_mode = GridMode::NONE;  // the fused substep keeps its grid in LDS
     h->old_valid = false;
     return NB_OK;
@@ -330,7 +343,7 @@ int enqueue_substep(nb_mpm* h, float dt, Prof* pf, const TapeIO& io = TapeIO{}, 
   if (io.keys_in) dv.keys = io.keys_in;
   if (io.grid_node) dv.grid_node = io.grid_node;
   dv.grid_pre = io.grid_pre;
-  launch_bin(dv, p, h->NT, h->keys_valid, h->stream, pf);
+  bin(h, dv, p, pf);
   launch_p2g(dv, p, h->NT, h->stream, pf);
   launch_grid(dv, p, h->NT, true, true, dv.node_tiles, dv.counters + CNT_NODE_TILES, h->stream, pf);
   if (!io.g2p) {
@@ -340,10 +353,13 @@ int enqueue_substep(nb_mpm* h, float dt, Prof* pf, const TapeIO& io = TapeIO{}, 
     return NB_OK;
   }
   dv.keys = io.keys_out ? io.keys_out : h->d.keys;  // G2P writes the next substep's keys
-  launch_g2p(dv, p, true, h->stream, pf, io.rec_out);
+  const bool count = !(last && h->ptr_exported);
+  launch_g2p(dv, p, true, count, h->stream, pf, io.rec_out);
+  if (last) launch_g2p_fb(dv, p, io.rec_out ? io.rec_out : dv.rec, h->stream, pf);
   NB_HIP(hipGetLastError());
   h->bins_valid = true;
   h->keys_valid = true;
+  h->counted = h->counts_dirty = count;
   h->grid_mode = GridMode::SPARSE;
   h->old_valid = flip;
   return NB_OK;
@@ -358,7 +374,7 @@ int run_substeps(nb_mpm* h, float dt, uint32_t n, Prof* pf) {
   // writes the grid, so that the grid a caller reads after the call is the
   // last substep's, as after the reference's step
   for (uint32_t i = 0; i < n && rc == NB_OK; i++)
-    rc = enqueue_substep(h, dt, pf, TapeIO{}, h->fuse_g2p && i + 1 < n);
+    rc = enqueue_substep(h, dt, pf, i + 1 == n, TapeIO{}, h->fuse_g2p && i + 1 < n);
   if (rc == NB_OK) rc = sync_out(h);
   return rc;
 }
@@ -625,9 +641,10 @@ int engine_alloc(nb_mpm* h, void* hip_stream) {
   if (rc == NB_OK) rc = h->alloc(&d.sorted, h->cap);
   if (rc == NB_OK) rc = h->alloc(&d.cell_count, cells);
   if (rc == NB_OK) rc = h->alloc(&d.cell_end, cells);
-  if (rc == NB_OK) rc = h->alloc(&d.tile_flag, h->NT);
+  if (rc == NB_OK) rc = h->alloc(&d.bucket, h->cap);
+  if (rc == NB_OK) rc = h->alloc(&d.tile_cnt, h->NT);
   if (rc == NB_OK) rc = h->alloc(&d.tile_mark, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&d.blk_cnt, (h->NT + 255) / 256);
+  if (rc == NB_OK) rc = h->alloc(&d.tile_sums, (h->NT + 255) / 256 + 1);
   if (rc == NB_OK) rc = h->alloc(&d.tile_act, h->NT);
   if (rc == NB_OK) rc = h->alloc(&d.act_tiles, h->NT);
   if (rc == NB_OK) rc = h->alloc(&d.node_tiles, h->NT);
@@ -651,7 +668,7 @@ int engine_alloc(nb_mpm* h, void* hip_stream) {
 
   auto zero = [&](void* p, size_t bytes) { return hipMemsetAsync(p, 0, bytes, h->stream); };
   if (zero(d.cell_count, cells * 4) != hipSuccess || zero(d.cell_end, cells * 4) != hipSuccess ||
-      zero(d.tile_flag, h->NT) != hipSuccess || zero(d.counters, CNT_SLOTS * 4) != hipSuccess ||
+      zero(d.tile_cnt, size_t(h->NT) * 4) != hipSuccess || zero(d.counters, CNT_SLOTS * 4) != hipSuccess ||
       zero(d.grid_node, cells * 16) != hipSuccess || zero(d.grid_old, cells * 16) != hipSuccess ||
       zero(d.materials, size_t(h->max_materials()) * 64) != hipSuccess ||
       zero(d.colliders, NB_MAX_COLLIDERS * 64) != hipSuccess || zero(d.forces, NB_MAX_FORCES * 32) != hipSuccess ||
@@ -745,9 +762,10 @@ int nb_mpm_graph_substeps(nb_mpm* h, float dt_sub, uint32_t n) {
   if (!h) return fail(NB_ERR_ARG, "null handle");
   if (n == 0 || h->n_live == 0) return NB_OK;
   int rc = sync_in(h);
-  // the captured substep reads the keys the previous G2P wrote
-  if (rc == NB_OK && !h->keys_valid) {
-    rc = enqueue_substep(h, dt_sub, nullptr);
+  // the captured substep starts from the keys and counts the previous G2P left
+  // and leaves the same, and the fallback's queue, to the next
+  if (rc == NB_OK && !(h->keys_valid && h->counted)) {
+    rc = enqueue_substep(h, dt_sub, nullptr, n == 1);
     n--;
   }
   if (rc == NB_OK && n) {
@@ -760,7 +778,7 @@ int nb_mpm_graph_substeps(nb_mpm* h, float dt_sub, uint32_t n) {
         h->graph_exec = nullptr;
       }
       NB_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-      rc = enqueue_substep(h, dt_sub, nullptr);
+      rc = enqueue_substep(h, dt_sub, nullptr, false);
       hipGraph_t g = nullptr;
       const hipError_t e = hipStreamEndCapture(h->stream, &g);
       if (rc != NB_OK || e != hipSuccess) {
@@ -777,6 +795,8 @@ int nb_mpm_graph_substeps(nb_mpm* h, float dt_sub, uint32_t n) {
       h->graph_d = dv;
     }
     for (uint32_t i = 0; i < n; i++) NB_HIP(hipGraphLaunch(h->graph_exec, h->stream));
+    launch_g2p_fb(dv, p, dv.rec, h->stream, nullptr);
+    NB_HIP(hipGetLastError());
   }
   if (rc == NB_OK) rc = sync_out(h);
   return rc;
@@ -814,14 +834,15 @@ int nb_mpm_autotune(nb_mpm* h, float dt_sub, uint32_t trial_substeps, uint32_t f
   auto restore = [&]() {
     ok = ok && copy(h->d.rec, save_rec, rec_bytes) && copy(h->d.keys, save_keys, key_bytes);
     h->keys_valid = keys0;
+    h->counted = false;
   };
   // one trial: from the saved state, one warm substep, then reps timed
   auto trial = [&](const nb_mpm_tuning& t) -> float {
     h->tuning = t;
     restore();
-    int r = enqueue_substep(h, dt_sub, nullptr);
+    int r = enqueue_substep(h, dt_sub, nullptr, false);
     ok = ok && r == NB_OK && hipEventRecord(e0, h->stream) == hipSuccess;
-    for (uint32_t i = 0; i < reps && ok; i++) ok = enqueue_substep(h, dt_sub, nullptr) == NB_OK;
+    for (uint32_t i = 0; i < reps && ok; i++) ok = enqueue_substep(h, dt_sub, nullptr, i + 1 == reps) == NB_OK;
     ok = ok && hipEventRecord(e1, h->stream) == hipSuccess && hipEventSynchronize(e1) == hipSuccess;
     float ms = 0.f;
     ok = ok && hipEventElapsedTime(&ms, e0, e1) == hipSuccess;
@@ -889,7 +910,7 @@ namespace {
 // Bins of the current state (plain engine or batch), for the occupied-tile count.
 int launch_bin_only(nb_mpm* h) {
   SubParams p = h->params(0.f, false);
-  launch_bin(h->dev(), p, h->NT, h->keys_valid, h->stream, nullptr);
+  bin(h, h->dev(), p, nullptr);
   NB_HIP(hipGetLastError());
   NB_HIP(hipStreamSynchronize(h->stream));
   h->bins_valid = true;
@@ -1323,7 +1344,12 @@ int nb_mpm_run_bin(nb_mpm* h) {
   SubParams p = h->params(0.f, false);
   int rc = sync_in(h);
   if (rc != NB_OK) return rc;
-  if (h->n_live) launch_bin(h->dev(), p, h->NT, false, h->stream, nullptr);
+  if (h->n_live) {
+    const bool keys = h->keys_valid;
+    h->keys_valid = false;  // always from the records
+    bin(h, h->dev(), p, nullptr);
+    h->keys_valid = keys;
+  }
   NB_HIP(hipGetLastError());
   NB_HIP(hipStreamSynchronize(h->stream));
   h->bins_valid = true;
@@ -1344,6 +1370,11 @@ int nb_mpm_get_bins(nb_mpm* h, uint32_t* keys, uint32_t* sorted, uint32_t* cell_
     if (n) {
       if ((rc = download(h, cnt.data(), h->d.cell_count, size_t(h->NC) * 4)) != NB_OK) return rc;
       if ((rc = download(h, dev_end.data(), h->d.cell_end, size_t(h->NC) * 4)) != NB_OK) return rc;
+      // the device's counts are those of the occupied tiles only
+      std::vector<int32_t> act(h->NT);
+      if ((rc = download(h, act.data(), h->d.tile_act, size_t(h->NT) * 4)) != NB_OK) return rc;
+      for (uint32_t c = 0; c < h->NC; c++)
+        if (act[c >> kTileBits] < 0) cnt[c] = 0u;
     }
     if (cell_count) std::memcpy(cell_count, cnt.data(), size_t(h->NC) * 4);
     if (cell_end) {
@@ -1398,12 +1429,16 @@ int nb_mpm_run_g2p(nb_mpm* h, float dt_sub) {
   SubParams p = h->params(dt_sub, false);
   int rc = sync_in(h);
   if (rc != NB_OK) return rc;
-  if (h->n_live) launch_g2p(h->dev(), p, h->bins_valid, h->stream, nullptr);
+  if (h->n_live) {
+    launch_g2p(h->dev(), p, h->bins_valid, false, h->stream, nullptr);
+    launch_g2p_fb(h->dev(), p, h->d.rec, h->stream, nullptr);
+  }
   NB_HIP(hipGetLastError());
   if ((rc = sync_out(h)) != NB_OK) return rc;
   NB_HIP(hipStreamSynchronize(h->stream));
   h->bins_valid = false;  // positions moved
   h->keys_valid = h->n_live != 0;
+  h->counted = false;
   return NB_OK;
 }
 
@@ -1599,13 +1634,9 @@ int adj_alloc(nb_mpm* h, T** p, size_t count) {
 int adj_alloc_bins(nb_mpm* h, DevState& b) {
   const size_t cells = size_t(h->NT) * kTileCells;
   int rc = NB_OK;
-  if (rc == NB_OK) rc = adj_alloc(h, &b.rank, h->cap);
   if (rc == NB_OK) rc = adj_alloc(h, &b.sorted, h->cap);
   if (rc == NB_OK) rc = adj_alloc(h, &b.cell_count, cells);
   if (rc == NB_OK) rc = adj_alloc(h, &b.cell_end, cells);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.tile_flag, h->NT);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.tile_mark, h->NT);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.blk_cnt, (h->NT + 255) / 256);
   if (rc == NB_OK) rc = adj_alloc(h, &b.tile_act, h->NT);
   if (rc == NB_OK) rc = adj_alloc(h, &b.act_tiles, h->NT);
   if (rc == NB_OK) rc = adj_alloc(h, &b.node_tiles, h->NT);
@@ -1614,10 +1645,7 @@ int adj_alloc_bins(nb_mpm* h, DevState& b) {
   if (rc == NB_OK) rc = adj_alloc(h, &b.tile_order, h->NT);
   if (rc == NB_OK) rc = adj_alloc(h, &b.counters, CNT_SLOTS);
   if (rc == NB_OK &&
-      (hipMemsetAsync(b.cell_count, 0, cells * 4, h->stream) != hipSuccess ||
-       hipMemsetAsync(b.cell_end, 0, cells * 4, h->stream) != hipSuccess ||
-       hipMemsetAsync(b.tile_flag, 0, h->NT, h->stream) != hipSuccess ||
-       hipMemsetAsync(b.counters, 0, CNT_SLOTS * 4, h->stream) != hipSuccess ||
+      (hipMemsetAsync(b.counters, 0, CNT_SLOTS * 4, h->stream) != hipSuccess ||
        hipMemsetAsync(b.tile_act, 0xFF, size_t(h->NT) * 4, h->stream) != hipSuccess))
     rc = fail(NB_ERR_HIP, "hipMemsetAsync failed");
   if (rc == NB_OK) launch_fill_identity(b.tile_order, h->NT, h->stream);
@@ -1703,7 +1731,7 @@ int nb_mpm_adjoint_begin_tapes(nb_mpm* h, uint32_t n_substeps, uint32_t segment,
     // tenth of it left over
     const size_t cells = size_t(h->NT) * kTileCells;
     const size_t per_tape = size_t(A.seg - 1) * (rec * sizeof(float4) + size_t(h->cap) * 4) +
-                            size_t(A.seg) * (2 * cells * sizeof(float4) + 2 * cells * 4 + size_t(h->cap) * 8 +
+                            size_t(A.seg) * (2 * cells * sizeof(float4) + 2 * cells * 4 + size_t(h->cap) * 4 +
                                              size_t(h->NT) * 40);
     size_t free_b = 0, total_b = 0;
     NB_HIP(hipMemGetInfo(&free_b, &total_b));
@@ -1769,9 +1797,9 @@ int nb_mpm_forward_recorded(nb_mpm* h, float dt_sub) {
   if (!A.on) return fail(NB_ERR_STATE, "call nb_mpm_adjoint_begin first");
   int rc = sync_in(h);
   if (rc == NB_OK) rc = copy_rec(h, A.ckpt, h->d.rec);
-  h->keys_valid = false;  // the first substep writes its keys into the first key slot
+  h->keys_valid = h->counted = false;  // the first substep writes its keys into the first key slot
   for (uint32_t s = 0; s < A.n && rc == NB_OK; s++)
-    rc = enqueue_substep(h, dt_sub, nullptr, tape_io(h, s, adj_next(h, s), key_next(h, s)));
+    rc = enqueue_substep(h, dt_sub, nullptr, s + 1 == A.n, tape_io(h, s, adj_next(h, s), key_next(h, s)));
   h->grid_mode = GridMode::NONE;  // the grids went to the tape
   h->bins_valid = false;          // and the bins to the tape's bin buffers
   if (rc == NB_OK) rc = sync_out(h);
@@ -1828,11 +1856,12 @@ int nb_mpm_backward(nb_mpm* h, float* d_params, uint32_t params_cap) {
       // recompute the segment's records and grids from its checkpoint (its
       // last substep only up to the grid update: its result is the next checkpoint)
       h->keys_valid = true;
+      h->counted = false;
       for (uint32_t j = 0; j < len && rc == NB_OK; j++) {
         const bool last = j + 1 == len;
         TapeIO io = tape_io(h, s0 + j, last ? nullptr : adj_slot(h, s0 + j + 1), last ? nullptr : key_slot(h, s0 + j + 1));
         io.g2p = !last;
-        rc = enqueue_substep(h, A.dt, nullptr, io);
+        rc = enqueue_substep(h, A.dt, nullptr, false, io);
       }
       A.tape_seg[tape_of(h, uint32_t(sg))] = sg;
     }
@@ -1856,7 +1885,7 @@ int nb_mpm_backward(nb_mpm* h, float* d_params, uint32_t params_cap) {
   launch_aos_to_soa_ptrs(in, adj_fields(h), h->n_live, h->stream);
   // the engine's records still hold the state the recorded run ended in; the
   // bins, keys and grid are those of an earlier substep
-  h->keys_valid = false;
+  h->keys_valid = h->counted = false;
   h->bins_valid = false;
   h->grid_mode = GridMode::NONE;
   if (d_params) {

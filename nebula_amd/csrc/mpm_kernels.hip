@@ -2,8 +2,8 @@
 //
 // One substep (the reference's 11 dispatches, src/engine/MPMEngine.cpp:415-473)
 // runs here as:
-//   bin   k_bin_clear -> k_bin_keys -> k_bin_mark -> k_bin_compact ->
-//         k_bin_tile_scan -> k_bin_tile_offsets -> k_bin_scatter -> k_bin_stabilize
+//   bin   (count in the previous G2P, or k_bin_keys) -> k_bin_tiles (or
+//         k_bin_mark -> k_bin_compact) -> k_bin_scatter -> k_bin_sort
 //         (replaces zero_cells, mpm_hash_count, hash_scan_local/global,
 //          hash_add_base, mpm_hash_sort; output is bit-identical to the stable
 //          counting sort with END offsets of tests/helpers/MPMHarness.cpp:132-178,
@@ -38,297 +38,218 @@
 namespace nb {
 
 const char* const kKernelNames[kNumProfiledKernels] = {
-    "bin_clear", "bin_keys", "bin_mark", "bin_compact", "bin_tile_scan",
-    "bin_tile_offsets", "bin_scatter", "bin_stabilize", "p2g", "grid_update", "g2p", "g2p_grid", "g2p_fb"};
+    "bin_keys", "bin_tiles", "bin_compact", "bin_scatter", "bin_sort", "p2g", "grid_update", "g2p", "g2p_grid", "g2p_fb"};
 
 // ---------------------------------------------------------------------------
 // BIN
 // ---------------------------------------------------------------------------
-// Zero the dense cell counters of the tiles the previous bin occupied; outside
-// those tiles the counters are already zero.
-__global__ __launch_bounds__(512) void k_bin_clear(uint32_t* __restrict__ cell_count,
-                                                   const uint32_t* __restrict__ act_tiles,
-                                                   const uint32_t* __restrict__ counters) {
-  const uint32_t na = counters[CNT_ACTIVE];
-  for (uint32_t a = blockIdx.x; a < na; a += gridDim.x) {
-    cell_count[(size_t(act_tiles[a]) << kTileBits) + threadIdx.x] = 0u;
-  }
-}
+// The stable counting sort of the particles by cell, in two levels:
+//   count    particles per tile, and each particle's place in its tile, by one
+//            atomic per distinct tile of a wave: in G2P for the next substep
+//            (its waves hold neighbours, one or two tiles each), or in
+//            k_bin_keys when the state came from elsewhere
+//   tiles    k_bin_tiles, or k_bin_mark + k_bin_compact for large cubes: the
+//            ordered lists of occupied tiles and node tiles, each tile's first
+//            slot, P2G's tile order
+//   scatter  k_bin_scatter: every particle into its tile's range, any order
+//   sort     k_bin_sort: one block per occupied tile counts its cells in LDS
+//            and puts the tile's particles in (cell, index) order
+// No counter per cell in memory: nothing to clear, and the atomics go to a few
+// counters per wave.  Against a count per cell (clear, keys, mark, compact,
+// tile scan, tile offsets, scatter, stabilize: eight launches of 2.5-5 us of
+// stream time each where the work itself is less) the bin of 4,096 particles
+// went from 27 to 12.5 us of a substep; with the FP64 fallback's fix-up, which
+// now runs beside it, from 56 to 34 for 262,144 and from 121 to 73 for 4.19 M
+// (the count adds 2 and 12 us to G2P there).
 
-// Key of every particle (computed from the record, or read when the previous
-// G2P wrote it), its rank among equal keys (wave-aggregated atomics: one
-// atomic per distinct key per wave), and the occupied-tile flags.
-template <bool FROM_REC, bool BATCH>
-__global__ __launch_bounds__(256) void k_bin_keys(SubParams p, const float4* __restrict__ rec,
-                                                  uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
-                                                  uint32_t* __restrict__ cell_count, uint8_t* __restrict__ tile_flag) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool valid = i < p.n;
-  uint32_t key = 0xFFFFFFFFu;
-  if (valid) {
-    if (FROM_REC) {
-      const float4 x = rec[size_t(i) * kRec + R_P];
-      key = cell_key(particle_geo<BATCH>(p, i), x.x, x.y, x.z);
-      keys[i] = key;
-    } else {
-      key = keys[i];
-    }
-  }
-  // group the wave's lanes by key (ballots only), then one atomic per group,
-  // all groups in the same instruction
-  const uint32_t lane = threadIdx.x & 63;
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  uint64_t pending = __ballot(valid);
-  int my_leader = 0;
-  uint32_t my_pos = 0, my_cnt = 0;
+// One particle counted into its tile; returns its place there.  One atomic per
+// distinct tile among the active lanes.
+__device__ __forceinline__ uint32_t count_in_tile(uint32_t key, uint32_t* __restrict__ tile_cnt) {
+  const uint32_t tile = key >> kTileBits;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint64_t below = (1ull << lane) - 1ull;
+  uint64_t pending = __ballot(true);
+  int leader_of = 0;
+  uint32_t place = 0, cnt = 0;
   while (pending) {
     const int leader = __ffsll((unsigned long long)pending) - 1;
-    const uint32_t lkey = __shfl(key, leader);
-    const uint64_t peers = __ballot(valid && key == lkey);
-    if (valid && key == lkey) {
-      my_leader = leader;
-      my_pos = uint32_t(__popcll(peers & lt_mask));
+    const bool mine = tile == uint32_t(__shfl(int(tile), leader));
+    const uint64_t peers = __ballot(mine);
+    if (mine) {
+      leader_of = leader;
+      place = uint32_t(__popcll(peers & below));
     }
-    if (int(lane) == leader) my_cnt = uint32_t(__popcll(peers));
+    if (int(lane) == leader) cnt = uint32_t(__popcll(peers));
     pending &= ~peers;
   }
   uint32_t base = 0;
-  if (valid && my_pos == 0u) {
-    base = atomicAdd(&cell_count[key], my_cnt);
-    tile_flag[key >> kTileBits] = 1;
-  }
-  base = __shfl(base, my_leader);
-  if (valid) rank[i] = base + my_pos;
+  if (place == 0u) base = atomicAdd(&tile_cnt[tile], cnt);
+  return uint32_t(__shfl(int(base), leader_of)) + place;
 }
 
-// Per tile: bit0 = occupied, bit1 = some tile in its 3x3x3 neighbourhood is
-// occupied (its nodes can receive mass).  Each block of 256 tiles also stores
-// its counts of both kinds (occupied in the low, node tiles in the high half).
-template <bool BATCH>
-__global__ __launch_bounds__(256) void k_bin_mark(SubParams p, const uint8_t* __restrict__ tile_flag,
-                                                  uint8_t* __restrict__ tile_mark, uint64_t* __restrict__ blk_cnt,
-                                                  uint32_t nt) {
-  __shared__ uint64_t s_scan[256 / 64 + 1];
-  const uint32_t T = blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t m = 0;
-  if (T < nt) {
-    const SceneGeo g = tile_geo<BATCH>(p, T);  // neighbours stay inside the tile's scene
-    int tx, ty, tz;
-    tile_coords(g, T, tx, ty, tz);
-    const int td = int(g.tile_dim);
-    uint8_t node = 0;
-    for (int dz = -1; dz <= 1; dz++)
-      for (int dy = -1; dy <= 1; dy++)
-        for (int dx = -1; dx <= 1; dx++) {
-          int x = tx + dx, y = ty + dy, z = tz + dz;
-          if (x < 0 || y < 0 || z < 0 || x >= td || y >= td || z >= td) continue;
-          node |= tile_flag[tile_id(g, x, y, z)];
-        }
-    m = (tile_flag[T] ? 1u : 0u) | (node ? 2u : 0u);
-    tile_mark[T] = uint8_t(m);
-  }
-  uint64_t tot;
-  (void)block_exclusive_scan<256>(uint64_t(m & 1u) | (uint64_t(m >> 1) << 32), s_scan, tot);
-  if (threadIdx.x == 0) blk_cnt[blockIdx.x] = tot;
-}
-
-// Ordered compaction of occupied tiles and node tiles, one block per 256
-// tiles: the block's offsets are the sums of the counts of the blocks before
-// it; resets the occupied flags for the next bin.
-__global__ __launch_bounds__(256) void k_bin_compact(const uint8_t* __restrict__ tile_mark,
-                                                     const uint64_t* __restrict__ blk_cnt,
-                                                     uint8_t* __restrict__ tile_flag, int32_t* __restrict__ tile_act,
-                                                     uint32_t* __restrict__ act_tiles,
-                                                     uint32_t* __restrict__ node_tiles,
-                                                     uint32_t* __restrict__ counters, uint32_t nt) {
-  __shared__ uint64_t s_scan[256 / 64 + 1];
-  uint64_t before = 0;
-  for (uint32_t i = threadIdx.x; i < blockIdx.x; i += blockDim.x) before += blk_cnt[i];
-  uint64_t off;
-  (void)block_exclusive_scan<256>(before, s_scan, off);
-  const uint32_t T = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t m = T < nt ? tile_mark[T] : 0u;
-  uint64_t tot;
-  const uint64_t pre = block_exclusive_scan<256>(uint64_t(m & 1u) | (uint64_t(m >> 1) << 32), s_scan, tot);
-  const uint32_t oa = uint32_t(off) + uint32_t(pre), on = uint32_t(off >> 32) + uint32_t(pre >> 32);
-  if (T < nt) {
-    if (m & 1u) act_tiles[oa] = T;
-    tile_act[T] = (m & 1u) ? int32_t(oa) : -1;
-    if (m & 2u) node_tiles[on] = T;
-    tile_flag[T] = 0;
-  }
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
-    counters[CNT_ACTIVE] = uint32_t(off) + uint32_t(tot);
-    counters[CNT_NODE_TILES] = uint32_t(off >> 32) + uint32_t(tot >> 32);
-  }
-}
-
-// Per occupied tile: exclusive scan of its 512 cell counts (local cell start,
-// kept in cell_end until the scatter) and the tile total.
-__global__ __launch_bounds__(512) void k_bin_tile_scan(const uint32_t* __restrict__ cell_count,
-                                                       uint32_t* __restrict__ cell_end,
-                                                       const uint32_t* __restrict__ act_tiles,
-                                                       uint32_t* __restrict__ tile_total,
-                                                       const uint32_t* __restrict__ counters) {
-  __shared__ uint32_t s_wave[512 / 64 + 1];
-  const uint32_t na = counters[CNT_ACTIVE];
-  for (uint32_t a = blockIdx.x; a < na; a += gridDim.x) {
-    const size_t key = (size_t(act_tiles[a]) << kTileBits) + threadIdx.x;
-    uint32_t c = cell_count[key];
-    uint32_t tot;
-    uint32_t ex = block_exclusive_scan<512>(c, s_wave, tot);
-    cell_end[key] = ex;
-    if (threadIdx.x == 0) tile_total[a] = tot;
-  }
-}
-
-// Single block: exclusive scan of the tile totals in tile order, and the
-// list of the fused G2P's work units (kG2PUnit particles of a tile each, tile
-// by tile) with their count.  Particles (< 2^32) and units are scanned
-// together as the low and high halves of one 64-bit sum.
-__global__ __launch_bounds__(1024) void k_bin_tile_offsets(const uint32_t* __restrict__ tile_total,
-                                                           uint32_t* __restrict__ tile_start,
-                                                           uint32_t* __restrict__ tile_order,
-                                                           uint32_t* __restrict__ counters,
-                                                           uint2* __restrict__ units) {
-  __shared__ uint64_t s_wave[1024 / 64 + 1], s_wave2[1024 / 64 + 1];
-  const uint32_t na = counters[CNT_ACTIVE];
-  const uint32_t chunk = (na + 1023u) / 1024u;
-  const uint32_t lo = min(na, threadIdx.x * chunk), hi = min(na, lo + chunk);
-  auto units_of = [](uint32_t t) { return (t + kG2PUnit - 1u) / kG2PUnit; };
-  uint64_t s = 0;
-  for (uint32_t a = lo; a < hi; a++) {
-    const uint32_t t = tile_total[a];
-    s += (uint64_t(units_of(t)) << 32) + t;
-  }
-  uint64_t tot;
-  const uint64_t pre = block_exclusive_scan<1024>(s, s_wave, tot);
-  uint32_t o = uint32_t(pre), uo = uint32_t(pre >> 32);
-  for (uint32_t a = lo; a < hi; a++) {
-    const uint32_t t = tile_total[a];
-    tile_start[a] = o;
-    o += t;
-    for (uint32_t c = 0, nu = units_of(t); c < nu; c++) units[uo++] = make_uint2(a, c);
-  }
-  if (threadIdx.x == 0) counters[CNT_UNITS] = uint32_t(tot >> 32);
-  // P2G's order of the tiles: four classes by particle count, largest first,
-  // tile order within a class (a stable counting sort; the class counts are
-  // packed 16 bits each into one 64-bit block scan).  A block's work grows
-  // with its tile's particles, so the long tiles start first and the short
-  // ones fill the end of the launch.  Which block takes which tile does not
-  // change any result.
-  auto cls = [](uint32_t t) { return t >= 2048u ? 0u : (t >= 1024u ? 1u : (t >= 512u ? 2u : 3u)); };
-  uint64_t cnt = 0;
-  if (na < 65536u)
-    for (uint32_t a = lo; a < hi; a++) cnt += uint64_t(1) << (16u * cls(tile_total[a]));
-  uint64_t ctot;
-  const uint64_t cpre = block_exclusive_scan<1024>(cnt, s_wave2, ctot);
-  if (na >= 65536u) {
-    for (uint32_t a = lo; a < hi; a++) tile_order[a] = a;
-  } else {
-    uint32_t base[4];
-    uint32_t acc = 0;
-#pragma unroll
-    for (uint32_t c = 0; c < 4u; c++) {
-      base[c] = acc + (uint32_t(cpre >> (16u * c)) & 0xFFFFu);
-      acc += uint32_t(ctot >> (16u * c)) & 0xFFFFu;
-    }
-    for (uint32_t a = lo; a < hi; a++) {
-      const uint32_t c = cls(tile_total[a]);
-      const uint32_t pos = c == 0u ? base[0]++ : (c == 1u ? base[1]++ : (c == 2u ? base[2]++ : base[3]++));
-      tile_order[pos] = a;
-    }
-  }
-}
-
-// Place every particle at tile start + cell start + its rank.
-__global__ __launch_bounds__(256) void k_bin_scatter(uint32_t n, const uint32_t* __restrict__ keys,
-                                                     const uint32_t* __restrict__ rank,
-                                                     const uint32_t* __restrict__ cell_end,
-                                                     const int32_t* __restrict__ tile_act,
-                                                     const uint32_t* __restrict__ tile_start,
-                                                     uint32_t* __restrict__ sorted) {
+// Key of every particle (computed from its record, or read) and its count.
+template <bool FROM_REC, bool BATCH>
+__global__ __launch_bounds__(256) void k_bin_keys(SubParams p, const float4* __restrict__ rec,
+                                                  uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
+                                                  uint32_t* __restrict__ tile_cnt) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= p.n) return;
+  uint32_t key;
+  if (FROM_REC) {
+    const float4 x = rec[size_t(i) * kRec + R_P];
+    key = cell_key(particle_geo<BATCH>(p, i), x.x, x.y, x.z);
+    keys[i] = key;
+  } else {
+    key = keys[i];
+  }
+  rank[i] = count_in_tile(key, tile_cnt);
+}
+
+__global__ __launch_bounds__(256) void k_zero(uint32_t* __restrict__ a, uint32_t n) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) a[i] = 0u;
+}
+
+// A particle and its cell within its tile: one word while the index fits
+// beside the cell (up to 2^23 particles), else a pair.
+constexpr uint32_t kPackedParticles = 1u << 23;
+template <bool PACKED>
+struct BucketEntry;
+template <>
+struct BucketEntry<true> {
+  using T = uint32_t;
+  static __device__ __forceinline__ T make(uint32_t i, uint32_t cell) { return (i << kTileBits) | cell; }
+  static __device__ __forceinline__ uint32_t index(T e) { return e >> kTileBits; }
+  static __device__ __forceinline__ uint32_t cell(T e) { return e & uint32_t(kTileCells - 1); }
+};
+template <>
+struct BucketEntry<false> {
+  using T = uint2;
+  static __device__ __forceinline__ T make(uint32_t i, uint32_t cell) { return make_uint2(i, cell); }
+  static __device__ __forceinline__ uint32_t index(T e) { return e.x; }
+  static __device__ __forceinline__ uint32_t cell(T e) { return e.y; }
+};
+template <bool PACKED>
+__device__ __forceinline__ void scatter_one(uint32_t n, uint32_t i, const uint32_t* __restrict__ keys,
+                                            const uint32_t* __restrict__ rank, const int32_t* __restrict__ tile_act,
+                                            const uint32_t* __restrict__ tile_start, uint2* __restrict__ bucket_) {
+  using E = BucketEntry<PACKED>;
+  typename E::T* bucket = reinterpret_cast<typename E::T*>(bucket_);
   if (i >= n) return;
   const uint32_t key = keys[i];
   const int32_t a = tile_act[key >> kTileBits];
-  const uint32_t slot = tile_start[a] + cell_end[key] + rank[i];
-  if (slot < n) sorted[slot] = i;  // always true when the counters started at zero
+  const uint32_t slot = tile_start[a] + rank[i];
+  if (slot < n) bucket[slot] = E::make(i, key & uint32_t(kTileCells - 1));  // always true: the counts are the keys'
 }
 
-// Per cell: order its particles by index (the ranks of different waves arrive
-// in atomic order), then store the END offset, the reference's cellOffset.
-// Cells of up to 32 particles are sorted in registers by their thread:
-// independent loads, an odd-even transposition network as wide as the wave's
-// largest cell (8, 16 or 32) that stops once a round pair swaps nothing in the
-// wave, write-back only if the order changed.  Larger
-// cells (the SDF push-out piles particles up) are listed and then sorted by
-// the whole block: staged in LDS, each element's place is the number of
-// smaller elements (indices are distinct).  Cells beyond the LDS stage fall
-// back to an in-place insertion sort by their thread.
-constexpr int kRegSort = 32;
-constexpr uint32_t kBlockSort = 2048;
+// The tile's particles in (cell, index) order, its cells' counts and END
+// offsets (the reference's cellOffset).  The counts of different waves arrive
+// in any order, so a particle's place in its cell is the number of smaller
+// indices there, counted in LDS (a cell holds about 8; lanes of one cell read
+// the same words).  A tile beyond the LDS stage places its particles in memory
+// and orders cell by cell: up to 64 particles by the cell's wave (a bitonic
+// sort across its lanes), larger cells by the block in LDS, and cells beyond
+// that by an insertion sort of their thread.
+constexpr uint32_t kSortThreads = 512;
+constexpr uint32_t kSortStage = 6144;  // particles of a tile sorted in LDS
 
-template <int M>
-__device__ __forceinline__ void cell_reg_sort(uint32_t* __restrict__ sorted, uint32_t start, uint32_t m) {
-  uint32_t v[M];
-#pragma unroll
-  for (int i = 0; i < M; i++) v[i] = uint32_t(i) < m ? sorted[start + i] : 0xFFFFFFFFu;
-  bool changed = false;
-#pragma unroll
-  for (int round = 0; round < M; round += 2) {
-    bool swapped = false;
-#pragma unroll
-    for (int half = 0; half < 2; half++) {
-#pragma unroll
-      for (int i = half; i + 1 < M; i += 2) {
-        const uint32_t lo = min(v[i], v[i + 1]), hi = max(v[i], v[i + 1]);
-        swapped |= lo != v[i];
-        v[i] = lo;
-        v[i + 1] = hi;
-      }
-    }
-    changed |= swapped;
-    if (!__any(swapped)) break;
-  }
-  if (changed) {
-#pragma unroll
-    for (int i = 0; i < M; i++)
-      if (uint32_t(i) < m) sorted[start + i] = v[i];
-  }
-}
-
-__global__ __launch_bounds__(512) void k_bin_stabilize(uint32_t n, const uint32_t* __restrict__ cell_count,
-                                                       uint32_t* __restrict__ cell_end,
-                                                       const uint32_t* __restrict__ act_tiles,
-                                                       const uint32_t* __restrict__ tile_start,
-                                                       uint32_t* __restrict__ sorted,
-                                                       const uint32_t* __restrict__ counters) {
-  __shared__ uint32_t s_big_start[kTileCells], s_big_m[kTileCells];
-  __shared__ uint32_t s_vals[kBlockSort];
+template <bool PACKED>
+__global__ __launch_bounds__(kSortThreads) void k_bin_sort(uint32_t n, const uint2* __restrict__ bucket_,
+                                                           uint32_t* __restrict__ cell_count,
+                                                           uint32_t* __restrict__ cell_end,
+                                                           const uint32_t* __restrict__ act_tiles,
+                                                           const uint32_t* __restrict__ tile_start,
+                                                           const uint32_t* __restrict__ tile_total,
+                                                           uint32_t* __restrict__ sorted,
+                                                           const uint32_t* __restrict__ counters,
+                                                           uint32_t* __restrict__ fb_ctl) {
+  using E = BucketEntry<PACKED>;
+  const typename E::T* bucket = reinterpret_cast<const typename E::T*>(bucket_);
+  __shared__ uint32_t s_idx[kSortStage + 3];  // three words past the end, read but not counted
+  __shared__ uint16_t s_cell[kSortStage];
+  __shared__ uint32_t s_cur[kTileCells], s_start[kTileCells + 1];
+  __shared__ uint32_t s_wave[kSortThreads / 64 + 1];
+  __shared__ uint16_t s_big[kTileCells];
   __shared__ uint32_t s_nbig;
+  static_assert(kSortThreads == uint32_t(kTileCells), "one thread per cell");
+  const uint32_t lane = threadIdx.x & 63u;
+  // the FP64 fallback's queue, worked off beside the scatter, is empty again
+  if (fb_ctl != nullptr && blockIdx.x == 0u && threadIdx.x < kFbSlots) fb_ctl[threadIdx.x * kFbCtlStride] = 0u;
   const uint32_t na = counters[CNT_ACTIVE];
   for (uint32_t a = blockIdx.x; a < na; a += gridDim.x) {
-    if (threadIdx.x == 0) s_nbig = 0u;
+    const uint32_t first = tile_start[a], tot = min(tile_total[a], n - min(first, n));
+    const bool staged = tot <= kSortStage;
+    s_cur[threadIdx.x] = 0u;
+    if (threadIdx.x == 0u) s_nbig = 0u;
+    // the first four entries of a thread (2048 of the tile) stay in registers
+    typename E::T held[4];
+#pragma unroll
+    for (uint32_t r = 0; r < 4u; r++) {
+      const uint32_t e = r * kSortThreads + threadIdx.x;
+      if (e < tot) held[r] = bucket[first + e];
+    }
     __syncthreads();
+    auto each = [&](auto f) {
+#pragma unroll
+      for (uint32_t r = 0; r < 4u; r++)
+        if (r * kSortThreads + threadIdx.x < tot) f(held[r]);
+      for (uint32_t e = 4u * kSortThreads + threadIdx.x; e < tot; e += kSortThreads) f(bucket[first + e]);
+    };
+    each([&](typename E::T u) { (void)atomicAdd(&s_cur[E::cell(u)], 1u); });
+    __syncthreads();
+    const uint32_t cnt = s_cur[threadIdx.x];
+    uint32_t all;
+    const uint32_t ex = block_exclusive_scan<kSortThreads>(cnt, s_wave, all);
+    s_cur[threadIdx.x] = ex;
+    s_start[threadIdx.x] = ex;
+    if (threadIdx.x == 0u) s_start[kTileCells] = all;
     const size_t key = (size_t(act_tiles[a]) << kTileBits) + threadIdx.x;
-    const uint32_t start = tile_start[a] + cell_end[key];
-    const uint32_t cnt = cell_count[key];
-    const uint32_t stop = min(start + cnt, n);
-    const uint32_t m = stop > start ? stop - start : 0u;
-    const bool reg = m <= uint32_t(kRegSort);
-    if (reg) {
-      const uint32_t mr = m;
-      if (__any(mr > 16u)) cell_reg_sort<32>(sorted, start, mr);
-      else if (__any(mr > 8u)) cell_reg_sort<16>(sorted, start, mr);
-      else cell_reg_sort<8>(sorted, start, mr);
-    } else if (m <= kBlockSort) {
-      const uint32_t slot = atomicAdd(&s_nbig, 1u);
-      s_big_start[slot] = start;
-      s_big_m[slot] = m;
-    } else {
-      for (uint32_t k = start + 1; k < stop; k++) {
-        uint32_t v = sorted[k];
+    cell_count[key] = cnt;
+    cell_end[key] = first + ex + cnt;
+    __syncthreads();
+    if (staged) {
+      each([&](typename E::T u) {
+        const uint32_t c = E::cell(u), at = atomicAdd(&s_cur[c], 1u);
+        s_idx[at] = E::index(u);
+        s_cell[at] = uint16_t(c);
+      });
+      __syncthreads();
+      for (uint32_t e = threadIdx.x; e < tot; e += kSortThreads) {
+        const uint32_t v = s_idx[e], c = s_cell[e], b = s_start[c], m = s_start[c + 1u];
+        uint32_t r = b;
+        for (uint32_t j = b; j < m; j += 4u) {  // four reads in flight
+          const uint32_t w0 = s_idx[j], w1 = s_idx[j + 1u], w2 = s_idx[j + 2u], w3 = s_idx[j + 3u];
+          r += (w0 < v ? 1u : 0u) + (j + 1u < m && w1 < v ? 1u : 0u) + (j + 2u < m && w2 < v ? 1u : 0u) +
+               (j + 3u < m && w3 < v ? 1u : 0u);
+        }
+        sorted[first + r] = v;
+      }
+      __syncthreads();
+      continue;
+    }
+    each([&](typename E::T u) { sorted[first + atomicAdd(&s_cur[E::cell(u)], 1u)] = E::index(u); });
+    __threadfence_block();
+    __syncthreads();
+    const uint32_t start = first + ex;
+    uint64_t mid = __ballot(cnt >= 2u && cnt <= 64u);
+    while (mid) {
+      const int l = __ffsll((unsigned long long)mid) - 1;
+      mid &= mid - 1ull;
+      const uint32_t m = uint32_t(__shfl(int(cnt), l));
+      uint32_t* seg = sorted + uint32_t(__shfl(int(start), l));
+      uint32_t v = lane < m ? seg[lane] : 0xFFFFFFFFu;
+      for (uint32_t k = 2; k <= 64u; k <<= 1)
+        for (uint32_t j = k >> 1; j >= 1u; j >>= 1) {
+          const uint32_t o = uint32_t(__shfl_xor(int(v), int(j)));
+          v = ((lane & k) == 0u) == ((lane & j) == 0u) ? min(v, o) : max(v, o);
+        }
+      if (lane < m) seg[lane] = v;
+    }
+    if (cnt > 64u && cnt <= kSortStage) {
+      s_big[atomicAdd(&s_nbig, 1u)] = uint16_t(threadIdx.x);
+    } else if (cnt > kSortStage) {
+      for (uint32_t k = start + 1; k < start + cnt; k++) {
+        const uint32_t v = sorted[k];
         uint32_t j = k;
         while (j > start && sorted[j - 1] > v) {
           sorted[j] = sorted[j - 1];
@@ -337,21 +258,21 @@ __global__ __launch_bounds__(512) void k_bin_stabilize(uint32_t n, const uint32_
         sorted[j] = v;
       }
     }
-    cell_end[key] = start + cnt;
     __syncthreads();
     const uint32_t nbig = s_nbig;
-    for (uint32_t b = 0; b < nbig; b++) {
-      const uint32_t bs = s_big_start[b], bm = s_big_m[b];
-      for (uint32_t e = threadIdx.x; e < bm; e += blockDim.x) s_vals[e] = sorted[bs + e];
+    for (uint32_t q = 0; q < nbig; q++) {
+      const uint32_t c = s_big[q], bs = first + s_start[c], bm = s_start[c + 1u] - s_start[c];
+      for (uint32_t e = threadIdx.x; e < bm; e += kSortThreads) s_idx[e] = sorted[bs + e];
       __syncthreads();
-      for (uint32_t e = threadIdx.x; e < bm; e += blockDim.x) {
-        const uint32_t v = s_vals[e];
+      for (uint32_t e = threadIdx.x; e < bm; e += kSortThreads) {
+        const uint32_t v = s_idx[e];
         uint32_t r = 0;
-        for (uint32_t j = 0; j < bm; j++) r += s_vals[j] < v ? 1u : 0u;
+        for (uint32_t j = 0; j < bm; j++) r += s_idx[j] < v ? 1u : 0u;
         sorted[bs + r] = v;
       }
       __syncthreads();
     }
+    __syncthreads();
   }
 }
 
@@ -1119,7 +1040,8 @@ __device__ __forceinline__ uint32_t queue_fb(const SubParams& p, uint32_t k, uin
 // it).  k: the particle's place in the G2P order, which picks its queue slot.
 template <bool FLIP, bool BATCH>
 __device__ __forceinline__ void g2p_particle(const SubParams& p, uint32_t k, uint32_t q, const float4* r, float4* ro,
-                                             uint32_t* __restrict__ keys, const nb_material& mat,
+                                             uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
+                                             uint32_t* __restrict__ tile_cnt, const nb_material& mat,
                                              const G2PGather& gth, const float4 pp, const float4 vel,
                                              const float* __restrict__ sdf) {
   const float xp = pp.x, yp = pp.y, zp = pp.z, Vp = pp.w;
@@ -1286,7 +1208,9 @@ __device__ __forceinline__ void g2p_particle(const SubParams& p, uint32_t k, uin
   ro[R_T] = make_float4(tau.m[0][0], tau.m[1][1], tau.m[2][2], Fn.m[0][0]);
   ro[R_FA] = make_float4(Fn.m[0][1], Fn.m[0][2], Fn.m[1][0], Fn.m[1][1]);
   ro[R_FB] = make_float4(Fn.m[1][2], Fn.m[2][0], Fn.m[2][1], Fn.m[2][2]);
-  keys[q] = cell_key(ge, xn, yn, zn);  // the next substep's bin key
+  const uint32_t key = cell_key(ge, xn, yn, zn);  // the next substep's bin key, and its count
+  keys[q] = key;
+  if (tile_cnt != nullptr) rank[q] = count_in_tile(key, tile_cnt);
   // F and tau were set to I and 0: the fallback's entry is dropped
   if (fb_at != kFbNone && (jreset || pushed)) reinterpret_cast<uint32_t*>(p.fb_queue + size_t(fb_at) * kFbEntry)[1] = 0u;
 }
@@ -1300,7 +1224,8 @@ __device__ __forceinline__ uint32_t particle_material(const SubParams& p, const 
 // G2P of particle q (place k of the G2P order) reading the updated grid from HBM.
 template <bool FLIP, bool BATCH>
 __device__ __forceinline__ void g2p_one(const SubParams& p, uint32_t k, uint32_t q, const float4* rec_in, float4* rec_out,
-                                        uint32_t* __restrict__ keys, const nb_material* __restrict__ mats,
+                                        uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
+                                        uint32_t* __restrict__ tile_cnt, const nb_material* __restrict__ mats,
                                         const nb_material* s_mats, const float4* __restrict__ grid_node,
                                         const float4* __restrict__ grid_old, const float* __restrict__ sdf) {
   const SceneGeo g = particle_geo<BATCH>(p, q);
@@ -1339,7 +1264,7 @@ __device__ __forceinline__ void g2p_one(const SubParams& p, uint32_t k, uint32_t
   const float4 vel = r[R_V];
   const uint32_t mid = particle_material(p, vel);
   const nb_material mat = BATCH ? mats[mid] : s_mats[mid];
-  g2p_particle<FLIP, BATCH>(p, k, q, r, ro, keys, mat, gth, pp, vel, sdf);
+  g2p_particle<FLIP, BATCH>(p, k, q, r, ro, keys, rank, tile_cnt, mat, gth, pp, vel, sdf);
 }
 
 // a plain engine's material table is staged in LDS; a batch's (up to
@@ -1364,7 +1289,8 @@ template <bool FLIP, bool BATCH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_g2p(SubParams p,
                                                                                    const float4* rec_in,
                                                                                    float4* rec_out,
-                                             uint32_t* __restrict__ keys,
+                                             uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
+                                             uint32_t* __restrict__ tile_cnt,
                                              const nb_material* __restrict__ mats,
                                              const uint32_t* __restrict__ sorted,
                                              const float4* __restrict__ grid_node,
@@ -1374,19 +1300,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   const uint32_t k = xcd_chunk(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   if (k >= p.n) return;
   const uint32_t q = sorted ? sorted[k] : k;
-  g2p_one<FLIP, BATCH>(p, k, q, rec_in, rec_out, keys, mats, s_mats, grid_node, grid_old, sdf);
+  g2p_one<FLIP, BATCH>(p, k, q, rec_in, rec_out, keys, rank, tile_cnt, mats, s_mats, grid_node, grid_old, sdf);
 }
 
 // The FP64 fallback's second half: for every entry G2P queued (queue_fb),
 // the return map and Hencky stress in FP64 from the trial F (mode 1), or the
 // Hencky stress of the record's F (mode 2), rounded once; F is replaced and
 // the stress added to the record's (the mud viscosity term, or zero).
-// Every block reads the slots' lengths and the grid strides over their
-// concatenation; k_g2p_fb_reset then zeroes the lengths for the next G2P.
-// (A count of finished blocks, the last one zeroing, cost tens of ns per
-// block: device-scope atomics on one address serialise across the XCDs.)
+// Every block reads the slots' lengths and the `blocks` blocks stride over
+// their concatenation.  Within a call it runs beside the next substep's
+// scatter, which does not touch the records (a launch of its own was 12-19 us
+// of latency chain per substep), and the sort after that zeroes the lengths; a
+// call's last substep runs it alone
+// (k_g2p_fb), then k_g2p_fb_reset.  (A count of finished blocks, the last one
+// zeroing, cost tens of ns per block: device-scope atomics on one address
+// serialise across the XCDs.)
 template <bool BATCH>
-__global__ __launch_bounds__(256) void k_g2p_fb(SubParams p, float4* rec, const nb_material* __restrict__ mats) {
+__device__ __forceinline__ void fb_entries(const SubParams& p, float4* rec, const nb_material* __restrict__ mats,
+                                           uint32_t block, uint32_t blocks) {
   __shared__ nb_material s_mats[BATCH ? 1 : NB_MAX_MATERIALS];
   stage_materials<BATCH>(p, mats, s_mats);
   // the slots' lengths and their exclusive prefix (wave 0), so that the
@@ -1406,7 +1337,11 @@ __global__ __launch_bounds__(256) void k_g2p_fb(SubParams p, float4* rec, const 
   __syncthreads();
   const uint32_t total = s_pre[kFbSlots];
   const bool cs = p.corrected_svd != 0u;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
+  // consecutive waves of entries go to different blocks, so that a short queue
+  // is spread over the CUs (its FP64 chains are latency: 1,400 entries in two
+  // blocks of 1024 took 28 us, spread 14)
+  const uint32_t wave_of = (threadIdx.x >> 6) * blocks + block;
+  for (uint32_t i = wave_of * 64u + (threadIdx.x & 63u); i < total; i += blocks * blockDim.x) {
     // the slot holding entry i of the concatenated queue: the last s with s_pre[s] <= i
     uint32_t slot = 0u;
 #pragma unroll
@@ -1459,8 +1394,304 @@ __global__ __launch_bounds__(256) void k_g2p_fb(SubParams p, float4* rec, const 
   }
 }
 
+template <bool BATCH>
+__global__ __launch_bounds__(256) void k_g2p_fb(SubParams p, float4* rec, const nb_material* __restrict__ mats) {
+  fb_entries<BATCH>(p, rec, mats, blockIdx.x, gridDim.x);
+}
+
 __global__ __launch_bounds__(64) void k_g2p_fb_reset(uint32_t* __restrict__ fb_ctl) {
   if (threadIdx.x < kFbSlots) fb_ctl[threadIdx.x * kFbCtlStride] = 0u;
+}
+
+// ---------------------------------------------------------------------------
+// the bin's tile pass and scatter (after the fallback, which runs beside them)
+// ---------------------------------------------------------------------------
+// Every particle and its cell into its tile's range, at its place of the count.
+// The launch's first fb_blocks blocks work off the FP64 fallback's queue of the
+// G2P before (they are the longer ones); the sort empties it.
+template <bool PACKED, bool BATCH>
+__global__ __launch_bounds__(256) void k_bin_scatter_fb(SubParams p, float4* rec, const nb_material* __restrict__ mats,
+                                                        const uint32_t* __restrict__ keys,
+                                                        const uint32_t* __restrict__ rank,
+                                                        const int32_t* __restrict__ tile_act,
+                                                        const uint32_t* __restrict__ tile_start,
+                                                        uint2* __restrict__ bucket, uint32_t fb_blocks) {
+  if (blockIdx.x < fb_blocks) fb_entries<BATCH>(p, rec, mats, blockIdx.x, fb_blocks);
+  else scatter_one<PACKED>(p.n, (blockIdx.x - fb_blocks) * blockDim.x + threadIdx.x, keys, rank, tile_act, tile_start, bucket);
+}
+template <bool PACKED>
+__global__ __launch_bounds__(256) void k_bin_scatter(uint32_t n, const uint32_t* __restrict__ keys,
+                                                     const uint32_t* __restrict__ rank,
+                                                     const int32_t* __restrict__ tile_act,
+                                                     const uint32_t* __restrict__ tile_start,
+                                                     uint2* __restrict__ bucket) {
+  scatter_one<PACKED>(n, blockIdx.x * blockDim.x + threadIdx.x, keys, rank, tile_act, tile_start, bucket);
+}
+
+// P2G's order of the tiles: four classes by particle count, largest first,
+// tile order within a class.  A block's work grows with its tile's particles,
+// so the long tiles start first and the short ones fill the end of the launch.
+// Which block takes which tile does not change any result.
+__device__ __forceinline__ uint32_t tile_class(uint32_t t) {
+  return t >= 2048u ? 0u : (t >= 1024u ? 1u : (t >= 512u ? 2u : 3u));
+}
+__device__ __forceinline__ uint32_t tile_units(uint32_t t) { return (t + kG2PUnit - 1u) / kG2PUnit; }
+
+// Cubes of up to kSmallTiles tiles (128^3 cells): one block does the whole
+// pass in one launch.  Thread t holds the tiles [t C, (t + 1) C).  Per tile:
+// occupied; node tile (a tile of its 3x3x3 neighbourhood is occupied: its nodes
+// can receive mass), found axis by axis in LDS (27 reads a tile at once took
+// 25 us for 4,096 tiles, all on one CU).  4.6 us for 64 tiles, 5.7 for 512, 10.4
+// for 4,096, where the two launches below take 5.8 + 6.0; they spread larger
+// cubes over the chip.
+constexpr uint32_t kSmallTiles = 4096;
+template <bool BATCH>
+__global__ __launch_bounds__(1024) void k_bin_tiles(SubParams p, uint32_t* __restrict__ tile_cnt,
+                                                    int32_t* __restrict__ tile_act,
+                                                    uint32_t* __restrict__ act_tiles,
+                                                    uint32_t* __restrict__ node_tiles,
+                                                    uint32_t* __restrict__ tile_total,
+                                                    uint32_t* __restrict__ tile_start,
+                                                    uint32_t* __restrict__ tile_order,
+                                                    uint32_t* __restrict__ counters, uint2* __restrict__ units,
+                                                    uint32_t nt) {
+  constexpr uint32_t C = kSmallTiles / 1024u;
+  __shared__ uint8_t s_occ[2][kSmallTiles];
+  __shared__ uint64_t s_scan[3 * (1024 / 64 + 1)];
+  const uint32_t c = (nt + 1023u) / 1024u, t0 = threadIdx.x * c;
+  uint32_t cnt[C];
+  int at3[C][3], td[C];
+  SceneGeo g;
+#pragma unroll
+  for (uint32_t k = 0; k < C; k++) {
+    const uint32_t T = t0 + k;
+    cnt[k] = 0u;
+    if (k < c && T < nt) {
+      cnt[k] = tile_cnt[T];
+      g = tile_geo<BATCH>(p, T);  // neighbours stay inside the tile's scene
+      tile_coords(g, T, at3[k][0], at3[k][1], at3[k][2]);
+      td[k] = int(g.tile_dim);
+      s_occ[0][T] = cnt[k] ? 1 : 0;
+      if (cnt[k]) tile_cnt[T] = 0u;  // ready for the next count
+    }
+  }
+  // occupied in the 3x3x3 neighbourhood, axis by axis
+  uint32_t node = 0;  // bit k: tile t0 + k is a node tile
+#pragma unroll
+  for (int axis = 0; axis < 3; axis++) {
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < C; k++) {
+      const uint32_t T = t0 + k;
+      if (k < c && T < nt) {
+        const SceneGeo gk = BATCH ? tile_geo<BATCH>(p, T) : g;
+        uint32_t any = s_occ[axis & 1][T];
+#pragma unroll
+        for (int d = -1; d <= 1; d += 2) {
+          const int v = at3[k][axis] + d;
+          const bool in = uint32_t(v) < uint32_t(td[k]);
+          const int w = in ? v : at3[k][axis];
+          any |= s_occ[axis & 1][tile_id(gk, axis == 0 ? w : at3[k][0], axis == 1 ? w : at3[k][1], axis == 2 ? w : at3[k][2])];
+        }
+        s_occ[1 - (axis & 1)][T] = uint8_t(any);
+        if (axis == 2 && any) node |= 1u << k;
+      }
+    }
+  }
+  uint64_t lists = 0, places = 0, classes = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < C; k++) {
+    lists += uint64_t(cnt[k] ? 1u : 0u) | (uint64_t((node >> k) & 1u) << 32);
+    places += uint64_t(cnt[k]) | (uint64_t(tile_units(cnt[k])) << 32);
+    if (cnt[k]) classes += uint64_t(1) << (16u * tile_class(cnt[k]));
+  }
+  const uint64_t own[3] = {lists, places, classes};
+  uint64_t pre3[3], tot3[3];
+  block_exclusive_scan3<1024>(own, s_scan, pre3, tot3);
+  const uint64_t l0 = pre3[0], p0 = pre3[1], c0 = pre3[2];
+  const uint64_t n_lists = tot3[0], n_places = tot3[1], n_classes = tot3[2];
+  uint32_t oa = uint32_t(l0), on = uint32_t(l0 >> 32), os = uint32_t(p0), ou = uint32_t(p0 >> 32);
+  uint32_t at[4], before = 0;
+#pragma unroll
+  for (uint32_t q = 0; q < 4u; q++) {
+    at[q] = before + (uint32_t(c0 >> (16u * q)) & 0xFFFFu);
+    before += uint32_t(n_classes >> (16u * q)) & 0xFFFFu;
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < C; k++) {
+    const uint32_t T = t0 + k;
+    if (!(k < c && T < nt)) continue;
+    tile_act[T] = cnt[k] ? int32_t(oa) : -1;
+    if (cnt[k]) {
+      act_tiles[oa] = T;
+      tile_total[oa] = cnt[k];
+      tile_start[oa] = os;
+      for (uint32_t u = 0, nu = tile_units(cnt[k]); u < nu; u++) units[ou++] = make_uint2(oa, u);
+      const uint32_t q = tile_class(cnt[k]);
+      tile_order[q == 0u ? at[0]++ : (q == 1u ? at[1]++ : (q == 2u ? at[2]++ : at[3]++))] = oa;
+      os += cnt[k];
+      oa++;
+    }
+    if ((node >> k) & 1u) node_tiles[on++] = T;
+  }
+  if (threadIdx.x == 0u) {
+    counters[CNT_ACTIVE] = uint32_t(n_lists);
+    counters[CNT_NODE_TILES] = uint32_t(n_lists >> 32);
+    counters[CNT_UNITS] = uint32_t(n_places >> 32);
+  }
+}
+
+// Larger cubes: 256 tiles a block in two launches.  k_bin_mark: each tile's
+// marks (bit 0 occupied, bit 1 node tile) and its block's sums; the blocks after
+// the first `tile_blocks` work off the fallback's queue.
+template <bool BATCH>
+__global__ __launch_bounds__(256) void k_bin_mark(SubParams p, float4* rec, const nb_material* __restrict__ mats,
+                                                  const uint32_t* __restrict__ tile_cnt,
+                                                  uint8_t* __restrict__ tile_mark, TileSums* __restrict__ sums,
+                                                  uint32_t nt, uint32_t tile_blocks) {
+  if (blockIdx.x >= tile_blocks) {
+    fb_entries<BATCH>(p, rec, mats, blockIdx.x - tile_blocks, gridDim.x - tile_blocks);
+    return;
+  }
+  __shared__ uint64_t s_scan[3 * (256 / 64 + 1)];
+  const uint32_t T = blockIdx.x * blockDim.x + threadIdx.x;
+  uint32_t m = 0, cnt = 0;
+  if (T < nt) {
+    const SceneGeo g = tile_geo<BATCH>(p, T);
+    int tx, ty, tz;
+    tile_coords(g, T, tx, ty, tz);
+    const int td = int(g.tile_dim);
+    cnt = tile_cnt[T];
+    uint32_t any = 0;
+#pragma unroll
+    for (int o = 0; o < 27; o++) {  // all loads in flight together
+      const int x = tx + o % 3 - 1, y = ty + (o / 3) % 3 - 1, z = tz + o / 9 - 1;
+      const bool in = uint32_t(x) < uint32_t(td) && uint32_t(y) < uint32_t(td) && uint32_t(z) < uint32_t(td);
+      any |= in ? tile_cnt[tile_id(g, in ? x : tx, in ? y : ty, in ? z : tz)] : 0u;
+    }
+    m = (cnt ? 1u : 0u) | (any ? 2u : 0u);
+    tile_mark[T] = uint8_t(m);
+  }
+  const uint64_t own[3] = {uint64_t(m & 1u) | (uint64_t(m >> 1) << 32), uint64_t(cnt) | (uint64_t(tile_units(cnt)) << 32),
+                           cnt ? uint64_t(1) << (16u * tile_class(cnt)) : uint64_t(0)};
+  uint64_t pre3[3], tot3[3];
+  block_exclusive_scan3<256>(own, s_scan, pre3, tot3);
+  if (threadIdx.x == 0u) {
+    TileSums t;
+    t.lists = tot3[0];
+    t.places = tot3[1];
+#pragma unroll
+    for (uint32_t q = 0; q < 4u; q++) t.cls[q] = uint32_t(tot3[2] >> (16u * q)) & 0xFFFFu;
+    sums[blockIdx.x] = t;
+  }
+}
+
+// Beyond kSumBlocks blocks: their sums scanned in place by one block, the
+// total behind the last (a block of k_bin_compact otherwise adds up those
+// before it, and all of them, by itself).
+constexpr uint32_t kSumBlocks = 1024;
+__global__ __launch_bounds__(1024) void k_bin_sums(TileSums* __restrict__ sums, uint32_t nb) {
+  __shared__ uint64_t s_scan[1024 / 64 + 1];
+  const uint32_t per = (nb + 1023u) / 1024u, lo = min(nb, threadIdx.x * per), hi = min(nb, lo + per);
+  TileSums t{};
+  for (uint32_t i = lo; i < hi; i++) {
+    t.lists += sums[i].lists;
+    t.places += sums[i].places;
+    for (int q = 0; q < 4; q++) t.cls[q] += sums[i].cls[q];
+  }
+  TileSums run, tot;
+  run.lists = block_exclusive_scan<1024>(t.lists, s_scan, tot.lists);
+  run.places = block_exclusive_scan<1024>(t.places, s_scan, tot.places);
+  uint64_t c01, c23;
+  const uint64_t a = block_exclusive_scan<1024>(uint64_t(t.cls[0]) | (uint64_t(t.cls[1]) << 32), s_scan, c01);
+  const uint64_t b = block_exclusive_scan<1024>(uint64_t(t.cls[2]) | (uint64_t(t.cls[3]) << 32), s_scan, c23);
+  run.cls[0] = uint32_t(a); run.cls[1] = uint32_t(a >> 32); run.cls[2] = uint32_t(b); run.cls[3] = uint32_t(b >> 32);
+  tot.cls[0] = uint32_t(c01); tot.cls[1] = uint32_t(c01 >> 32); tot.cls[2] = uint32_t(c23); tot.cls[3] = uint32_t(c23 >> 32);
+  for (uint32_t i = lo; i < hi; i++) {
+    const TileSums x = sums[i];
+    sums[i] = run;
+    run.lists += x.lists;
+    run.places += x.places;
+    for (int q = 0; q < 4; q++) run.cls[q] += x.cls[q];
+  }
+  if (threadIdx.x == 0u) sums[nb] = tot;
+}
+
+template <bool SCANNED>
+__global__ __launch_bounds__(256) void k_bin_compact(const uint8_t* __restrict__ tile_mark,
+                                                     const TileSums* __restrict__ sums,
+                                                     uint32_t* __restrict__ tile_cnt, int32_t* __restrict__ tile_act,
+                                                     uint32_t* __restrict__ act_tiles,
+                                                     uint32_t* __restrict__ node_tiles,
+                                                     uint32_t* __restrict__ tile_total,
+                                                     uint32_t* __restrict__ tile_start,
+                                                     uint32_t* __restrict__ tile_order,
+                                                     uint32_t* __restrict__ counters, uint2* __restrict__ units,
+                                                     uint32_t nt) {
+  __shared__ uint64_t s_scan[3 * (256 / 64 + 1)];
+  __shared__ uint64_t s_sum[256 / 64][8];
+  TileSums pre, tot;
+  if (SCANNED) {
+    pre = sums[blockIdx.x];
+    tot = sums[gridDim.x];
+  } else {
+    uint64_t v[8] = {};  // lists, places, two pairs of classes: of the blocks before this one, and of all
+    for (uint32_t i = threadIdx.x; i < gridDim.x; i += blockDim.x) {
+      const TileSums x = sums[i];
+      const uint64_t w[4] = {x.lists, x.places, uint64_t(x.cls[0]) | (uint64_t(x.cls[1]) << 32),
+                             uint64_t(x.cls[2]) | (uint64_t(x.cls[3]) << 32)};
+      const bool before = i < blockIdx.x;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        v[q] += before ? w[q] : 0u;
+        v[4 + q] += w[q];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1) v[q] += __shfl_xor(v[q], d);
+      if ((threadIdx.x & 63u) == 0u) s_sum[threadIdx.x >> 6][q] = v[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] = (s_sum[0][q] + s_sum[1][q]) + (s_sum[2][q] + s_sum[3][q]);
+    pre.lists = v[0];
+    pre.places = v[1];
+    pre.cls[0] = uint32_t(v[2]); pre.cls[1] = uint32_t(v[2] >> 32); pre.cls[2] = uint32_t(v[3]); pre.cls[3] = uint32_t(v[3] >> 32);
+    tot.lists = v[4];
+    tot.places = v[5];
+    tot.cls[0] = uint32_t(v[6]); tot.cls[1] = uint32_t(v[6] >> 32); tot.cls[2] = uint32_t(v[7]); tot.cls[3] = uint32_t(v[7] >> 32);
+  }
+  const uint32_t T = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t m = T < nt ? tile_mark[T] : 0u, cnt = (m & 1u) ? tile_cnt[T] : 0u;
+  const uint32_t q = tile_class(cnt);
+  const uint64_t own[3] = {uint64_t(m & 1u) | (uint64_t(m >> 1) << 32), uint64_t(cnt) | (uint64_t(tile_units(cnt)) << 32),
+                           cnt ? uint64_t(1) << (16u * q) : uint64_t(0)};
+  uint64_t pre3[3], tot3[3];
+  block_exclusive_scan3<256>(own, s_scan, pre3, tot3);
+  const uint64_t l0 = pre.lists + pre3[0], p0 = pre.places + pre3[1], c0 = pre3[2];
+  if (T < nt) {
+    const uint32_t oa = uint32_t(l0);
+    tile_act[T] = cnt ? int32_t(oa) : -1;
+    if (cnt) {
+      act_tiles[oa] = T;
+      tile_total[oa] = cnt;
+      tile_start[oa] = uint32_t(p0);
+      for (uint32_t u = 0, nu = tile_units(cnt); u < nu; u++) units[uint32_t(p0 >> 32) + u] = make_uint2(oa, u);
+      uint32_t at = uint32_t(c0 >> (16u * q)) & 0xFFFFu;
+#pragma unroll
+      for (uint32_t k = 0; k < 4u; k++) at += k < q ? tot.cls[k] : (k == q ? pre.cls[k] : 0u);
+      tile_order[at] = oa;
+      tile_cnt[T] = 0u;  // ready for the next count
+    }
+    if (m & 2u) node_tiles[uint32_t(l0 >> 32)] = T;
+  }
+  if (blockIdx.x == 0u && threadIdx.x == 0u) {
+    counters[CNT_ACTIVE] = uint32_t(tot.lists);
+    counters[CNT_NODE_TILES] = uint32_t(tot.lists >> 32);
+    counters[CNT_UNITS] = uint32_t(tot.places >> 32);
+  }
 }
 
 // Grid update and G2P fused, one block per work unit: a unit is up to
@@ -1477,7 +1708,8 @@ __global__ __launch_bounds__(64) void k_g2p_fb_reset(uint32_t* __restrict__ fb_c
 // exported grid stays that of the last substep).
 template <bool FLIP, bool BATCH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_g2p_tile(
-    SubParams p, const float4* rec_in, float4* rec_out, uint32_t* __restrict__ keys,
+    SubParams p, const float4* rec_in, float4* rec_out, uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
+    uint32_t* __restrict__ tile_cnt,
     const nb_material* __restrict__ mats, const uint32_t* __restrict__ sorted, const uint2* __restrict__ units,
     const uint32_t* __restrict__ act_tiles, const uint32_t* __restrict__ tile_start,
     const uint32_t* __restrict__ tile_total, const uint32_t* __restrict__ counters,
@@ -1568,7 +1800,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
       const float4 vel = r[R_V];
       const uint32_t mid = particle_material(p, vel);
       const nb_material mat = BATCH ? mats[mid] : s_mats[mid];
-      g2p_particle<FLIP, BATCH>(p, k, q, r, ro, keys, mat, gth, pp, vel, sdf);
+      g2p_particle<FLIP, BATCH>(p, k, q, r, ro, keys, rank, tile_cnt, mat, gth, pp, vel, sdf);
     }
   }
 }
@@ -1671,40 +1903,106 @@ struct ProfScope {
   }
 };
 
-void launch_bin(const DevState& d, const SubParams& p, uint32_t n_tiles, bool keys_valid, hipStream_t s, Prof* pf) {
+// blocks of `threads` for the fallback's queue: at most one thread per
+// particle, and enough for a queue of a million entries to have a thread each
+// (a block past the queue's end only reads the 64 lengths)
+static inline uint32_t fb_blocks(const SubParams& p, uint32_t threads) {
+  return p.svd_fp64 ? std::min(cdiv(p.n, threads), (1u << 20) / threads) : 0u;
+}
+
+// the fallback's queue in a launch of its own
+static void launch_fb_entries(const DevState& d, const SubParams& p, float4* rec, hipStream_t s) {
+  const uint32_t g = fb_blocks(p, 256);
+  if (!g) return;
+  if (p.n_scenes > 0)
+    k_g2p_fb<true><<<g, 256, 0, s>>>(p, rec, d.materials);
+  else
+    k_g2p_fb<false><<<g, 256, 0, s>>>(p, rec, d.materials);
+}
+
+void launch_clear_counts(const DevState& d, uint32_t n_tiles, hipStream_t s) {
+  k_zero<<<cdiv(n_tiles, 256), 256, 0, s>>>(d.tile_cnt, n_tiles);
+}
+
+void launch_bin(const DevState& d, const SubParams& p, uint32_t n_tiles, BinFrom from, hipStream_t s, Prof* pf) {
   const uint32_t tg = tile_grid(n_tiles, p.tile_blocks);
   const bool batch = p.n_scenes > 0;
-  { ProfScope ps(pf, 0, s); k_bin_clear<<<tg, 512, 0, s>>>(d.cell_count, d.act_tiles, d.counters); }
-  {
-    ProfScope ps(pf, 1, s);
+  if (from != BinFrom::COUNTED) {
+    ProfScope ps(pf, 0, s);
     const uint32_t nb = cdiv(p.n, 256);
-    if (keys_valid)
-      k_bin_keys<false, false><<<nb, 256, 0, s>>>(p, d.rec, d.keys, d.rank, d.cell_count, d.tile_flag);
+    if (from == BinFrom::KEYS)
+      k_bin_keys<false, false><<<nb, 256, 0, s>>>(p, d.rec, d.keys, d.rank, d.tile_cnt);
     else if (batch)
-      k_bin_keys<true, true><<<nb, 256, 0, s>>>(p, d.rec, d.keys, d.rank, d.cell_count, d.tile_flag);
+      k_bin_keys<true, true><<<nb, 256, 0, s>>>(p, d.rec, d.keys, d.rank, d.tile_cnt);
     else
-      k_bin_keys<true, false><<<nb, 256, 0, s>>>(p, d.rec, d.keys, d.rank, d.cell_count, d.tile_flag);
+      k_bin_keys<true, false><<<nb, 256, 0, s>>>(p, d.rec, d.keys, d.rank, d.tile_cnt);
   }
   {
+    ProfScope ps(pf, 1, s);
+    if (n_tiles <= kSmallTiles) {
+#define NB_TILES(BT)                                                                                             \
+  k_bin_tiles<BT><<<1, 1024, 0, s>>>(p, d.tile_cnt, d.tile_act, d.act_tiles, d.node_tiles, d.tile_total,         \
+                                     d.tile_start, d.tile_order, d.counters, d.units, n_tiles)
+      if (batch) NB_TILES(true); else NB_TILES(false);
+#undef NB_TILES
+    } else {
+      const uint32_t tb = cdiv(n_tiles, 256), g = tb + fb_blocks(p, 256);
+      if (batch)
+        k_bin_mark<true><<<g, 256, 0, s>>>(p, d.rec, d.materials, d.tile_cnt, d.tile_mark, d.tile_sums, n_tiles, tb);
+      else
+        k_bin_mark<false><<<g, 256, 0, s>>>(p, d.rec, d.materials, d.tile_cnt, d.tile_mark, d.tile_sums, n_tiles, tb);
+    }
+  }
+  if (n_tiles > kSmallTiles) {
     ProfScope ps(pf, 2, s);
-    if (batch)
-      k_bin_mark<true><<<cdiv(n_tiles, 256), 256, 0, s>>>(p, d.tile_flag, d.tile_mark, d.blk_cnt, n_tiles);
-    else
-      k_bin_mark<false><<<cdiv(n_tiles, 256), 256, 0, s>>>(p, d.tile_flag, d.tile_mark, d.blk_cnt, n_tiles);
+    const uint32_t tb = cdiv(n_tiles, 256);
+#define NB_COMPACT(SC)                                                                                            \
+  k_bin_compact<SC><<<tb, 256, 0, s>>>(d.tile_mark, d.tile_sums, d.tile_cnt, d.tile_act, d.act_tiles, d.node_tiles, \
+                                       d.tile_total, d.tile_start, d.tile_order, d.counters, d.units, n_tiles)
+    if (tb > kSumBlocks) {
+      k_bin_sums<<<1, 1024, 0, s>>>(d.tile_sums, tb);
+      NB_COMPACT(true);
+    } else {
+      NB_COMPACT(false);
+    }
+#undef NB_COMPACT
   }
   {
     ProfScope ps(pf, 3, s);
-    k_bin_compact<<<cdiv(n_tiles, 256), 256, 0, s>>>(d.tile_mark, d.blk_cnt, d.tile_flag, d.tile_act, d.act_tiles,
-                                                     d.node_tiles, d.counters, n_tiles);
+    // small cubes: the fallback's queue beside the scatter, while that is
+    // short (262,144 particles: 14.7 us together, 5 + 14 apart); beyond 2^20
+    // particles its registers would slow the scatter (4.19 M: 39 against 20 + 16)
+    const bool apart = p.n > (1u << 20);
+    const uint32_t nb = cdiv(p.n, 256), fb = n_tiles <= kSmallTiles && !apart ? fb_blocks(p, 256) : 0u;
+    if (n_tiles <= kSmallTiles && apart) launch_fb_entries(d, p, d.rec, s);
+#define NB_SCATTER_FB(PK, BT)                                                                                   \
+  k_bin_scatter_fb<PK, BT><<<nb + fb, 256, 0, s>>>(p, d.rec, d.materials, d.keys, d.rank, d.tile_act, d.tile_start, \
+                                                   d.bucket, fb)
+    const bool packed = p.n <= kPackedParticles;
+    if (!fb) {
+      if (packed) k_bin_scatter<true><<<nb, 256, 0, s>>>(p.n, d.keys, d.rank, d.tile_act, d.tile_start, d.bucket);
+      else k_bin_scatter<false><<<nb, 256, 0, s>>>(p.n, d.keys, d.rank, d.tile_act, d.tile_start, d.bucket);
+    } else if (packed) {
+      if (batch) NB_SCATTER_FB(true, true); else NB_SCATTER_FB(true, false);
+    } else {
+      if (batch) NB_SCATTER_FB(false, true); else NB_SCATTER_FB(false, false);
+    }
+#undef NB_SCATTER_FB
   }
-  { ProfScope ps(pf, 4, s); k_bin_tile_scan<<<tg, 512, 0, s>>>(d.cell_count, d.cell_end, d.act_tiles, d.tile_total, d.counters); }
-  { ProfScope ps(pf, 5, s); k_bin_tile_offsets<<<1, 1024, 0, s>>>(d.tile_total, d.tile_start, d.tile_order, d.counters, d.units); }
-  { ProfScope ps(pf, 6, s); k_bin_scatter<<<cdiv(p.n, 256), 256, 0, s>>>(p.n, d.keys, d.rank, d.cell_end, d.tile_act, d.tile_start, d.sorted); }
-  { ProfScope ps(pf, 7, s); k_bin_stabilize<<<tg, 512, 0, s>>>(p.n, d.cell_count, d.cell_end, d.act_tiles, d.tile_start, d.sorted, d.counters); }
+  {
+    ProfScope ps(pf, 4, s);
+    uint32_t* fb_ctl = p.svd_fp64 ? p.fb_ctl : nullptr;
+    if (p.n <= kPackedParticles)
+      k_bin_sort<true><<<tg, kSortThreads, 0, s>>>(p.n, d.bucket, d.cell_count, d.cell_end, d.act_tiles, d.tile_start,
+                                                   d.tile_total, d.sorted, d.counters, fb_ctl);
+    else
+      k_bin_sort<false><<<tg, kSortThreads, 0, s>>>(p.n, d.bucket, d.cell_count, d.cell_end, d.act_tiles, d.tile_start,
+                                                    d.tile_total, d.sorted, d.counters, fb_ctl);
+  }
 }
 
 void launch_p2g(const DevState& d, const SubParams& p, uint32_t n_tiles, hipStream_t s, Prof* pf) {
-  ProfScope ps(pf, 8, s);
+  ProfScope ps(pf, 5, s);
   if (p.n_scenes > 0)
     k_p2g<true><<<tile_grid(n_tiles, p.tile_blocks), kP2GThreads, 0, s>>>(p, d.rec, d.materials, d.cell_count, d.cell_end, d.sorted,
                                                            d.act_tiles, d.tile_order, d.tile_start, d.tile_total,
@@ -1717,7 +2015,7 @@ void launch_p2g(const DevState& d, const SubParams& p, uint32_t n_tiles, hipStre
 
 void launch_grid(const DevState& d, const SubParams& p, uint32_t n_tiles, bool from_partials, bool update,
                  const uint32_t* tiles, const uint32_t* count, hipStream_t s, Prof* pf) {
-  ProfScope ps(pf, 9, s);
+  ProfScope ps(pf, 6, s);
   const uint32_t g = tile_grid(n_tiles, p.tile_blocks);
 #define NB_GRID_LAUNCH(FP, UP, BT, NZ)                                                                       \
   k_grid<FP, UP, BT, NZ><<<g, 512, 0, s>>>(p, d.partial, d.tile_act, tiles, count, d.grid_node, d.grid_old, \
@@ -1752,11 +2050,11 @@ void launch_g2p_fused(const DevState& d, const SubParams& p, uint32_t n_tiles, h
   const uint32_t g = tile_grid(max_units, p.tile_blocks);
   const bool flip = p.flip_ratio > 0.01f, bt = p.n_scenes > 0;
 #define NB_G2PT(FL, BT)                                                                                    \
-  k_g2p_tile<FL, BT><<<g, 256, 0, s>>>(p, d.rec, d.rec, d.keys, d.materials, d.sorted, d.units, d.act_tiles, \
+  k_g2p_tile<FL, BT><<<g, 256, 0, s>>>(p, d.rec, d.rec, d.keys, d.rank, d.tile_cnt, d.materials, d.sorted, d.units, d.act_tiles, \
                                        d.tile_start, d.tile_total, d.counters, d.tile_act, d.partial, d.sdf, \
                                        d.colliders, d.forces)
   {
-    ProfScope ps(pf, 11, s);
+    ProfScope ps(pf, 8, s);
     if (bt) {
       if (flip) NB_G2PT(true, true); else NB_G2PT(false, true);
     } else {
@@ -1764,32 +2062,27 @@ void launch_g2p_fused(const DevState& d, const SubParams& p, uint32_t n_tiles, h
     }
   }
 #undef NB_G2PT
-  launch_g2p_fb(d, p, d.rec, s, pf);
 }
 
-// The FP64 fallback's fix-up after a G2P (nothing to do when it is off).
+// The FP64 fallback's fix-up after a call's last G2P, which leaves its queue
+// empty (nothing to do when it is off).
 void launch_g2p_fb(const DevState& d, const SubParams& p, float4* rec, hipStream_t s, Prof* pf) {
   if (!p.svd_fp64) return;
-  ProfScope ps(pf, 12, s);
-  // a fixed grid, at most one thread per particle, that strides over the
-  // queue: 4096 blocks give every entry its own thread up to a queue of a
-  // million (a block past the queue's end only reads the 64 lengths)
-  const uint32_t g = std::min(cdiv(p.n, 256u), 4096u);
-  if (p.n_scenes > 0)
-    k_g2p_fb<true><<<g, 256, 0, s>>>(p, rec, d.materials);
-  else
-    k_g2p_fb<false><<<g, 256, 0, s>>>(p, rec, d.materials);
+  ProfScope ps(pf, 9, s);
+  launch_fb_entries(d, p, rec, s);
   k_g2p_fb_reset<<<1, 64, 0, s>>>(p.fb_ctl);
 }
 
-void launch_g2p(const DevState& d, const SubParams& p, bool use_sorted, hipStream_t s, Prof* pf, float4* rec_out) {
+void launch_g2p(const DevState& d, const SubParams& p, bool use_sorted, bool count, hipStream_t s, Prof* pf,
+                float4* rec_out) {
+  uint32_t* tile_cnt = count ? d.tile_cnt : nullptr;
   const uint32_t* srt = use_sorted ? d.sorted : nullptr;
   float4* out = rec_out ? rec_out : d.rec;
   const bool flip = p.flip_ratio > 0.01f, bt = p.n_scenes > 0;
   {
-    ProfScope ps(pf, 10, s);
+    ProfScope ps(pf, 7, s);
 #define NB_G2P_LAUNCH(FL, BT) \
-  k_g2p<FL, BT><<<cdiv(p.n, bs), bs, 0, s>>>(p, d.rec, out, d.keys, d.materials, srt, d.grid_node, d.grid_old, d.sdf)
+  k_g2p<FL, BT><<<cdiv(p.n, bs), bs, 0, s>>>(p, d.rec, out, d.keys, d.rank, tile_cnt, d.materials, srt, d.grid_node, d.grid_old, d.sdf)
     const uint32_t bs = (p.g2p_block == 64u || p.g2p_block == 128u) ? p.g2p_block : 256u;  // launch bound 256
     if (bt) {
       if (flip) NB_G2P_LAUNCH(true, true);
@@ -1800,7 +2093,6 @@ void launch_g2p(const DevState& d, const SubParams& p, bool use_sorted, hipStrea
     }
 #undef NB_G2P_LAUNCH
   }
-  launch_g2p_fb(d, p, out, s, pf);
 }
 
 // ---------------------------------------------------------------------------

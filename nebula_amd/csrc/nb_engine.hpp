@@ -7,8 +7,8 @@
 //              which the ABI exposes, and the working copy the kernels use:
 //              one 128-byte record per particle (the same 32 floats,
 //              reordered), converted at the API boundary
-//   bins       keys[N], rank[N], sorted[N]; cell_count/cell_end dense over the
-//              Morton cube (only occupied 8^3 tiles are ever touched)
+//   bins       keys[N], rank[N], bucket[N], sorted[N]; cell_count/cell_end dense
+//              over the Morton cube (valid in the occupied 8^3 tiles)
 //   tiles      the Morton cube cut into 8^3-cell tiles (tile id = key >> 9):
 //              per-tile flags, active-tile list, dilated node-tile list
 //   partials   per active tile, the 10^3 node box its particles reach
@@ -130,17 +130,25 @@ constexpr uint32_t kFbCtlStride = 64;
 // materials a batch's table may hold (a plain engine: NB_MAX_MATERIALS)
 constexpr uint32_t kBatchMaxMaterials = NB_MAX_BATCH_MATERIALS;
 
+// sums over 256 tiles: occupied (low) and node tiles (high half), particles
+// (low) and work units (high half), occupied tiles per class of P2G's order
+struct TileSums {
+  uint64_t lists, places;
+  uint32_t cls[4];
+};
+
 struct DevState {
   float4* field[NB_NUM_FIELDS];  // reference layout, what the ABI exposes
   float4* rec;                   // capacity * kRec: working particle records
   uint32_t* keys;
-  uint32_t* rank;
+  uint32_t* rank;         // each particle's place among its tile's, as counted
+  uint2* bucket;          // (particle, cell in tile), tile by tile
   uint32_t* sorted;
   uint32_t* cell_count;   // NT*512
   uint32_t* cell_end;     // NT*512
-  uint8_t* tile_flag;     // NT: tile holds a particle (set by the key pass)
+  uint32_t* tile_cnt;     // NT: particles per tile being counted; zero once the tile pass has read it
   uint8_t* tile_mark;     // NT: bit0 active, bit1 node tile (dilation)
-  uint64_t* blk_cnt;      // NT/256: per 256 tiles, active (low) and node (high) counts
+  TileSums* tile_sums;    // NT/256 + 1: per 256 tiles
   int32_t* tile_act;      // NT: index in act_tiles or -1
   uint32_t* act_tiles;    // NT
   uint32_t* node_tiles;   // NT
@@ -163,7 +171,7 @@ struct DevState {
 };
 
 // names of the kernels, in the order the profiler indexes them
-constexpr int kNumProfiledKernels = 13;
+constexpr int kNumProfiledKernels = 10;
 extern const char* const kKernelNames[kNumProfiledKernels];
 
 // Optional per-kernel timing: HIP events recorded around each launch on the
@@ -182,8 +190,12 @@ struct Prof {
 };
 
 // ---- launchers (mpm_kernels.hip); pf may be null ----
-// keys_valid: the previous G2P wrote every particle's key (else compute them)
-void launch_bin(const DevState& d, const SubParams& p, uint32_t n_tiles, bool keys_valid, hipStream_t s, Prof* pf);
+// what the bin starts from: the records; the keys; the keys and the tile counts
+// (tile_cnt, rank) that a G2P left
+enum class BinFrom { RECORDS, KEYS, COUNTED };
+// (the FP64 fallback's queue of the G2P before is worked off on d.rec beside it)
+void launch_bin(const DevState& d, const SubParams& p, uint32_t n_tiles, BinFrom from, hipStream_t s, Prof* pf);
+void launch_clear_counts(const DevState& d, uint32_t n_tiles, hipStream_t s);
 void launch_p2g(const DevState& d, const SubParams& p, uint32_t n_tiles, hipStream_t s, Prof* pf);
 // Sum partials into grid_node and apply the grid update (+ dense-SDF BC).
 // update=false only sums (pass-level P2G export).  tiles/count select the
@@ -191,12 +203,15 @@ void launch_p2g(const DevState& d, const SubParams& p, uint32_t n_tiles, hipStre
 void launch_grid(const DevState& d, const SubParams& p, uint32_t n_tiles, bool from_partials, bool update,
                  const uint32_t* tiles, const uint32_t* count, hipStream_t s, Prof* pf);
 // use_sorted: visit particles in bin order (else index order)
+// count: also count the particles into their next tiles (tile_cnt, rank)
+// Particles for the FP64 fallback are left in its queue: the next launch_bin
+// works it off, or launch_g2p_fb.
 // rec_out: where the updated records go (nullptr: in place over d.rec)
 // Grid update and G2P in one kernel (k_g2p_tile), from the partials P2G wrote
 // and the work units the bin listed; the grid arrays are not written.
 void launch_g2p_fused(const DevState& d, const SubParams& p, uint32_t n_tiles, hipStream_t s, Prof* pf);
 void launch_g2p_fb(const DevState& d, const SubParams& p, float4* rec, hipStream_t s, Prof* pf);
-void launch_g2p(const DevState& d, const SubParams& p, bool use_sorted, hipStream_t s, Prof* pf,
+void launch_g2p(const DevState& d, const SubParams& p, bool use_sorted, bool count, hipStream_t s, Prof* pf,
                 float4* rec_out = nullptr);
 void launch_sdf_sphere(float* sdf, const SubParams& p, float r, float cx, float cy, float cz, hipStream_t s);
 // the Morton SDF of a triangle mesh (n x 12 floats: normal, v0, v1, v2) on a grid of res cells of size cs

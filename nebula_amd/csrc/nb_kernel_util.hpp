@@ -55,6 +55,46 @@ __device__ __forceinline__ T block_exclusive_scan(T v, T* s_wave, T& total) {
   return excl;
 }
 
+// Three 64-bit scans with one set of barriers; s must hold 3 (BS/64 + 1) values.
+template <int BS>
+__device__ __forceinline__ void block_exclusive_scan3(const uint64_t (&v)[3], uint64_t* s, uint64_t (&excl)[3],
+                                                      uint64_t (&total)[3]) {
+  constexpr int NW = BS / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint64_t x[3] = {v[0], v[1], v[2]};
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      const uint64_t y = __shfl_up(x[q], d);
+      if (lane >= d) x[q] += y;
+    }
+  }
+  if (lane == 63) {
+#pragma unroll
+    for (int q = 0; q < 3; q++) s[q * (NW + 1) + wave] = x[q];
+  }
+  __syncthreads();
+  if (wave < 3) {  // wave q scans the waves' sums of value q
+    uint64_t* w = s + wave * (NW + 1);
+    const uint64_t own = lane < NW ? w[lane] : 0u;
+    uint64_t run = own;
+#pragma unroll
+    for (int d = 1; d < NW; d <<= 1) {
+      const uint64_t y = __shfl_up(run, d);
+      if (lane >= d) run += y;
+    }
+    if (lane < NW) w[lane] = run - own;
+    if (lane == NW - 1) w[NW] = run;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 3; q++) {
+    excl[q] = x[q] - v[q] + s[q * (NW + 1) + wave];
+    total[q] = s[q * (NW + 1) + NW];
+  }
+}
+
 // Workgroups are dealt to the 8 XCDs (each with its own L2) round-robin by
 // id.  Block b is given chunk xcd_chunk(b, nb) of the work, so that each XCD
 // walks one contiguous eighth of the chunks: neighbouring particles, and the
