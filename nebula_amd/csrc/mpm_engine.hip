@@ -206,6 +206,7 @@ struct nb_mpm {
     p.tile_blocks = tuning.tile_blocks;
     p.g2p_block = tuning.g2p_block;
     p.p2g_item = tuning.p2g_item;
+    p.by_item = p2g_item_waves(n_live, n_scenes, d.item_cap);
     if (batch()) {
       p.n_scenes = n_scenes;
       p.scenes = d_scenes;
@@ -654,6 +655,11 @@ int engine_alloc(nb_mpm* h, void* hip_stream) {
   if (rc == NB_OK) rc = h->alloc(&d.tile_order, h->NT);
   if (rc == NB_OK) rc = h->alloc(&d.counters, CNT_SLOTS);
   if (rc == NB_OK) rc = h->alloc(&d.partial, size_t(h->cap_tiles) * kBoxNodes);
+  d.item_cap = std::min(h->cap, kItemParticles);
+  if (rc == NB_OK) rc = h->alloc(&d.items, d.item_cap);
+  if (rc == NB_OK) rc = h->alloc(&d.cell_item, cells);
+  if (rc == NB_OK) rc = h->alloc(&d.tile_items, h->NT);
+  if (rc == NB_OK) rc = h->alloc(&d.item_sum, size_t(27) * d.item_cap);
   if (rc == NB_OK) rc = h->alloc(&d.grid_node, cells);
   if (rc == NB_OK) rc = h->alloc(&d.grid_old, cells);
   if (rc == NB_OK) rc = h->alloc(&d.materials, h->max_materials());
@@ -1395,6 +1401,7 @@ int nb_mpm_run_p2g(nb_mpm* h, float dt_sub) {
   if (h->batch()) return fail(NB_ERR_UNSUPPORTED, "%s: not available on a batch of scenes", __func__);
   if (!h->bins_valid) return fail(NB_ERR_STATE, "no bins: call nb_mpm_run_bin first");
   SubParams p = h->params(dt_sub, false);
+  p.by_item = 0;  // the bins may be older than the items
   int rc = sync_in(h);
   if (rc != NB_OK) return rc;
   if (h->n_live) {

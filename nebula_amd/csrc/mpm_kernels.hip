@@ -31,6 +31,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "nb_device_math.hpp"
 #include "nb_engine.hpp"
 #include "nb_kernel_util.hpp"
@@ -39,6 +42,23 @@ namespace nb {
 
 const char* const kKernelNames[kNumProfiledKernels] = {
     "bin_keys", "bin_tiles", "bin_compact", "bin_scatter", "bin_sort", "p2g", "grid_update", "g2p", "g2p_grid", "g2p_fb"};
+
+// ---------------------------------------------------------------------------
+// P2G's work items: a cell of up to p2g_item particles is one item, a more
+// crowded one is split into up to kMaxChunks
+// ---------------------------------------------------------------------------
+constexpr uint32_t kMaxChunks = 4;
+
+__device__ __forceinline__ uint32_t p2g_chunks(uint32_t count, uint32_t item) {
+  return count == 0u ? 0u : min((count + item - 1u) / item, kMaxChunks);
+}
+// item length groups, longest first: >= 12, 10-11, 8-9, 6-7, <= 5 particles
+constexpr uint32_t kGroups = 5;
+__device__ __forceinline__ uint32_t p2g_group(uint32_t count, uint32_t chunks) {
+  if (chunks == 0u) return 0u;
+  const uint32_t per = (count + chunks - 1u) / chunks;
+  return per >= 12u ? 0u : (per >= 10u ? 1u : (per >= 8u ? 2u : (per >= 6u ? 3u : 4u)));
+}
 
 // ---------------------------------------------------------------------------
 // BIN
@@ -162,13 +182,16 @@ __global__ __launch_bounds__(kSortThreads) void k_bin_sort(uint32_t n, const uin
                                                            const uint32_t* __restrict__ tile_total,
                                                            uint32_t* __restrict__ sorted,
                                                            const uint32_t* __restrict__ counters,
-                                                           uint32_t* __restrict__ fb_ctl) {
+                                                           uint32_t* __restrict__ fb_ctl, uint32_t p2g_item,
+                                                           uint4* __restrict__ items, uint16_t* __restrict__ cell_item,
+                                                           uint32_t* __restrict__ tile_items) {
   using E = BucketEntry<PACKED>;
   const typename E::T* bucket = reinterpret_cast<const typename E::T*>(bucket_);
   __shared__ uint32_t s_idx[kSortStage + 3];  // three words past the end, read but not counted
   __shared__ uint16_t s_cell[kSortStage];
   __shared__ uint32_t s_cur[kTileCells], s_start[kTileCells + 1];
   __shared__ uint32_t s_wave[kSortThreads / 64 + 1];
+  __shared__ uint64_t s_wave64[kSortThreads / 64 + 1];
   __shared__ uint16_t s_big[kTileCells];
   __shared__ uint32_t s_nbig;
   static_assert(kSortThreads == uint32_t(kTileCells), "one thread per cell");
@@ -206,6 +229,29 @@ __global__ __launch_bounds__(kSortThreads) void k_bin_sort(uint32_t n, const uin
     const size_t key = (size_t(act_tiles[a]) << kTileBits) + threadIdx.x;
     cell_count[key] = cnt;
     cell_end[key] = first + ex + cnt;
+    if (items != nullptr && na <= kItemTiles) {
+      // the tile's P2G work items, in the order k_p2g makes them, at the places
+      // of its first particles (an item holds at least one); the other places
+      // stay empty
+      const uint32_t chunks = p2g_chunks(cnt, p2g_item), group = p2g_group(cnt, chunks);
+      uint64_t tot64;
+      const uint64_t pre = block_exclusive_scan<kSortThreads>(uint64_t(chunks) << (12 * group), s_wave64, tot64);
+      uint32_t at = 0, n_items = 0;
+#pragma unroll
+      for (int k = 0; k < int(kGroups); k++) {
+        if (group == uint32_t(k)) at = n_items + (uint32_t(pre >> (12 * k)) & 4095u);
+        n_items += uint32_t(tot64 >> (12 * k)) & 4095u;
+      }
+      const uint32_t per = chunks ? (cnt + chunks - 1u) / chunks : 0u;
+      for (uint32_t q = 0; q < chunks; q++) {
+        const uint32_t kbeg = min(q * per, cnt), kend = min(kbeg + per, cnt);
+        items[first + at + q] = make_uint4(first + ex + kbeg, kend - kbeg, uint32_t(key), 0u);
+      }
+      cell_item[key] = uint16_t(at | (chunks << 11));
+      const uint32_t layers = __syncthreads_or(chunks == 4u) ? 4u : (__syncthreads_or(chunks == 3u) ? 3u : (__syncthreads_or(chunks == 2u) ? 2u : 1u));
+      if (threadIdx.x == 0u) tile_items[a] = n_items | (layers << 16);
+      for (uint32_t e = n_items + threadIdx.x; e < tot; e += kSortThreads) items[first + e] = make_uint4(0u, 0u, 0u, 0u);
+    }
     __syncthreads();
     if (staged) {
       each([&](typename E::T u) {
@@ -293,19 +339,6 @@ __global__ __launch_bounds__(kSortThreads) void k_bin_sort(uint32_t n, const uin
 constexpr int kP2GThreads = 256;
 constexpr uint32_t kIdxStage = 4096;  // particle indices staged in LDS per pass
 
-constexpr uint32_t kMaxChunks = 4;
-
-__device__ __forceinline__ uint32_t p2g_chunks(uint32_t count, uint32_t item) {
-  return count == 0u ? 0u : min((count + item - 1u) / item, kMaxChunks);
-}
-// item length groups, longest first: >= 12, 10-11, 8-9, 6-7, <= 5 particles
-constexpr uint32_t kGroups = 5;
-__device__ __forceinline__ uint32_t p2g_group(uint32_t count, uint32_t chunks) {
-  if (chunks == 0u) return 0u;
-  const uint32_t per = (count + chunks - 1u) / chunks;
-  return per >= 12u ? 0u : (per >= 10u ? 1u : (per >= 8u ? 2u : (per >= 6u ? 3u : 4u)));
-}
-
 // One particle's node contributions, in the factored chains described at the
 // walk below.  MASK: wx and wyz are set to zero at each node whose weight
 // (wx wy) wz the reference skips (fma(a, 0, s) leaves s as it was); every
@@ -355,7 +388,59 @@ __device__ __forceinline__ uint32_t p2g_group(uint32_t count, uint32_t chunks) {
     }                                                                                                 \
   }
 
-template <bool BATCH>
+// A tile's box from its items' sums: four blocks per tile, a node a thread.  Node
+// b of the box is reached from the cells b - (0, 1, 2) along each axis; a table
+// of the tile's cells with two empty layers on every side tells each one's
+// items.  Their sums are loaded together, then added in k_p2g's order: 256 items
+// at a time, chunk layer by chunk layer, offset by offset.
+constexpr int kTabEdge = 12, kTabCells = kTabEdge * kTabEdge * kTabEdge;
+constexpr int kMergeBlocks = 4;
+static_assert(kBoxNodes % kMergeBlocks == 0 && kBoxNodes / kMergeBlocks <= kP2GThreads, "a node a thread");
+
+__device__ __forceinline__ void p2g_merge_items(uint16_t* s_tab, uint32_t na, const P2GItems& q,
+                                                const uint32_t* __restrict__ act_tiles,
+                                                const uint32_t* __restrict__ tile_start, float4* __restrict__ partial) {
+  const int at = ((int(morton_compact(threadIdx.x >> 1)) + 2) * kTabEdge + int(morton_compact(threadIdx.x)) + 2) * kTabEdge +
+                 int(morton_compact(2u * threadIdx.x)) + 2;
+  for (uint32_t w = blockIdx.x; w < kMergeBlocks * na; w += gridDim.x) {
+    const uint32_t a = w / kMergeBlocks;
+    const uint32_t pair = reinterpret_cast<const uint32_t*>(q.cell_item + (size_t(act_tiles[a]) << kTileBits))[threadIdx.x];
+    const uint32_t ti = q.tile_items[a], start = tile_start[a];
+    __syncthreads();
+    for (int e = threadIdx.x; e < kTabCells / 2; e += kP2GThreads) reinterpret_cast<uint32_t*>(s_tab)[e] = 0u;
+    __syncthreads();
+    *reinterpret_cast<uint32_t*>(s_tab + at) = pair;  // cells 2t and 2t + 1, neighbours in x
+    __syncthreads();
+    const uint32_t batches = ((ti & 0xFFFFu) + kP2GThreads - 1u) / kP2GThreads, layers = ti >> 16;
+    if (threadIdx.x >= kBoxNodes / kMergeBlocks) continue;
+    const int e = int(w % kMergeBlocks) * (kBoxNodes / kMergeBlocks) + int(threadIdx.x);
+    const uint16_t* tab = s_tab + ((e / (kBox * kBox) + 2) * kTabEdge + (e / kBox) % kBox + 2) * kTabEdge + e % kBox + 2;
+    uint32_t t[27];
+#pragma unroll
+    for (int o = 0; o < 27; o++) t[o] = tab[-(((o / 9) * kTabEdge + (o / 3) % 3) * kTabEdge + o % 3)];
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 v[27];
+    for (uint32_t b = 0; b < batches; b++)
+      for (uint32_t l = 0; l < layers; l++) {
+        // with one layer the sums stay loaded from batch to batch
+        if (layers > 1u || b == 0u) {
+#pragma unroll
+          for (int o = 0; o < 27; o++)
+            v[o] = l < (t[o] >> 11) ? q.item_sum[size_t(o) * q.item_cap + start + (t[o] & 2047u) + l]
+                                    : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int o = 0; o < 27; o++) {
+          const bool turn = l < (t[o] >> 11) && ((t[o] & 2047u) + l) / kP2GThreads == b;
+          s.x += turn ? v[o].x : 0.f; s.y += turn ? v[o].y : 0.f;
+          s.z += turn ? v[o].z : 0.f; s.w += turn ? v[o].w : 0.f;
+        }
+      }
+    partial[size_t(a) * kBoxNodes + e] = s;
+  }
+}
+
+template <bool BATCH, bool ITEMS>
 __global__ __launch_bounds__(kP2GThreads, 2) void k_p2g(SubParams p, const float4* __restrict__ rec,
                                                      const nb_material* __restrict__ mats,
                                                      const uint32_t* __restrict__ cell_count,
@@ -366,7 +451,7 @@ __global__ __launch_bounds__(kP2GThreads, 2) void k_p2g(SubParams p, const float
                                                      const uint32_t* __restrict__ tile_start,
                                                      const uint32_t* __restrict__ tile_total,
                                                      const uint32_t* __restrict__ counters,
-                                                     float4* __restrict__ partial) {
+                                                     P2GItems items, float4* __restrict__ partial) {
   __shared__ float s_m[kBoxNodes], s_x[kBoxNodes], s_y[kBoxNodes], s_z[kBoxNodes];
   __shared__ uint16_t s_item[kTileCells * kMaxChunks];  // cell | chunk << 9
   __shared__ uint32_t s_layers;
@@ -374,8 +459,13 @@ __global__ __launch_bounds__(kP2GThreads, 2) void k_p2g(SubParams p, const float
   __shared__ uint32_t s_idx[kIdxStage];
   __shared__ uint64_t s_scan64[kP2GThreads / 64 + 1];
   __shared__ float s_rho0[BATCH ? kBatchMaxMaterials : NB_MAX_MATERIALS];
-  for (uint32_t i = threadIdx.x; i < p.material_count; i += kP2GThreads) s_rho0[i] = mats[i].rho0;
   const uint32_t na = counters[CNT_ACTIVE];
+  if (ITEMS && na <= kItemTiles) {
+    static_assert(sizeof(s_idx) >= kTabCells * sizeof(uint16_t), "the table's place");
+    p2g_merge_items(reinterpret_cast<uint16_t*>(s_idx), na, items, act_tiles, tile_start, partial);
+    return;
+  }
+  for (uint32_t i = threadIdx.x; i < p.material_count; i += kP2GThreads) s_rho0[i] = mats[i].rho0;
   const bool apic = p.flip_ratio < -0.5f;
   const uint32_t mlast = p.material_count - 1u;
 
@@ -613,6 +703,185 @@ __global__ __launch_bounds__(kP2GThreads, 2) void k_p2g(SubParams p, const float
 }
 
 #undef NB_P2G_CHAINS
+
+// P2G of small scenes: the walk over work items apart from their merge.  A block
+// per tile leaves most CUs idle (4,096 particles are 8 tiles, 85,184 are 64) and
+// walks a tile's items on one CU.  Here the bin lists the items of all tiles;
+// k_p2g_items takes 64 of them a wave, anywhere on the chip, and leaves the sums
+// of their 27 nodes in memory, item by item (432 bytes each); k_p2g then collects
+// a tile's box from them (p2g_merge_items) in the order in which it merges the
+// items of a tile that it walks itself, so a box has the same bits.  SPLIT waves
+// share an item's four sums (momentum x, y, z and mass): the walk is bound by its
+// chain of up to p2g_item particles, some 490 instructions each for all four
+// sums, 320 for two, 230 for one.  Walk and merge against the box form: 11 + 6 us
+// for 23 at 4,096 particles (SPLIT 4), 16 + 8 for 41 at 85,184 (SPLIT 2),
+// 19 + 9 for 40 at 262,144.  The merge inside the grid update, without a box
+// between, spills its 27 places (84 us at 262,144 particles).
+template <int CHM, bool BATCH>
+__device__ __forceinline__ void p2g_item_sums(const SubParams& p, const float4* __restrict__ rec, const uint4 it,
+                                              const uint32_t* __restrict__ sorted, const float* s_rho0,
+                                              float* __restrict__ out, size_t stride) {
+  constexpr bool CX = CHM & 1, CY = CHM & 2, CZ = CHM & 4, CM = CHM & 8;
+  const bool apic = p.flip_ratio < -0.5f;
+  const uint32_t mlast = p.material_count - 1u;
+  const SceneGeo g = tile_geo<BATCH>(p, it.z >> kTileBits);
+  const float D_inv = 4.f / (g.h * g.h);
+  const float inv_h = g.inv_h;
+  const uint32_t cell = it.z - g.key_base;
+  const int cx = int(morton_compact(cell)), cy = int(morton_compact(cell >> 1)), cz = int(morton_compact(cell >> 2));
+  float am[27], ax[27], ay[27], az[27];
+#pragma unroll
+  for (int o = 0; o < 27; o++) { am[o] = 0.f; ax[o] = 0.f; ay[o] = 0.f; az[o] = 0.f; }
+  // stencil, set-up and chains: those of k_p2g
+  struct Stencil {
+    Axis3 x, y, z;
+  };
+  auto stencil = [&](const float4& pp, Stencil& q) -> bool {
+    const float fx = (pp.x - g.wmin[0]) * inv_h, fy = (pp.y - g.wmin[1]) * inv_h;
+    const float fz = (pp.z - g.wmin[2]) * inv_h;
+    bool ok = axis_stencil_cell(fx, pp.x, g.wmin[0], g.h, inv_h, cx, q.x);
+    ok &= axis_stencil_cell(fy, pp.y, g.wmin[1], g.h, inv_h, cy, q.y);
+    ok &= axis_stencil_cell(fz, pp.z, g.wmin[2], g.h, inv_h, cz, q.z);
+    if (ok) {
+      auto mpos = [](const Axis3& a) { return a.w[2] > 0.f ? fminf(a.w[0], a.w[2]) : a.w[0]; };
+      return (mpos(q.x) * mpos(q.y)) * mpos(q.z) < 1.0001e-12f;
+    }
+    axis_stencil_f(fx, pp.x, g.wmin[0], g.h, inv_h, cx - 1, q.x);
+    axis_stencil_f(fy, pp.y, g.wmin[1], g.h, inv_h, cy - 1, q.y);
+    axis_stencil_f(fz, pp.z, g.wmin[2], g.h, inv_h, cz - 1, q.z);
+    return (min_positive3(q.x.w) * min_positive3(q.y.w)) * min_positive3(q.z.w) < 1.0001e-12f;
+  };
+  struct Rec {
+    float4 P, V, B0, B1, B2, T;
+  };
+  auto load = [&](Rec& r, uint32_t i) {
+    const float4* q = rec + size_t(i) * kRec;
+    r.P = q[R_P]; r.V = q[R_V];
+    r.B0 = q[R_B0]; r.B1 = q[R_B1]; r.B2 = q[R_B2];
+    r.T = q[R_T];
+  };
+  auto add = [&](const Rec& r, const Stencil& q, float keep, auto masked) {
+    constexpr bool MASK = decltype(masked)::value;
+    const uint32_t mid = __float_as_uint(r.V.w);
+    const float m = s_rho0[mid > mlast ? mlast : mid] * r.P.w * keep;
+    const float sc = apic ? m * D_inv : 0.f, st = p.dt * r.P.w * keep;
+    float mwx[3], Q[3][3], R[3][3], S[3][3];  // [sum][offset]
+    auto one = [&](int c, float b0, float b1, float b2, float t0_, float t1_, float t2_, float v) {
+      const float c0 = sc * b0, c1 = sc * b1, c2 = sc * b2, t0 = st * t0_, t1 = st * t1_, t2 = st * t2_, mv = m * v;
+#pragma unroll
+      for (int i = 0; i < 3; i++) {
+        const float wdx = q.x.w[i] * q.x.dx[i], wdz = q.z.w[i] * q.z.dx[i];
+        Q[c][i] = fmaf(-q.x.g[i], t0, wdx * c0);
+        R[c][i] = fmaf(q.y.w[i], fmaf(c1, q.y.dx[i], mv), -(q.y.g[i] * t1));
+        S[c][i] = fmaf(-q.z.g[i], t2, wdz * c2);
+      }
+    };
+    if (CX) one(0, r.B0.x, r.B1.x, r.B2.x, r.T.x, r.B0.w, r.B1.w, r.V.x);
+    if (CY) one(1, r.B0.y, r.B1.y, r.B2.y, r.B0.w, r.T.y, r.B2.w, r.V.y);
+    if (CZ) one(2, r.B0.z, r.B1.z, r.B2.z, r.B1.w, r.B2.w, r.T.z, r.V.z);
+#pragma unroll
+    for (int i = 0; i < 3; i++) mwx[i] = m * q.x.w[i];
+#pragma unroll
+    for (int kz = 0; kz < 3; kz++)
+#pragma unroll
+      for (int jy = 0; jy < 3; jy++) {
+        const float wyz = q.y.w[jy] * q.z.w[kz];
+        float P[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+          if ((CHM >> c) & 1) P[c] = fmaf(q.z.w[kz], R[c][jy], q.y.w[jy] * S[c][kz]);
+#pragma unroll
+        for (int ix = 0; ix < 3; ix++) {
+          const int o = (kz * 3 + jy) * 3 + ix;
+          float wx = q.x.w[ix], wn = wyz;
+          if (MASK) {
+            const bool live = (q.x.w[ix] * q.y.w[jy]) * q.z.w[kz] >= 1e-12f;
+            wx = live ? wx : 0.f;
+            wn = live ? wn : 0.f;
+          }
+          if (CM) am[o] = fmaf(mwx[ix], wn, am[o]);
+          if (CX) ax[o] = fmaf(wn, Q[0][ix], fmaf(wx, P[0], ax[o]));
+          if (CY) ay[o] = fmaf(wn, Q[1][ix], fmaf(wx, P[1], ay[o]));
+          if (CZ) az[o] = fmaf(wn, Q[2][ix], fmaf(wx, P[2], az[o]));
+        }
+      }
+  };
+  // the walk of k_p2g: sub-cutoff particles scaled to zero here and added
+  // after it by the masked chains; the next record is loaded while this one is
+  // scattered, its index one step before
+  const uint32_t kbeg = it.x, kend = it.x + it.y;
+  uint32_t tiny_at = 0xFFFFFFFFu;
+  bool tiny_all = false;
+  Rec next;
+  uint32_t i1 = 0;
+  if (kbeg < kend) load(next, sorted[kbeg]);
+  if (kbeg + 1u < kend) i1 = sorted[kbeg + 1u];
+  for (uint32_t k = kbeg; k < kend; k++) {
+    const Rec r = next;
+    if (k + 1u < kend) load(next, i1);
+    if (k + 2u < kend) i1 = sorted[k + 2u];
+    Stencil q;
+    const bool tiny = stencil(r.P, q);
+    if (tiny) {
+      const uint32_t off = k - kbeg;
+      if (off >= 0xFFFFu || (tiny_at >> 16) != 0xFFFFu) tiny_all = true;
+      else if ((tiny_at & 0xFFFFu) == 0xFFFFu) tiny_at = 0xFFFF0000u | off;
+      else tiny_at = (tiny_at & 0xFFFFu) | (off << 16);
+    }
+    add(r, q, tiny ? 0.f : 1.f, std::false_type{});
+  }
+  const uint32_t n_exact = tiny_all ? kend - kbeg
+                                    : ((tiny_at & 0xFFFFu) != 0xFFFFu ? 1u : 0u) + ((tiny_at >> 16) != 0xFFFFu ? 1u : 0u);
+  for (uint32_t x = 0; x < n_exact; x++) {
+    load(next, sorted[kbeg + (tiny_all ? x : (x == 0u ? (tiny_at & 0xFFFFu) : (tiny_at >> 16)))]);
+    Stencil q;
+    if (stencil(next.P, q)) add(next, q, 1.f, std::true_type{});
+  }
+#pragma unroll
+  for (int o = 0; o < 27; o++) {
+    float* w = out + size_t(o) * stride;
+    if (CHM == 15) {
+      *reinterpret_cast<float4*>(w) = make_float4(ax[o], ay[o], az[o], am[o]);
+    } else {
+      if (CX) w[0] = ax[o];
+      if (CY) w[1] = ay[o];
+      if (CZ) w[2] = az[o];
+      if (CM) w[3] = am[o];
+    }
+  }
+}
+
+// grid: SPLIT times the chunks of 64 places, the chunks padded to a multiple of
+// the XCDs so that an item's waves share an L2
+template <int SPLIT, bool BATCH>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_p2g_items(
+    SubParams p, const float4* __restrict__ rec, const nb_material* __restrict__ mats,
+    const uint32_t* __restrict__ sorted, const uint4* __restrict__ items, float4* __restrict__ item_sum,
+    uint32_t item_cap, const uint32_t* __restrict__ counters) {
+  if (counters[CNT_ACTIVE] > kItemTiles) return;
+  __shared__ float s_rho0[BATCH ? kBatchMaxMaterials : NB_MAX_MATERIALS];
+  const uint32_t chunks = gridDim.x / uint32_t(SPLIT);
+  const uint32_t slot = xcd_chunk(blockIdx.x % chunks, chunks) * 64u + threadIdx.x;
+  const uint4 it = slot < p.n ? items[slot] : make_uint4(0u, 0u, 0u, 0u);
+  for (uint32_t i = threadIdx.x; i < p.material_count; i += 64u) s_rho0[i] = mats[i].rho0;
+  __syncthreads();
+  if (it.y == 0u) return;
+  float* out = reinterpret_cast<float*>(item_sum + slot);
+  const size_t stride = size_t(item_cap) * 4u;
+  const uint32_t part = blockIdx.x / chunks;
+  if (SPLIT == 1) {
+    p2g_item_sums<15, BATCH>(p, rec, it, sorted, s_rho0, out, stride);
+  } else if (SPLIT == 2) {
+    if (part == 0u) p2g_item_sums<9, BATCH>(p, rec, it, sorted, s_rho0, out, stride);
+    else p2g_item_sums<6, BATCH>(p, rec, it, sorted, s_rho0, out, stride);
+  } else {
+    if (part == 0u) p2g_item_sums<1, BATCH>(p, rec, it, sorted, s_rho0, out, stride);
+    else if (part == 1u) p2g_item_sums<2, BATCH>(p, rec, it, sorted, s_rho0, out, stride);
+    else if (part == 2u) p2g_item_sums<4, BATCH>(p, rec, it, sorted, s_rho0, out, stride);
+    else p2g_item_sums<8, BATCH>(p, rec, it, sorted, s_rho0, out, stride);
+  }
+}
+
 
 // ---------------------------------------------------------------------------
 // GRID UPDATE
@@ -1992,25 +2261,42 @@ void launch_bin(const DevState& d, const SubParams& p, uint32_t n_tiles, BinFrom
   {
     ProfScope ps(pf, 4, s);
     uint32_t* fb_ctl = p.svd_fp64 ? p.fb_ctl : nullptr;
+    uint4* items = p.by_item ? d.items : nullptr;
     if (p.n <= kPackedParticles)
       k_bin_sort<true><<<tg, kSortThreads, 0, s>>>(p.n, d.bucket, d.cell_count, d.cell_end, d.act_tiles, d.tile_start,
-                                                   d.tile_total, d.sorted, d.counters, fb_ctl);
+                                                   d.tile_total, d.sorted, d.counters, fb_ctl, p.p2g_item, items, d.cell_item, d.tile_items);
     else
       k_bin_sort<false><<<tg, kSortThreads, 0, s>>>(p.n, d.bucket, d.cell_count, d.cell_end, d.act_tiles, d.tile_start,
-                                                    d.tile_total, d.sorted, d.counters, fb_ctl);
+                                                    d.tile_total, d.sorted, d.counters, fb_ctl, p.p2g_item, items, d.cell_item, d.tile_items);
   }
 }
 
 void launch_p2g(const DevState& d, const SubParams& p, uint32_t n_tiles, hipStream_t s, Prof* pf) {
   ProfScope ps(pf, 5, s);
-  if (p.n_scenes > 0)
-    k_p2g<true><<<tile_grid(n_tiles, p.tile_blocks), kP2GThreads, 0, s>>>(p, d.rec, d.materials, d.cell_count, d.cell_end, d.sorted,
-                                                           d.act_tiles, d.tile_order, d.tile_start, d.tile_total,
-                                                           d.counters, d.partial);
-  else
-    k_p2g<false><<<tile_grid(n_tiles, p.tile_blocks), kP2GThreads, 0, s>>>(p, d.rec, d.materials, d.cell_count, d.cell_end,
-                                                            d.sorted, d.act_tiles, d.tile_order, d.tile_start,
-                                                            d.tile_total, d.counters, d.partial);
+  const P2GItems q{d.cell_item, d.tile_items, d.item_sum, d.item_cap};
+  if (p.by_item) {
+    const uint32_t chunks = cdiv(cdiv(p.n, 64), kXCDs) * kXCDs;
+#define NB_ITEMS(SP, BT) \
+  k_p2g_items<SP, BT><<<SP * chunks, 64, 0, s>>>(p, d.rec, d.materials, d.sorted, d.items, d.item_sum, d.item_cap, d.counters)
+    if (p.by_item == 4u) {
+      if (p.n_scenes > 0) NB_ITEMS(4, true); else NB_ITEMS(4, false);
+    } else if (p.by_item == 2u) {
+      if (p.n_scenes > 0) NB_ITEMS(2, true); else NB_ITEMS(2, false);
+    } else {
+      if (p.n_scenes > 0) NB_ITEMS(1, true); else NB_ITEMS(1, false);
+    }
+#undef NB_ITEMS
+  }
+#define NB_P2G(BT, IT)                                                                                                   \
+  k_p2g<BT, IT><<<IT ? tile_grid(kMergeBlocks * n_tiles, p.tile_blocks) : tile_grid(n_tiles, p.tile_blocks), kP2GThreads, 0, \
+                  s>>>(p, d.rec, d.materials, d.cell_count, d.cell_end, d.sorted, d.act_tiles, d.tile_order,             \
+                       d.tile_start, d.tile_total, d.counters, q, d.partial)
+  if (p.n_scenes > 0) {
+    if (p.by_item) NB_P2G(true, true); else NB_P2G(true, false);
+  } else {
+    if (p.by_item) NB_P2G(false, true); else NB_P2G(false, false);
+  }
+#undef NB_P2G
 }
 
 void launch_grid(const DevState& d, const SubParams& p, uint32_t n_tiles, bool from_partials, bool update,

@@ -118,6 +118,7 @@ struct SubParams {
   uint32_t tile_blocks;
   uint32_t g2p_block;
   uint32_t p2g_item;
+  uint32_t by_item;  // > 0: P2G item by item, with so many waves an item
   uint32_t n_scenes;
   const SceneGeo* scenes;
   const uint32_t* tile_scene;
@@ -127,6 +128,34 @@ struct SubParams {
 constexpr uint32_t kFbSlots = 64;
 constexpr uint32_t kFbEntry = 5;
 constexpr uint32_t kFbCtlStride = 64;
+// P2G item by item (k_p2g_items): up to this many particles and scenes, and, as
+// the device sees it, up to kItemTiles occupied tiles.  Measured per substep of a
+// block at 8 particles a cell, box form / item form: 4,096 particles (8 tiles)
+// 54 / 52 us, 32,768 (13 tiles) 80 / 62, 65,536 (48) 87 / 70, 131,072 (70)
+// 95 / 80, 262,144 (125) 103 / 94, 393,216 (180) 115 / 113, 524,288 (216)
+// 124 / 126; at 3 a cell 65,536 (100) 67 / 64, 131,072 (180) 71 / 74: from some
+// 144 tiles on, the blocks of the box form fill the chip and the item sums'
+// traffic is what tells.  A scene that has more tiles pays 3 us for the walk's
+// empty launch; one of more particles never has it, nor a batch of more scenes
+// (a scene seldom covers fewer than 8 tiles).
+constexpr uint32_t kItemParticles = 1u << 18;
+constexpr uint32_t kItemScenes = 16;
+constexpr uint32_t kItemTiles = 144;
+// Waves that share an item's four sums (0: box form).  Us per substep with 1 / 2
+// / 4: 4,096 particles 56.9 / 54.4 / 52.1, 32,768 64.8 / 63.5 / 62.2, 65,536
+// 70.7 / 69.7 / 73.5, 85,184 84.0 / 82.7 / 83.9, 131,072 81.5 / 89.2 / 94.0:
+// more waves shorten the chain while there are SIMDs without one.
+inline uint32_t p2g_item_waves(uint32_t n, uint32_t n_scenes, uint32_t item_cap) {
+  if (n > item_cap || n_scenes > kItemScenes) return 0u;
+  return n <= 32768u ? 4u : (n <= 98304u ? 2u : 1u);
+}
+// P2G's work items and their sums
+struct P2GItems {
+  const uint16_t* cell_item;
+  const uint32_t* tile_items;
+  const float4* item_sum;
+  uint32_t item_cap;
+};
 // materials a batch's table may hold (a plain engine: NB_MAX_MATERIALS)
 constexpr uint32_t kBatchMaxMaterials = NB_MAX_BATCH_MATERIALS;
 
@@ -161,6 +190,12 @@ struct DevState {
   float4* fb_queue;       // (cap + kFbSlots) * kFbEntry: particles G2P leaves to k_g2p_fb (FP64 fallback)
   uint32_t* fb_ctl;       // kFbSlots * kFbCtlStride + 1: slot lengths (zero between substeps)
   float4* partial;        // cap_tiles * 1000
+  uint4* items;           // item_cap: P2G's work items (first place in `sorted`, particles, cell key)
+  uint16_t* cell_item;    // NT*512: a cell's first item among its tile's | items << 11
+  uint32_t* tile_items;   // NT: items of an occupied tile | chunk layers << 16
+  float4* item_sum;       // 27 * item_cap: sums per offset and item
+  uint32_t item_cap;      // particles the item buffers hold
+  uint32_t item_pad;
   float4* grid_node;      // NT*512
   float4* grid_old;       // NT*512
   float4* grid_pre;       // NT*512 or null: (momentum / mass, mass) before the update, kept for the adjoint
