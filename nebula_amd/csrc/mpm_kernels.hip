@@ -1553,9 +1553,12 @@ __device__ __forceinline__ void stage_materials(const SubParams& p, const nb_mat
 // G2P reading the updated grid from HBM, one thread per particle in bin order.
 // rec_out may equal rec_in: every record slot written is data-dependent on the
 // load of the same slot (or not read at all), so updating in place is safe.
-// 4 waves per SIMD (<= 128 VGPRs): the gather's latency needs the occupancy
+// 4 waves per SIMD (<= 128 VGPRs): the gather's latency needs the occupancy.
+// FLIP gathers a second grid and keeps 168: at 4 waves it spilled 37 registers,
+// at 3 none (85,184 particles 29.8 -> 23.5 us; a whole FLIP substep of 4.19 M
+// 1029 -> 953 us, of 262,144 132 -> 127).
 template <bool FLIP, bool BATCH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_g2p(SubParams p,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FLIP ? 3 : 4))) void k_g2p(SubParams p,
                                                                                    const float4* rec_in,
                                                                                    float4* rec_out,
                                              uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
