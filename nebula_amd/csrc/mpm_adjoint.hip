@@ -12,7 +12,8 @@
 //                  writes d/dF, the position part from G2P's weights, and the
 //                  coefficients of dL/dv_node: w A + w M_B d + M_G grad w
 //   k_adj_scatter  the coefficients scattered to a grid adjoint, tile by
-//                  tile like P2G (register sums, fixed-order LDS merge)
+//                  tile like P2G (register sums, fixed-order LDS merge; small
+//                  scenes: k_adj_cells walks the cells, k_adj_scatter merges)
 //   k_grid_bwd     per node: the grid update backwards -> dL/dp, dL/dm
 //   k_p2g_bwd      per particle: P2G backwards as a 27-node gather
 //                  -> d/dv, d/dB, d/dtau and the position part from P2G
@@ -23,6 +24,9 @@
 // gradients and Hessians.  Everything is deterministic.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <algorithm>
+#include <type_traits>
 
 #include "nb_adjoint_math.hpp"
 #include "nb_device_math.hpp"
@@ -570,7 +574,195 @@ __global__ __launch_bounds__(256) void k_g2p_bwd(SubParams p, const float4* __re
 // ---------------------------------------------------------------------------
 constexpr int kAdjThreads = 256;
 
-template <bool BATCH>
+// The 27 nodes' sums of a cell's particles [kbeg, kend) of the bin order, for
+// the components of CH (bit r: component r).  Walks of one component have registers
+// for a form without the weight cut's selects, taken by a wave with no particle on it.
+template <int CH>
+__device__ __forceinline__ void adj_cell_sums(const SceneGeo& sg, int cx, int cy, int cz, uint32_t kbeg, uint32_t kend,
+                                              const float4* __restrict__ rec, const float4* __restrict__ coef,
+                                              const uint32_t* __restrict__ sorted, float (&sum)[3][27]) {
+#pragma unroll
+  for (int rr = 0; rr < 3; rr++)
+#pragma unroll
+    for (int o = 0; o < 27; o++) sum[rr][o] = 0.f;
+  // the next particle's position and coefficients are loaded while this
+  // one is scattered
+  float4 npp, nco[kCoef];
+  auto load = [&](uint32_t kk) {
+    const uint32_t q = sorted[kk];
+    npp = rec[size_t(q) * kRec + R_P];
+    const float4* co = coef + size_t(q) * kCoef;
+#pragma unroll
+    for (int jj = 0; jj < kCoef; jj++) nco[jj] = co[jj];
+  };
+  if (kbeg < kend) load(kbeg);
+  for (uint32_t kk = kbeg; kk < kend; kk++) {
+    const float4 pp = npp;
+    float cf[kCoef * 4];
+#pragma unroll
+    for (int jj = 0; jj < kCoef; jj++) {
+      const float4 v4 = nco[jj];
+      cf[4 * jj] = v4.x; cf[4 * jj + 1] = v4.y; cf[4 * jj + 2] = v4.z; cf[4 * jj + 3] = v4.w;
+    }
+    if (kk + 1 < kend) load(kk + 1);
+    AxisD X, Y, Z;
+    axis_stencil_d(cell_coord(sg, pp.x, 0), pp.x, sg.wmin[0], sg.h, cx - 1, X);
+    axis_stencil_d(cell_coord(sg, pp.y, 1), pp.y, sg.wmin[1], sg.h, cy - 1, Y);
+    axis_stencil_d(cell_coord(sg, pp.z, 2), pp.z, sg.wmin[2], sg.h, cz - 1, Z);
+    // dL/dv_node = w (A + M_B d) + M_G grad w, factored per (y, z) row:
+    //   = wx P + (wx dx) Q + gx R  with
+    //   P = wy wz (A + dy M_B[1] + dz M_B[2]) + gy wz M_G[1] + wy gz M_G[2],
+    //   Q = wy wz M_B[0],  R = wy wz M_G[0]
+    // G2P's weight cut as its forward takes it: on a particle with a node
+    // of 0 < w < 1e-12, the nodes with (wx wy) wz < 1e-12 get nothing.
+    const uint32_t cutm = cut_mask(X.w, Y.w, Z.w, 1e-12f);
+    float wdx[3];
+#pragma unroll
+    for (int ix = 0; ix < 3; ix++) wdx[ix] = X.w[ix] * X.dx[ix];
+    auto add = [&](auto masked) {
+      constexpr bool MASK = decltype(masked)::value;
+#pragma unroll
+      for (int kz = 0; kz < 3; kz++)
+#pragma unroll
+        for (int jy = 0; jy < 3; jy++) {
+          const float wyz = Y.w[jy] * Z.w[kz], gyz = Y.g[jy] * Z.w[kz], wgz = Y.w[jy] * Z.g[kz];
+#pragma unroll
+          for (int rr = 0; rr < 3; rr++) {
+            if (!((CH >> rr) & 1)) continue;
+            const float t = fmaf(Z.dx[kz], cf[9 + rr], fmaf(Y.dx[jy], cf[6 + rr], cf[rr]));
+            const float P = fmaf(wgz, cf[18 + rr], fmaf(gyz, cf[15 + rr], wyz * t));
+            const float Q = wyz * cf[3 + rr], R = wyz * cf[12 + rr];
+#pragma unroll
+            for (int ix = 0; ix < 3; ix++) {
+              const int o = (kz * 3 + jy) * 3 + ix;
+              const float next = fmaf(X.g[ix], R, fmaf(wdx[ix], Q, fmaf(X.w[ix], P, sum[rr][o])));
+              sum[rr][o] = MASK && ((cutm >> o) & 1u) ? sum[rr][o] : next;
+            }
+          }
+        }
+    };
+    if (CH == 7 || __any(cutm != 0u)) add(std::true_type{});
+    else add(std::false_type{});
+  }
+}
+
+// Where a cell's sums stand: the cells of a wave close together, from the place of
+// the wave's first particle in the bin order on (an occupied cell holds at least
+// one, so the places of different waves do not meet).  kbeg: the cell's first
+// particle; lane: its place among its 64 cells.
+__device__ __forceinline__ uint32_t cell_place(uint32_t kbeg, bool occupied, uint32_t lane) {
+  const uint64_t below = __ballot(occupied) & ((uint64_t(1) << lane) - 1u);
+  return uint32_t(__builtin_amdgcn_readfirstlane(int(kbeg))) + uint32_t(__popcll(below));
+}
+
+// The scatter of small scenes: walk and merge apart, as in the forward's P2G.  A
+// block per tile (61 us at 32,768 particles: two batches of 256 cells, each a chain
+// over its fullest cell and 27 barrier phases) uses a quarter of the CUs or less
+// there.  Here a wave takes 64 cells of a tile, anywhere on the chip, and leaves
+// their nodes' sums in memory; k_adj_scatter collects the boxes in the order in
+// which it adds the cells of a tile it walks itself, so the bits are the same.  A
+// lane walks a cell of its own, so the chain over the fullest cell bounds it;
+// SPLIT = 3 waves share the three components: 20 + 7 us at 32,768 particles
+// (27 + 7 with one wave for all three).
+template <int SPLIT, bool BATCH>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_adj_cells(
+    SubParams p, const float4* __restrict__ rec, const float4* __restrict__ coef,
+    const uint32_t* __restrict__ cell_count, const uint32_t* __restrict__ cell_end,
+    const uint32_t* __restrict__ sorted, const uint32_t* __restrict__ act_tiles,
+    const uint32_t* __restrict__ counters, float4* __restrict__ cell_sum, uint32_t stride) {
+  constexpr uint32_t kWaves = kTileCells / 64;
+  const uint32_t na = counters[CNT_ACTIVE];
+  if (na > kAdjItemTiles) return;
+  for (uint32_t w = blockIdx.x; w < SPLIT * kWaves * na; w += gridDim.x) {
+    const uint32_t part = w / (kWaves * na), v = w % (kWaves * na);
+    const uint32_t a = v / kWaves, c = (v % kWaves) * 64u + threadIdx.x;
+    const uint32_t T = act_tiles[a];
+    const size_t key = (size_t(T) << kTileBits) + c;
+    const uint32_t kend = cell_end[key], cnt = cell_count[key];
+    const uint32_t place = cell_place(kend - cnt, cnt != 0u, threadIdx.x);
+    if (cnt == 0u) continue;
+    const SceneGeo sg = tile_geo<BATCH>(p, T);
+    int tx, ty, tz;
+    tile_coords(sg, T, tx, ty, tz);
+    const int cx = tx * 8 + int(morton_compact(c)), cy = ty * 8 + int(morton_compact(c >> 1));
+    const int cz = tz * 8 + int(morton_compact(c >> 2));
+    float sum[3][27];
+    float4* out = cell_sum + place;
+    if (SPLIT == 1) {
+      adj_cell_sums<7>(sg, cx, cy, cz, kend - cnt, kend, rec, coef, sorted, sum);
+#pragma unroll
+      for (int o = 0; o < 27; o++) out[size_t(o) * stride] = make_float4(sum[0][o], sum[1][o], sum[2][o], 0.f);
+    } else if (part == 0u) {
+      adj_cell_sums<1>(sg, cx, cy, cz, kend - cnt, kend, rec, coef, sorted, sum);
+#pragma unroll
+      for (int o = 0; o < 27; o++) out[size_t(o) * stride].x = sum[0][o];
+    } else if (part == 1u) {
+      adj_cell_sums<2>(sg, cx, cy, cz, kend - cnt, kend, rec, coef, sorted, sum);
+#pragma unroll
+      for (int o = 0; o < 27; o++) out[size_t(o) * stride].y = sum[1][o];
+    } else {
+      adj_cell_sums<4>(sg, cx, cy, cz, kend - cnt, kend, rec, coef, sorted, sum);
+#pragma unroll
+      for (int o = 0; o < 27; o++) out[size_t(o) * stride].z = sum[2][o];
+    }
+  }
+}
+
+// A tile's box from its cells' sums: four blocks per tile, a node a thread, as in
+// the forward's merge.  The table holds 0 for an empty cell, else 1 + the place of
+// its sums, and whether it is among the cells that k_adj_scatter would add in its
+// second batch of 256.
+constexpr int kTabEdge = 12, kTabCells = kTabEdge * kTabEdge * kTabEdge;
+constexpr int kMergeBlocks = 4;
+constexpr uint32_t kSecond = 0x80000000u;
+
+__device__ __forceinline__ void adj_merge_cells(uint32_t* s_tab, uint32_t* s_wave, uint32_t na,
+                                                const uint32_t* __restrict__ cell_count,
+                                                const uint32_t* __restrict__ cell_end,
+                                                const uint32_t* __restrict__ act_tiles,
+                                                const float4* __restrict__ cell_sum, uint32_t stride,
+                                                float4* __restrict__ partial_adj) {
+  static_assert(kTileCells == 2 * kAdjThreads, "two cells a thread");
+  for (uint32_t w = blockIdx.x; w < kMergeBlocks * na; w += gridDim.x) {
+    const uint32_t a = w / kMergeBlocks;
+    const size_t tbase = size_t(act_tiles[a]) << kTileBits;
+    uint32_t base = 0;
+    __syncthreads();
+    for (int e = threadIdx.x; e < kTabCells; e += kAdjThreads) s_tab[e] = 0u;
+    for (uint32_t c = threadIdx.x; c < uint32_t(kTileCells); c += kAdjThreads) {
+      const uint32_t cnt = cell_count[tbase + c], place = cell_place(cell_end[tbase + c] - cnt, cnt != 0u, threadIdx.x & 63u);
+      uint32_t n_occ;
+      const uint32_t rank = base + block_exclusive_scan<kAdjThreads>(uint32_t(cnt != 0u), s_wave, n_occ);
+      base += n_occ;
+      __syncthreads();
+      if (cnt != 0u)
+        s_tab[((int(morton_compact(c >> 2)) + 2) * kTabEdge + int(morton_compact(c >> 1)) + 2) * kTabEdge +
+              int(morton_compact(c)) + 2] = (place + 1u) | (rank >= uint32_t(kAdjThreads) ? kSecond : 0u);
+    }
+    __syncthreads();
+    if (threadIdx.x >= kBoxNodes / kMergeBlocks) continue;
+    const int e = int(w % kMergeBlocks) * (kBoxNodes / kMergeBlocks) + int(threadIdx.x);
+    const uint32_t* tab = s_tab + ((e / (kBox * kBox) + 2) * kTabEdge + (e / kBox) % kBox + 2) * kTabEdge + e % kBox + 2;
+    uint32_t t[27];
+    float4 v[27];
+#pragma unroll
+    for (int o = 0; o < 27; o++) t[o] = tab[-(((o / 9) * kTabEdge + (o / 3) % 3) * kTabEdge + o % 3)];
+#pragma unroll
+    for (int o = 0; o < 27; o++)
+      v[o] = t[o] ? cell_sum[size_t(o) * stride + (t[o] & ~kSecond) - 1u] : make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t b = 0; b < (base > uint32_t(kAdjThreads) ? 2u : 1u); b++) {
+#pragma unroll
+      for (int o = 0; o < 27; o++) {
+        const bool turn = t[o] >> 31 == b;
+        s.x += turn ? v[o].x : 0.f; s.y += turn ? v[o].y : 0.f; s.z += turn ? v[o].z : 0.f;
+      }
+    }
+    partial_adj[size_t(a) * kBoxNodes + e] = s;
+  }
+}
+
+template <bool BATCH, bool CELLS>
 __global__ __launch_bounds__(kAdjThreads) void k_adj_scatter(SubParams p, const float4* __restrict__ rec,
                                                              const float4* __restrict__ coef,
                                                              const uint32_t* __restrict__ cell_count,
@@ -579,11 +771,19 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_scatter(SubParams p, const 
                                                              const uint32_t* __restrict__ act_tiles,
                                                              const uint32_t* __restrict__ tile_order,
                                                              const uint32_t* __restrict__ counters,
+                                                             const float4* __restrict__ cell_sum, uint32_t stride,
                                                              float4* __restrict__ partial_adj) {
-  __shared__ float s_x[kBoxNodes], s_y[kBoxNodes], s_z[kBoxNodes];
+  __shared__ float s_box[3 * kBoxNodes];
+  float *s_x = s_box, *s_y = s_box + kBoxNodes, *s_z = s_box + 2 * kBoxNodes;
   __shared__ uint16_t s_cell[kTileCells];
   __shared__ uint32_t s_wave[kAdjThreads / 64 + 1];
   const uint32_t na = counters[CNT_ACTIVE];
+  if (CELLS && na <= kAdjItemTiles) {
+    static_assert(sizeof(s_box) >= kTabCells * sizeof(uint32_t), "the table's place");
+    adj_merge_cells(reinterpret_cast<uint32_t*>(s_box), s_wave, na, cell_count, cell_end, act_tiles, cell_sum, stride,
+                    partial_adj);
+    return;
+  }
   for (uint32_t a0 = blockIdx.x; a0 < na; a0 += gridDim.x) {
     // largest tiles first, as in the forward's P2G
     const uint32_t ao = tile_order[a0], a = ao < na ? ao : a0;
@@ -611,66 +811,8 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_scatter(SubParams p, const 
         kend = cell_end[tbase + c];
         kbeg = kend - cell_count[tbase + c];
       }
-      float ax[27], ay[27], az[27];
-#pragma unroll
-      for (int o = 0; o < 27; o++) { ax[o] = 0.f; ay[o] = 0.f; az[o] = 0.f; }
-      // the next particle's position and coefficients are loaded while this
-      // one is scattered
-      float4 npp, nco[kCoef];
-      auto load = [&](uint32_t kk) {
-        const uint32_t q = sorted[kk];
-        npp = rec[size_t(q) * kRec + R_P];
-        const float4* co = coef + size_t(q) * kCoef;
-#pragma unroll
-        for (int jj = 0; jj < kCoef; jj++) nco[jj] = co[jj];
-      };
-      if (kbeg < kend) load(kbeg);
-      for (uint32_t kk = kbeg; kk < kend; kk++) {
-        const float4 pp = npp;
-        float cf[kCoef * 4];
-#pragma unroll
-        for (int jj = 0; jj < kCoef; jj++) {
-          const float4 v4 = nco[jj];
-          cf[4 * jj] = v4.x; cf[4 * jj + 1] = v4.y; cf[4 * jj + 2] = v4.z; cf[4 * jj + 3] = v4.w;
-        }
-        if (kk + 1 < kend) load(kk + 1);
-        AxisD X, Y, Z;
-        axis_stencil_d(cell_coord(sg, pp.x, 0), pp.x, sg.wmin[0], sg.h, cx - 1, X);
-        axis_stencil_d(cell_coord(sg, pp.y, 1), pp.y, sg.wmin[1], sg.h, cy - 1, Y);
-        axis_stencil_d(cell_coord(sg, pp.z, 2), pp.z, sg.wmin[2], sg.h, cz - 1, Z);
-        // dL/dv_node = w (A + M_B d) + M_G grad w, factored per (y, z) row:
-        //   = wx P + (wx dx) Q + gx R  with
-        //   P = wy wz (A + dy M_B[1] + dz M_B[2]) + gy wz M_G[1] + wy gz M_G[2],
-        //   Q = wy wz M_B[0],  R = wy wz M_G[0]
-        // G2P's weight cut as its forward takes it: on a particle with a node
-        // of 0 < w < 1e-12, the nodes with (wx wy) wz < 1e-12 get nothing.
-        const uint32_t cutm = cut_mask(X.w, Y.w, Z.w, 1e-12f);
-        float wdx[3];
-#pragma unroll
-        for (int ix = 0; ix < 3; ix++) wdx[ix] = X.w[ix] * X.dx[ix];
-#pragma unroll
-        for (int kz = 0; kz < 3; kz++)
-#pragma unroll
-          for (int jy = 0; jy < 3; jy++) {
-            const float wyz = Y.w[jy] * Z.w[kz], gyz = Y.g[jy] * Z.w[kz], wgz = Y.w[jy] * Z.g[kz];
-            float P[3], Q[3], R[3];
-#pragma unroll
-            for (int rr = 0; rr < 3; rr++) {
-              const float t = fmaf(Z.dx[kz], cf[9 + rr], fmaf(Y.dx[jy], cf[6 + rr], cf[rr]));
-              P[rr] = fmaf(wgz, cf[18 + rr], fmaf(gyz, cf[15 + rr], wyz * t));
-              Q[rr] = wyz * cf[3 + rr];
-              R[rr] = wyz * cf[12 + rr];
-            }
-#pragma unroll
-            for (int ix = 0; ix < 3; ix++) {
-              const int o = (kz * 3 + jy) * 3 + ix;
-              const bool cut = (cutm >> o) & 1u;
-              ax[o] = cut ? ax[o] : fmaf(X.g[ix], R[0], fmaf(wdx[ix], Q[0], fmaf(X.w[ix], P[0], ax[o])));
-              ay[o] = cut ? ay[o] : fmaf(X.g[ix], R[1], fmaf(wdx[ix], Q[1], fmaf(X.w[ix], P[1], ay[o])));
-              az[o] = cut ? az[o] : fmaf(X.g[ix], R[2], fmaf(wdx[ix], Q[2], fmaf(X.w[ix], P[2], az[o])));
-            }
-          }
-      }
+      float sum[3][27];
+      adj_cell_sums<7>(sg, cx, cy, cz, kbeg, kend, rec, coef, sorted, sum);
 #pragma unroll
       for (int kz = 0; kz < 3; kz++)
 #pragma unroll
@@ -680,7 +822,7 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_scatter(SubParams p, const 
             const int o = (kz * 3 + jy) * 3 + ix;
             const int e = ((lz + kz) * kBox + (ly + jy)) * kBox + (lx + ix);
             __syncthreads();
-            if (have) { s_x[e] += ax[o]; s_y[e] += ay[o]; s_z[e] += az[o]; }
+            if (have) { s_x[e] += sum[0][o]; s_y[e] += sum[1][o]; s_z[e] += sum[2][o]; }
           }
       __syncthreads();
     }
@@ -963,9 +1105,21 @@ static void adjoint_kernels(const DevState& d, const AdjState& a, const SubParam
   const uint32_t nblk = cdiv_a(p.n, 256);
   k_g2p_bwd<BATCH><<<nblk, 256, 0, s>>>(p, d.rec, adj_in, adj_out, a.coef, a.pg_acc,
                                          d.materials, d.sorted, d.grid_node, d.sdf);
-  k_adj_scatter<BATCH><<<tile_grid_a(n_tiles, p.tile_blocks), kAdjThreads, 0, s>>>(p, d.rec, a.coef, d.cell_count, d.cell_end,
-                                                                    d.sorted, d.act_tiles, d.tile_order, d.counters,
-                                                                    a.partial_adj);
+  const uint32_t waves = adj_cell_waves(p.n, p.n_scenes, d.item_cap);
+  const uint32_t cell_blocks = std::min((kTileCells / 64u) * std::max(waves, 1u) * n_tiles, 2048u);
+#define NB_ADJ_CELLS(SP)                                                                                               \
+  k_adj_cells<SP, BATCH><<<cell_blocks, 64, 0, s>>>(p, d.rec, a.coef, d.cell_count, d.cell_end, d.sorted, d.act_tiles, \
+                                                    d.counters, d.item_sum, d.item_cap)
+#define NB_ADJ_SCATTER(CL)                                                                                               \
+  k_adj_scatter<BATCH, CL><<<tile_grid_a((CL ? kMergeBlocks : 1u) * n_tiles, p.tile_blocks), kAdjThreads, 0, s>>>(       \
+      p, d.rec, a.coef, d.cell_count, d.cell_end, d.sorted, d.act_tiles, d.tile_order, d.counters, d.item_sum, d.item_cap, \
+      a.partial_adj)
+  if (waves == 3u) NB_ADJ_CELLS(3);
+  else if (waves == 1u) NB_ADJ_CELLS(1);
+  if (waves) NB_ADJ_SCATTER(true);
+  else NB_ADJ_SCATTER(false);
+#undef NB_ADJ_CELLS
+#undef NB_ADJ_SCATTER
   if (p.noise_forces)
     k_grid_bwd<BATCH, true><<<tile_grid_a(n_tiles, p.tile_blocks), 512, 0, s>>>(
         p, d.grid_pre, a.partial_adj, d.tile_act, d.node_tiles, d.counters + CNT_NODE_TILES, a.grid_adj, d.sdf, d.forces);

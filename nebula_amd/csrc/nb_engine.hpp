@@ -193,7 +193,7 @@ struct DevState {
   uint4* items;           // item_cap: P2G's work items (first place in `sorted`, particles, cell key)
   uint16_t* cell_item;    // NT*512: a cell's first item among its tile's | items << 11
   uint32_t* tile_items;   // NT: items of an occupied tile | chunk layers << 16
-  float4* item_sum;       // 27 * item_cap: sums per offset and item
+  float4* item_sum;       // 27 * item_cap: sums per offset and item (in the adjoint: per offset and cell)
   uint32_t item_cap;      // particles the item buffers hold
   uint32_t item_pad;
   float4* grid_node;      // NT*512
@@ -262,6 +262,18 @@ void launch_soa_to_aos_ptrs(const FieldPtrs& f, float4* rec, uint32_t n, hipStre
 void launch_aos_to_soa_ptrs(const float4* rec, const FieldPtrs& f, uint32_t n, hipStream_t s);
 
 // Buffers of the reverse-mode substep (mpm_adjoint.hip).
+// The adjoint's scatter cell by cell (k_adj_cells): waves that share a cell's three
+// components, 0 for the box form; on the device up to kAdjItemTiles tiles.  A
+// gradient of 20 substeps with 0 / 1 / 3 waves, ms: 8,000 particles 5.66 / 5.74 /
+// 5.54, 32,768 7.64 / 7.11 / 6.96, 110,592 8.23 / 7.76 / 7.69; batches of 2 scenes
+// (65,536) 4.17 / 3.62 / 3.49, 4 (131,072) 4.77 / 4.25 / 4.26, 6 (196,608) 5.72 /
+// 5.30 / 5.45, 16 (524,288) 8.87 / 8.88 / 9.12.  At 256 tiles walk and merge (45 +
+// 14 us) are even with the boxes (62).
+constexpr uint32_t kAdjItemTiles = 256;
+inline uint32_t adj_cell_waves(uint32_t n, uint32_t n_scenes, uint32_t item_cap) {
+  if (n > item_cap || n_scenes > kItemScenes) return 0u;
+  return n <= 131072u ? 3u : 1u;
+}
 struct AdjState {
   float4* coef;         // capacity * 6: per-particle grid-adjoint coefficients
   float4* partial_adj;  // cap_tiles * kBoxNodes: per-tile grid-adjoint boxes
