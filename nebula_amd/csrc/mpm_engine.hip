@@ -62,6 +62,37 @@ int set_error(int code, const char* fmt, ...) {
 }
 }  // namespace nb
 
+// Device buffers cut from one allocation: an allocation and its release cost some
+// 10 us on the host, which for the 72 buffers of a recording of five substeps' tape
+// was 0.8 ms of a 5.8 ms gradient (20 substeps of 32,768 particles).  Buffers whose
+// device pointers are handed out are not cut but allocated one by one (h->alloc),
+// so that a handed-out pointer is an allocation's own.
+struct Carve {
+  struct Part {
+    void* p;  // address of the pointer to set
+    size_t bytes;
+  };
+  std::vector<Part> parts;
+  template <class T>
+  void add(T** p, size_t count) {
+    parts.push_back({p, (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256});
+  }
+  int commit(std::vector<void*>& owner) const {
+    size_t total = 0;
+    for (const Part& r : parts) total += r.bytes;
+    void* base = nullptr;
+    hipError_t e = hipMalloc(&base, total);
+    if (e != hipSuccess) return fail(NB_ERR_HIP, "hipMalloc(%zu) failed: %s", total, hipGetErrorString(e));
+    owner.push_back(base);
+    char* at = static_cast<char*>(base);
+    for (const Part& r : parts) {
+      std::memcpy(r.p, &at, sizeof(at));
+      at += r.bytes;
+    }
+    return NB_OK;
+  }
+};
+
 struct nb_mpm {
   nb_mpm_config cfg{};
   nb_mpm_knobs knobs{};
@@ -143,6 +174,8 @@ struct nb_mpm {
     // and ends, tile lists) at t seg + j: the backward reads them instead of
     // binning again
     std::vector<DevState> slot_bins;  // n_tapes * seg
+    uint32_t* slot_tiles = nullptr;   // their six tile lists, each of all slots
+    uint32_t* slot_counters = nullptr;
     float4* adj_a = nullptr;  // cap * kRec
     float4* adj_b = nullptr;
     float4* field[NB_NUM_FIELDS] = {};  // adjoint in the reference layout
@@ -563,9 +596,6 @@ int nb_mpm_create_batch(const nb_mpm_scene* scenes, uint32_t n_scenes, void* hip
   h->scenes_host = geo;
   h->scene_first = first;
   int rc = engine_alloc(h, hip_stream);
-  if (rc == NB_OK) rc = h->alloc(&h->d_scenes, n_scenes);
-  if (rc == NB_OK) rc = h->alloc(&h->d_tile_scene, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&h->d_pscene, h->cap);
   if (rc != NB_OK) return cleanup_fail(rc);
   {
     std::vector<uint32_t> ts(h->NT), ps(std::max(h->cap, 1u));
@@ -636,39 +666,46 @@ int engine_alloc(nb_mpm* h, void* hip_stream) {
   const size_t cells = size_t(h->NT) * kTileCells;
   int rc = NB_OK;
   for (int f = 0; f < NB_NUM_FIELDS && rc == NB_OK; f++) rc = h->alloc(&d.field[f], h->cap);
-  if (rc == NB_OK) rc = h->alloc(&d.rec, size_t(h->cap) * kRec);
-  if (rc == NB_OK) rc = h->alloc(&d.keys, h->cap);
-  if (rc == NB_OK) rc = h->alloc(&d.rank, h->cap);
-  if (rc == NB_OK) rc = h->alloc(&d.sorted, h->cap);
-  if (rc == NB_OK) rc = h->alloc(&d.cell_count, cells);
-  if (rc == NB_OK) rc = h->alloc(&d.cell_end, cells);
-  if (rc == NB_OK) rc = h->alloc(&d.bucket, h->cap);
-  if (rc == NB_OK) rc = h->alloc(&d.tile_cnt, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&d.tile_mark, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&d.tile_sums, (h->NT + 255) / 256 + 1);
-  if (rc == NB_OK) rc = h->alloc(&d.tile_act, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&d.act_tiles, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&d.node_tiles, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&d.all_tiles, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&d.tile_total, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&d.tile_start, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&d.tile_order, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&d.counters, CNT_SLOTS);
-  if (rc == NB_OK) rc = h->alloc(&d.partial, size_t(h->cap_tiles) * kBoxNodes);
+  Carve c;
+  c.add(&d.rec, size_t(h->cap) * kRec);
+  c.add(&d.keys, h->cap);
+  c.add(&d.rank, h->cap);
+  c.add(&d.sorted, h->cap);
+  c.add(&d.cell_count, cells);
+  c.add(&d.cell_end, cells);
+  c.add(&d.bucket, h->cap);
+  c.add(&d.tile_cnt, h->NT);
+  c.add(&d.tile_mark, h->NT);
+  c.add(&d.tile_sums, (h->NT + 255) / 256 + 1);
+  c.add(&d.tile_act, h->NT);
+  c.add(&d.act_tiles, h->NT);
+  c.add(&d.node_tiles, h->NT);
+  c.add(&d.all_tiles, h->NT);
+  c.add(&d.tile_total, h->NT);
+  c.add(&d.tile_start, h->NT);
+  c.add(&d.tile_order, h->NT);
+  c.add(&d.counters, CNT_SLOTS);
+  c.add(&d.partial, size_t(h->cap_tiles) * kBoxNodes);
   d.item_cap = std::min(h->cap, kItemParticles);
-  if (rc == NB_OK) rc = h->alloc(&d.items, d.item_cap);
-  if (rc == NB_OK) rc = h->alloc(&d.cell_item, cells);
-  if (rc == NB_OK) rc = h->alloc(&d.tile_items, h->NT);
-  if (rc == NB_OK) rc = h->alloc(&d.item_sum, size_t(27) * d.item_cap);
-  if (rc == NB_OK) rc = h->alloc(&d.grid_node, cells);
-  if (rc == NB_OK) rc = h->alloc(&d.grid_old, cells);
-  if (rc == NB_OK) rc = h->alloc(&d.materials, h->max_materials());
-  if (rc == NB_OK) rc = h->alloc(&d.colliders, NB_MAX_COLLIDERS);
-  if (rc == NB_OK) rc = h->alloc(&d.forces, NB_MAX_FORCES);
-  if (rc == NB_OK) rc = h->alloc(&h->d_svd_stats, NB_SVD_FB_STATS);
-  if (rc == NB_OK) rc = h->alloc(&d.units, size_t(h->NT) + h->cap / kG2PUnit + 1);
-  if (rc == NB_OK) rc = h->alloc(&d.fb_queue, (size_t(h->cap) + kFbSlots) * kFbEntry);
-  if (rc == NB_OK) rc = h->alloc(&d.fb_ctl, kFbSlots * kFbCtlStride + 1);
+  c.add(&d.items, d.item_cap);
+  c.add(&d.cell_item, cells);
+  c.add(&d.tile_items, h->NT);
+  c.add(&d.item_sum, size_t(27) * d.item_cap);
+  c.add(&d.grid_node, cells);
+  c.add(&d.grid_old, cells);
+  c.add(&d.materials, h->max_materials());
+  c.add(&d.colliders, NB_MAX_COLLIDERS);
+  c.add(&d.forces, NB_MAX_FORCES);
+  c.add(&h->d_svd_stats, NB_SVD_FB_STATS);
+  c.add(&d.units, size_t(h->NT) + h->cap / kG2PUnit + 1);
+  c.add(&d.fb_queue, (size_t(h->cap) + kFbSlots) * kFbEntry);
+  c.add(&d.fb_ctl, kFbSlots * kFbCtlStride + 1);
+  if (h->batch()) {
+    c.add(&h->d_scenes, h->n_scenes);
+    c.add(&h->d_tile_scene, h->NT);
+    c.add(&h->d_pscene, h->cap);
+  }
+  if (rc == NB_OK) rc = c.commit(h->allocs);
   if (rc != NB_OK) return rc;
   d.sdf = nullptr;
 
@@ -685,8 +722,8 @@ int engine_alloc(nb_mpm* h, void* hip_stream) {
       return fail(NB_ERR_HIP, "hipMemsetAsync failed");
   if (hipMemsetAsync(d.tile_act, 0xFF, size_t(h->NT) * 4, h->stream) != hipSuccess)
     return fail(NB_ERR_HIP, "hipMemsetAsync failed");
-  launch_fill_identity(d.all_tiles, h->NT, h->stream);
-  launch_fill_identity(d.tile_order, h->NT, h->stream);
+  launch_fill_identity(d.all_tiles, 1, h->NT, h->stream);
+  launch_fill_identity(d.tile_order, 1, h->NT, h->stream);
   {
     uint32_t all = h->NT;
     if (hipMemcpyAsync(d.counters + CNT_ALL_TILES, &all, 4, hipMemcpyHostToDevice, h->stream) != hipSuccess ||
@@ -1637,26 +1674,40 @@ int adj_alloc(nb_mpm* h, T** p, size_t count) {
   *p = reinterpret_cast<T*>(q);
   return NB_OK;
 }
-// one set of bin buffers, in the state a fresh engine's bins start in
-int adj_alloc_bins(nb_mpm* h, DevState& b) {
-  const size_t cells = size_t(h->NT) * kTileCells;
-  int rc = NB_OK;
-  if (rc == NB_OK) rc = adj_alloc(h, &b.sorted, h->cap);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.cell_count, cells);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.cell_end, cells);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.tile_act, h->NT);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.act_tiles, h->NT);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.node_tiles, h->NT);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.tile_total, h->NT);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.tile_start, h->NT);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.tile_order, h->NT);
-  if (rc == NB_OK) rc = adj_alloc(h, &b.counters, CNT_SLOTS);
-  if (rc == NB_OK &&
-      (hipMemsetAsync(b.counters, 0, CNT_SLOTS * 4, h->stream) != hipSuccess ||
-       hipMemsetAsync(b.tile_act, 0xFF, size_t(h->NT) * 4, h->stream) != hipSuccess))
-    rc = fail(NB_ERR_HIP, "hipMemsetAsync failed");
-  if (rc == NB_OK) launch_fill_identity(b.tile_order, h->NT, h->stream);
-  return rc;
+// the bin buffers of all tape slots; the tile lists and counters of each stand in
+// one array, `stride` apart, to be cleared by one call (adj_clear_bins)
+size_t adj_tile_stride(const nb_mpm* h) { return (size_t(h->NT) + 63) / 64 * 64; }
+void adj_add_bins(nb_mpm* h, Carve& c, size_t slots) {
+  auto& A = h->adj;
+  A.slot_bins.assign(slots, DevState{});
+  for (DevState& b : A.slot_bins) {
+    c.add(&b.sorted, h->cap);
+    c.add(&b.cell_count, size_t(h->NT) * kTileCells);
+    c.add(&b.cell_end, size_t(h->NT) * kTileCells);
+  }
+  c.add(&A.slot_tiles, 6 * slots * adj_tile_stride(h));
+  c.add(&A.slot_counters, slots * CNT_SLOTS);
+}
+// in the state a fresh engine's bins start in
+int adj_clear_bins(nb_mpm* h) {
+  auto& A = h->adj;
+  const size_t slots = A.slot_bins.size(), stride = adj_tile_stride(h);
+  uint32_t* all[6];
+  for (int k = 0; k < 6; k++) all[k] = A.slot_tiles + size_t(k) * slots * stride;
+  for (size_t j = 0; j < slots; j++) {
+    DevState& b = A.slot_bins[j];
+    b.tile_act = reinterpret_cast<int32_t*>(all[0] + j * stride);
+    b.tile_order = all[1] + j * stride;
+    b.act_tiles = all[2] + j * stride;
+    b.node_tiles = all[3] + j * stride;
+    b.tile_total = all[4] + j * stride;
+    b.tile_start = all[5] + j * stride;
+    b.counters = A.slot_counters + j * CNT_SLOTS;
+  }
+  NB_HIP(hipMemsetAsync(A.slot_counters, 0, slots * CNT_SLOTS * 4, h->stream));
+  NB_HIP(hipMemsetAsync(all[0], 0xFF, slots * stride * 4, h->stream));
+  launch_fill_identity(all[1], uint32_t(slots), uint32_t(stride), h->stream);
+  return NB_OK;
 }
 void adj_free(nb_mpm* h) {
   if (h->stream) (void)hipStreamSynchronize(h->stream);
@@ -1748,37 +1799,32 @@ int nb_mpm_adjoint_begin_tapes(nb_mpm* h, uint32_t n_substeps, uint32_t segment,
   }
   A.n_tapes = std::min(tapes, A.n_ckpt);
   const uint32_t n_blocks = (h->cap + 255u) / 256u;  // blocks of the G2P backward
-  int rc = NB_OK;
-  if (rc == NB_OK) rc = adj_alloc(h, &A.ckpt, rec * A.n_ckpt);
-  if (rc == NB_OK) rc = adj_alloc(h, &A.tape, rec * (A.seg - 1) * A.n_tapes);
-  float4* kc = nullptr;
-  float4* kt = nullptr;
-  if (rc == NB_OK) rc = adj_alloc(h, &kc, (size_t(h->cap) * A.n_ckpt + 3) / 4);
-  if (rc == NB_OK) rc = adj_alloc(h, &kt, (size_t(h->cap) * (A.seg - 1) * A.n_tapes + 3) / 4);
-  if (rc == NB_OK) rc = adj_alloc(h, &A.grid_tape, size_t(A.seg) * A.n_tapes * 2 * h->NT * kTileCells);
-  A.slot_bins.assign(size_t(A.seg) * A.n_tapes, DevState{});
-  for (size_t j = 0; j < A.slot_bins.size() && rc == NB_OK; j++) rc = adj_alloc_bins(h, A.slot_bins[j]);
   A.tape_seg.assign(A.n_tapes, -1);
-  if (rc == NB_OK) rc = adj_alloc(h, &A.adj_a, rec);
-  if (rc == NB_OK) rc = adj_alloc(h, &A.adj_b, rec);
-  for (int f = 0; f < NB_NUM_FIELDS && rc == NB_OK; f++) rc = adj_alloc(h, &A.field[f], h->cap);
-  if (rc == NB_OK) rc = adj_alloc(h, &A.a.coef, size_t(h->cap) * 6);
-  if (rc == NB_OK) rc = adj_alloc(h, &A.a.partial_adj, size_t(h->cap_tiles) * kBoxNodes);
-  if (rc == NB_OK) rc = adj_alloc(h, &A.a.grid_adj, size_t(h->NT) * kTileCells);
-  float4* pg = nullptr;
   A.a.pg_materials = std::max(h->material_count, 1u);
-  if (rc == NB_OK) rc = adj_alloc(h, &A.a.pg_acc, size_t(n_blocks) * A.a.pg_materials);
-  if (rc == NB_OK) rc = adj_alloc(h, &A.a.pg_chunk, size_t(h->max_materials()) * ((n_blocks + 63) / 64));
-  if (rc == NB_OK) rc = adj_alloc(h, &pg, h->max_materials());
+  Carve c;
+  c.add(&A.ckpt, rec * A.n_ckpt);
+  c.add(&A.tape, rec * (A.seg - 1) * A.n_tapes);
+  c.add(&A.ckpt_keys, size_t(h->cap) * A.n_ckpt);
+  c.add(&A.tape_keys, size_t(h->cap) * (A.seg - 1) * A.n_tapes);
+  c.add(&A.grid_tape, size_t(A.seg) * A.n_tapes * 2 * h->NT * kTileCells);
+  adj_add_bins(h, c, size_t(A.seg) * A.n_tapes);
+  c.add(&A.adj_a, rec);
+  c.add(&A.adj_b, rec);
+  c.add(&A.a.coef, size_t(h->cap) * 6);
+  c.add(&A.a.partial_adj, size_t(h->cap_tiles) * kBoxNodes);
+  c.add(&A.a.grid_adj, size_t(h->NT) * kTileCells);
+  c.add(&A.a.pg_acc, size_t(n_blocks) * A.a.pg_materials);
+  c.add(&A.a.pg_chunk, size_t(h->max_materials()) * ((n_blocks + 63) / 64));
+  c.add(&A.a.pgrad, size_t(h->max_materials()) * 4);
+  int rc = c.commit(A.allocs);
+  for (int f = 0; f < NB_NUM_FIELDS && rc == NB_OK; f++) rc = adj_alloc(h, &A.field[f], h->cap);
+  if (rc == NB_OK) rc = adj_clear_bins(h);
   if (rc != NB_OK) {
     std::string keep = g_err;
     adj_free(h);
     g_err = keep;
     return rc;
   }
-  A.ckpt_keys = reinterpret_cast<uint32_t*>(kc);
-  A.tape_keys = reinterpret_cast<uint32_t*>(kt);
-  A.a.pgrad = reinterpret_cast<float*>(pg);
   for (int f = 0; f < NB_NUM_FIELDS; f++) NB_HIP(hipMemsetAsync(A.field[f], 0, size_t(h->cap) * 16, h->stream));
   NB_HIP(hipStreamSynchronize(h->stream));
   A.on = true;

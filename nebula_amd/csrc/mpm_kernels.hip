@@ -2095,9 +2095,10 @@ __global__ void k_sdf_sphere(float* __restrict__ sdf, SubParams p, float r, floa
   sdf[c] = d - r;
 }
 
+// rows of 0, 1, ..., n - 1
 __global__ void k_fill_identity(uint32_t* __restrict__ a, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = i;
+  if (i < n) a[size_t(blockIdx.y) * n + i] = i;
 }
 
 // F = I, B = 0, tau = 0 for rows [first, first+count) (appendParticles)
@@ -2669,7 +2670,10 @@ void launch_sdf_sphere(float* sdf, const SubParams& p, float r, float cx, float 
   k_sdf_sphere<<<cdiv(nc, 256), 256, 0, s>>>(sdf, p, r, cx, cy, cz);
 }
 
-void launch_fill_identity(uint32_t* a, uint32_t n, hipStream_t s) { k_fill_identity<<<cdiv(n, 256), 256, 0, s>>>(a, n); }
+void launch_fill_identity(uint32_t* a, uint32_t rows, uint32_t n, hipStream_t s) {
+  for (uint32_t r = 0; r < rows; r += 32768u)
+    k_fill_identity<<<dim3(cdiv(n, 256), std::min(rows - r, 32768u)), 256, 0, s>>>(a + size_t(r) * n, n);
+}
 
 void launch_soa_to_aos(const DevState& d, uint32_t n, hipStream_t s) {
   if (!n) return;

@@ -253,7 +253,7 @@ void launch_sdf_sphere(float* sdf, const SubParams& p, float r, float cx, float 
 // (sph: n_tris float4 of scratch)
 void launch_mesh_sdf(const float* tris, float4* sph, uint32_t n_tris, const int32_t res[3], uint32_t cube, float cs,
                      bool exact, float* sdf, hipStream_t s);
-void launch_fill_identity(uint32_t* a, uint32_t n, hipStream_t s);
+void launch_fill_identity(uint32_t* a, uint32_t rows, uint32_t n, hipStream_t s);
 void launch_init_particles(const DevState& d, uint32_t first, uint32_t count, hipStream_t s);
 void launch_copy(float4* dst, const float4* src, uint64_t n4, hipStream_t s);
 void launch_soa_to_aos(const DevState& d, uint32_t n, hipStream_t s);
