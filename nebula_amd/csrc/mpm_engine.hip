@@ -288,12 +288,15 @@ int download(nb_mpm* h, void* dst, const void* src, size_t bytes) {
 }
 
 // Refresh the particle records from the reference-layout arrays when those may
-// have changed since the records were last written back.
-int sync_in(nb_mpm* h) {
+// have changed since the records were last written back.  count: the caller
+// bins next, so the records' keys are written and counted on the way.
+int sync_in(nb_mpm* h, bool count = false) {
   if ((h->rec_stale || h->ptr_exported) && h->n_live) {
-    launch_soa_to_aos(h->d, h->n_live, h->stream);
+    if (count && h->counts_dirty) launch_clear_counts(h->d, h->NT, h->stream);
+    launch_soa_to_aos(h->d, h->params(0.f, false), count, h->stream);
     NB_HIP(hipGetLastError());
-    h->keys_valid = h->counted = false;
+    h->keys_valid = h->counted = count;
+    h->counts_dirty |= count;
   }
   h->rec_stale = false;
   return NB_OK;
@@ -403,7 +406,7 @@ int engine_alloc(nb_mpm* h, void* hip_stream);
 
 int run_substeps(nb_mpm* h, float dt, uint32_t n, Prof* pf) {
   if (n == 0 || h->n_live == 0) return NB_OK;
-  int rc = sync_in(h);
+  int rc = sync_in(h, true);
   // every substep but the last fuses the grid update into G2P; the last one
   // writes the grid, so that the grid a caller reads after the call is the
   // last substep's, as after the reference's step
@@ -804,7 +807,7 @@ int nb_mpm_set_tuning(nb_mpm* h, const nb_mpm_tuning* t) {
 int nb_mpm_graph_substeps(nb_mpm* h, float dt_sub, uint32_t n) {
   if (!h) return fail(NB_ERR_ARG, "null handle");
   if (n == 0 || h->n_live == 0) return NB_OK;
-  int rc = sync_in(h);
+  int rc = sync_in(h, true);
   // the captured substep starts from the keys and counts the previous G2P left
   // and leaves the same, and the fallback's queue, to the next
   if (rc == NB_OK && !(h->keys_valid && h->counted)) {

@@ -2116,20 +2116,45 @@ __global__ void k_init_FB(float4* F0, float4* F1, float4* F2, float4* B0, float4
 }
 
 // reference layout (eight float4 arrays) <-> one 128-byte record per particle
-__global__ __launch_bounds__(256) void k_soa_to_aos(FieldPtrs f, float4* __restrict__ rec, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float4 F0 = f.f[NB_FIELD_F0][i], F1 = f.f[NB_FIELD_F1][i], F2 = f.f[NB_FIELD_F2][i];
-  float4* r = rec + size_t(i) * kRec;
-  r[R_P] = f.f[NB_FIELD_P][i];
-  r[R_V] = f.f[NB_FIELD_V][i];
-  r[R_B0] = f.f[NB_FIELD_B0][i];
-  r[R_B1] = f.f[NB_FIELD_B1][i];
-  r[R_B2] = f.f[NB_FIELD_B2][i];
-  r[R_T] = make_float4(F0.w, F1.w, F2.w, F0.x);
-  r[R_FA] = make_float4(F0.y, F0.z, F1.x, F1.y);
-  r[R_FB] = make_float4(F1.z, F2.x, F2.y, F2.z);
+// Bound by memory.  A lane storing its particle's record would write 64 lines of 16
+// bytes an instruction (349 us for 4.19 M particles, 3.1 TB/s); the wave's 64
+// records go through LDS instead (slots rotated by the particle, so that neither
+// side meets in a bank) and leave as whole kilobytes.  COUNT: the keys and tile
+// counts of the bin, for which k_bin_keys would read the records again (126 us):
+// both together take 207 us.
+template <bool COUNT, bool BATCH>
+__global__ __launch_bounds__(256) void k_soa_to_aos(SubParams p, FieldPtrs f, float4* __restrict__ rec, uint32_t n,
+                                                    uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
+                                                    uint32_t* __restrict__ tile_cnt) {
+  __shared__ float4 s_rec[256 * kRec];
+  const uint32_t lane = threadIdx.x & 63u, first = blockIdx.x * blockDim.x + (threadIdx.x & ~63u), i = first + lane;
+  float4* s = s_rec + (threadIdx.x & ~63u) * kRec;
+  if (i < n) {
+    const float4 x = f.f[NB_FIELD_P][i];
+    const float4 F0 = f.f[NB_FIELD_F0][i], F1 = f.f[NB_FIELD_F1][i], F2 = f.f[NB_FIELD_F2][i];
+    auto put = [&](uint32_t slot, const float4 v) { s[lane * kRec + ((slot + lane) & (kRec - 1u))] = v; };
+    put(R_P, x);
+    put(R_V, f.f[NB_FIELD_V][i]);
+    put(R_B0, f.f[NB_FIELD_B0][i]);
+    put(R_B1, f.f[NB_FIELD_B1][i]);
+    put(R_B2, f.f[NB_FIELD_B2][i]);
+    put(R_T, make_float4(F0.w, F1.w, F2.w, F0.x));
+    put(R_FA, make_float4(F0.y, F0.z, F1.x, F1.y));
+    put(R_FB, make_float4(F1.z, F2.x, F2.y, F2.z));
+    if (COUNT) {
+      const uint32_t key = cell_key(particle_geo<BATCH>(p, i), x.x, x.y, x.z);
+      keys[i] = key;
+      rank[i] = count_in_tile(key, tile_cnt);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < uint32_t(kRec); k++) {
+    const uint32_t e = k * 64u + lane, r = e / kRec;
+    if (first + r < n) rec[size_t(first) * kRec + e] = s[r * kRec + ((e + r) & (kRec - 1u))];
+  }
 }
+static_assert(kRec == 8, "a record's slots rotate within eight");
 __global__ __launch_bounds__(256) void k_aos_to_soa(const float4* __restrict__ rec, FieldPtrs f, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -2675,11 +2700,14 @@ void launch_fill_identity(uint32_t* a, uint32_t rows, uint32_t n, hipStream_t s)
     k_fill_identity<<<dim3(cdiv(n, 256), std::min(rows - r, 32768u)), 256, 0, s>>>(a + size_t(r) * n, n);
 }
 
-void launch_soa_to_aos(const DevState& d, uint32_t n, hipStream_t s) {
-  if (!n) return;
+void launch_soa_to_aos(const DevState& d, const SubParams& p, bool count, hipStream_t s) {
+  if (!p.n) return;
   FieldPtrs f;
   for (int i = 0; i < NB_NUM_FIELDS; i++) f.f[i] = d.field[i];
-  k_soa_to_aos<<<cdiv(n, 256), 256, 0, s>>>(f, d.rec, n);
+  const uint32_t g = cdiv(p.n, 256);
+  if (!count) k_soa_to_aos<false, false><<<g, 256, 0, s>>>(p, f, d.rec, p.n, nullptr, nullptr, nullptr);
+  else if (p.n_scenes > 0) k_soa_to_aos<true, true><<<g, 256, 0, s>>>(p, f, d.rec, p.n, d.keys, d.rank, d.tile_cnt);
+  else k_soa_to_aos<true, false><<<g, 256, 0, s>>>(p, f, d.rec, p.n, d.keys, d.rank, d.tile_cnt);
 }
 
 void launch_aos_to_soa(const DevState& d, uint32_t n, hipStream_t s) {
@@ -2690,7 +2718,7 @@ void launch_aos_to_soa(const DevState& d, uint32_t n, hipStream_t s) {
 }
 
 void launch_soa_to_aos_ptrs(const FieldPtrs& f, float4* rec, uint32_t n, hipStream_t s) {
-  if (n) k_soa_to_aos<<<cdiv(n, 256), 256, 0, s>>>(f, rec, n);
+  if (n) k_soa_to_aos<false, false><<<cdiv(n, 256), 256, 0, s>>>(SubParams{}, f, rec, n, nullptr, nullptr, nullptr);
 }
 void launch_aos_to_soa_ptrs(const float4* rec, const FieldPtrs& f, uint32_t n, hipStream_t s) {
   if (n) k_aos_to_soa<<<cdiv(n, 256), 256, 0, s>>>(rec, f, n);

@@ -256,7 +256,8 @@ void launch_mesh_sdf(const float* tris, float4* sph, uint32_t n_tris, const int3
 void launch_fill_identity(uint32_t* a, uint32_t rows, uint32_t n, hipStream_t s);
 void launch_init_particles(const DevState& d, uint32_t first, uint32_t count, hipStream_t s);
 void launch_copy(float4* dst, const float4* src, uint64_t n4, hipStream_t s);
-void launch_soa_to_aos(const DevState& d, uint32_t n, hipStream_t s);
+// count: also the particles' keys and tile counts (d.tile_cnt is zero)
+void launch_soa_to_aos(const DevState& d, const SubParams& p, bool count, hipStream_t s);
 void launch_aos_to_soa(const DevState& d, uint32_t n, hipStream_t s);
 void launch_soa_to_aos_ptrs(const FieldPtrs& f, float4* rec, uint32_t n, hipStream_t s);
 void launch_aos_to_soa_ptrs(const float4* rec, const FieldPtrs& f, uint32_t n, hipStream_t s);
