@@ -835,8 +835,62 @@ __global__ __launch_bounds__(kAdjThreads) void k_adj_scatter(SubParams p, const 
 // ---------------------------------------------------------------------------
 // grid update backward
 // ---------------------------------------------------------------------------
-template <bool BATCH, bool NOISE>
-__global__ __launch_bounds__(512) void k_grid_bwd(SubParams p, const float4* __restrict__ grid_pre,
+// The part of a live node's backward after its forces: (vx, vy, vz) with them, pre
+// = (u, mass) before the update, sp = |u|, (gx, gy, gz) the velocity's adjoint.
+// Returns (dL/dp, dL/dm).
+__device__ __forceinline__ float4 grid_bwd_node(const SceneGeo& sg, int nx, int ny, int nz, float vx, float vy, float vz,
+                                                const float4 pre, float sp, float gx, float gy, float gz,
+                                                const float* __restrict__ sdf) {
+  const float mass = pre.w, u0x = pre.x, u0y = pre.y, u0z = pre.z;
+  const bool capped = sp > 15.f;
+  const int Nx = sg.grid_res[0] - 1, Ny = sg.grid_res[1] - 1, Nz = sg.grid_res[2] - 1;
+  bool wx = false, wy = false, wz = false;
+  if (nx <= 1 && vx < 0.f) { vx = 0.f; wx = true; }
+  if (nx >= Nx - 1 && vx > 0.f) { vx = 0.f; wx = true; }
+  if (ny <= 1 && vy < 0.f) { vy = 0.f; wy = true; }
+  if (ny >= Ny - 1 && vy > 0.f) { vy = 0.f; wy = true; }
+  if (nz <= 1 && vz < 0.f) { vz = 0.f; wz = true; }
+  if (nz >= Nz - 1 && vz > 0.f) { vz = 0.f; wz = true; }
+  bool sdf_zero = false, sdf_proj = false;
+  float ux = 0.f, uy = 0.f, uz = 0.f;
+  if (sdf) {
+    const float sd = sample_sdf(sdf, sg, nx, ny, nz);
+    if (sd < 0.f) {
+      sdf_zero = true;
+    } else if (sd < sg.h * 1.5f) {
+      const float ggx = sample_sdf(sdf, sg, nx + 1, ny, nz) - sample_sdf(sdf, sg, nx - 1, ny, nz);
+      const float ggy = sample_sdf(sdf, sg, nx, ny + 1, nz) - sample_sdf(sdf, sg, nx, ny - 1, nz);
+      const float ggz = sample_sdf(sdf, sg, nx, ny, nz + 1) - sample_sdf(sdf, sg, nx, ny, nz - 1);
+      const float gl = len3(ggx, ggy, ggz);
+      if (gl > 1e-6f) {
+        ux = ggx / gl; uy = ggy / gl; uz = ggz / gl;
+        if (vx * ux + vy * uy + vz * uz < 0.f) sdf_proj = true;
+      }
+    }
+  }
+  // backward
+  if (sdf_zero) { gx = gy = gz = 0.f; }
+  if (sdf_proj) {
+    const float gn = gx * ux + gy * uy + gz * uz;
+    gx -= gn * ux; gy -= gn * uy; gz -= gn * uz;
+  }
+  if (wx) gx = 0.f;
+  if (wy) gy = 0.f;
+  if (wz) gz = 0.f;
+  if (capped) {
+    const float hx = u0x / sp, hy = u0y / sp, hz = u0z / sp;
+    const float gh = gx * hx + gy * hy + gz * hz;
+    const float kk = 15.f / sp;
+    gx = kk * (gx - gh * hx); gy = kk * (gy - gh * hy); gz = kk * (gz - gh * hz);
+  }
+  const float im = 1.f / mass;
+  return make_float4(gx * im, gy * im, gz * im, -(gx * u0x + gy * u0y + gz * u0z) * im);
+}
+
+// with turbulence or noise: a block per node tile, whose nodes share the noise's
+// lattice points
+template <bool BATCH>
+__global__ __launch_bounds__(512) void k_grid_bwd_noise(SubParams p, const float4* __restrict__ grid_pre,
                                                   const float4* __restrict__ partial_adj,
                                                   const int32_t* __restrict__ tile_act,
                                                   const uint32_t* __restrict__ tiles, const uint32_t* __restrict__ count,
@@ -890,57 +944,54 @@ __global__ __launch_bounds__(512) void k_grid_bwd(SubParams p, const float4* __r
     if (capped) { const float kk = 15.f / sp; vx *= kk; vy *= kk; vz *= kk; }
     // forces add constants with respect to the state: they pass the adjoint
     // through, but the flags below depend on the velocity they produce
-    if constexpr (NOISE) {
-      __shared__ NoiseLds s_noise;
-      if (!__syncthreads_or(live)) continue;
-      tile_forces(vx, vy, vz, (float(nx) + 0.5f) * sg.h + sg.wmin[0], (float(ny) + 0.5f) * sg.h + sg.wmin[1],
-                  (float(nz) + 0.5f) * sg.h + sg.wmin[2], live, forces, p.force_count, p.dt, s_noise);
-    } else {
-      apply_forces(vx, vy, vz, forces, p.force_count, p.dt);
-    }
-    if (!live) continue;
-    const int Nx = sg.grid_res[0] - 1, Ny = sg.grid_res[1] - 1, Nz = sg.grid_res[2] - 1;
-    bool wx = false, wy = false, wz = false;
-    if (nx <= 1 && vx < 0.f) { vx = 0.f; wx = true; }
-    if (nx >= Nx - 1 && vx > 0.f) { vx = 0.f; wx = true; }
-    if (ny <= 1 && vy < 0.f) { vy = 0.f; wy = true; }
-    if (ny >= Ny - 1 && vy > 0.f) { vy = 0.f; wy = true; }
-    if (nz <= 1 && vz < 0.f) { vz = 0.f; wz = true; }
-    if (nz >= Nz - 1 && vz > 0.f) { vz = 0.f; wz = true; }
-    bool sdf_zero = false, sdf_proj = false;
-    float ux = 0.f, uy = 0.f, uz = 0.f;
-    if (sdf) {
-      const float sd = sample_sdf(sdf, sg, nx, ny, nz);
-      if (sd < 0.f) {
-        sdf_zero = true;
-      } else if (sd < sg.h * 1.5f) {
-        const float ggx = sample_sdf(sdf, sg, nx + 1, ny, nz) - sample_sdf(sdf, sg, nx - 1, ny, nz);
-        const float ggy = sample_sdf(sdf, sg, nx, ny + 1, nz) - sample_sdf(sdf, sg, nx, ny - 1, nz);
-        const float ggz = sample_sdf(sdf, sg, nx, ny, nz + 1) - sample_sdf(sdf, sg, nx, ny, nz - 1);
-        const float gl = len3(ggx, ggy, ggz);
-        if (gl > 1e-6f) {
-          ux = ggx / gl; uy = ggy / gl; uz = ggz / gl;
-          if (vx * ux + vy * uy + vz * uz < 0.f) sdf_proj = true;
-        }
+    __shared__ NoiseLds s_noise;
+    if (!__syncthreads_or(live)) continue;
+    tile_forces(vx, vy, vz, (float(nx) + 0.5f) * sg.h + sg.wmin[0], (float(ny) + 0.5f) * sg.h + sg.wmin[1],
+                (float(nz) + 0.5f) * sg.h + sg.wmin[2], live, forces, p.force_count, p.dt, s_noise);
+    if (live) grid_adj[nid] = grid_bwd_node(sg, nx, ny, nz, vx, vy, vz, pre, sp, gx, gy, gz, sdf);
+  }
+}
+
+// Per occupied tile, as the forward's k_grid_tiles.
+template <bool BATCH>
+__global__ __launch_bounds__(512) void k_grid_bwd(SubParams p, const float4* __restrict__ grid_pre,
+                                                  const float4* __restrict__ partial_adj,
+                                                  const int32_t* __restrict__ tile_act,
+                                                  const uint32_t* __restrict__ act_tiles,
+                                                  const uint32_t* __restrict__ counters, float4* __restrict__ grid_adj,
+                                                  const float* __restrict__ sdf, const nb_force* __restrict__ forces) {
+  __shared__ NeighbourTiles s_near;
+  const uint32_t na = counters[CNT_ACTIVE];
+  const bool split = na <= kGridSplitTiles;
+  for (uint32_t w = blockIdx.x; w < (split ? 2u * na : na); w += gridDim.x) {
+    const uint32_t T = act_tiles[w < na ? w : w - na];
+    const SceneGeo sg = tile_geo<BATCH>(p, T);
+    int tx, ty, tz;
+    tile_coords(sg, T, tx, ty, tz);
+    load_neighbours(sg, tx, ty, tz, tile_act, s_near);
+    const int last = s_near.open && (!split || w >= na) ? 1 : 0;
+#pragma unroll 1
+    for (int shell = w < na ? 0 : 1; shell <= last; shell++) {
+      int bx, by, bz;
+      float4 g;
+      if (!box_node(shell != 0, bx, by, bz) || !sum_boxes(s_near, shell != 0, bx, by, bz, partial_adj, g)) continue;
+      const int nx = tx * 8 + bx - 1, ny = ty * 8 + by - 1, nz = tz * 8 + bz - 1;
+      const size_t nid = node_id(sg, uint32_t(nx), uint32_t(ny), uint32_t(nz));
+      // the recorded forward's node state before the update: (momentum / mass, mass)
+      const float4 pre = grid_pre[nid];
+      if (pre.w < 1e-10f) {
+        grid_adj[nid] = make_float4(0.f, 0.f, 0.f, 0.f);
+        continue;
       }
+      // forward recompute (shaders/mpm_grid_update.comp:17-101, mpm_nanovdb_bc.comp:23-54)
+      const float sp = len3(pre.x, pre.y, pre.z);
+      float vx = pre.x, vy = pre.y, vz = pre.z;
+      if (sp > 15.f) { const float kk = 15.f / sp; vx *= kk; vy *= kk; vz *= kk; }
+      // forces add constants with respect to the state: they pass the adjoint
+      // through, but the flags below depend on the velocity they produce
+      apply_forces(vx, vy, vz, forces, p.force_count, p.dt);
+      grid_adj[nid] = grid_bwd_node(sg, nx, ny, nz, vx, vy, vz, pre, sp, g.x, g.y, g.z, sdf);
     }
-    // backward
-    if (sdf_zero) { gx = gy = gz = 0.f; }
-    if (sdf_proj) {
-      const float gn = gx * ux + gy * uy + gz * uz;
-      gx -= gn * ux; gy -= gn * uy; gz -= gn * uz;
-    }
-    if (wx) gx = 0.f;
-    if (wy) gy = 0.f;
-    if (wz) gz = 0.f;
-    if (capped) {
-      const float hx = u0x / sp, hy = u0y / sp, hz = u0z / sp;
-      const float gh = gx * hx + gy * hy + gz * hz;
-      const float kk = 15.f / sp;
-      gx = kk * (gx - gh * hx); gy = kk * (gy - gh * hy); gz = kk * (gz - gh * hz);
-    }
-    const float im = 1.f / mass;
-    grid_adj[nid] = make_float4(gx * im, gy * im, gz * im, -(gx * u0x + gy * u0y + gz * u0z) * im);
   }
 }
 
@@ -1121,11 +1172,11 @@ static void adjoint_kernels(const DevState& d, const AdjState& a, const SubParam
 #undef NB_ADJ_CELLS
 #undef NB_ADJ_SCATTER
   if (p.noise_forces)
-    k_grid_bwd<BATCH, true><<<tile_grid_a(n_tiles, p.tile_blocks), 512, 0, s>>>(
+    k_grid_bwd_noise<BATCH><<<tile_grid_a(n_tiles, p.tile_blocks), 512, 0, s>>>(
         p, d.grid_pre, a.partial_adj, d.tile_act, d.node_tiles, d.counters + CNT_NODE_TILES, a.grid_adj, d.sdf, d.forces);
   else
-    k_grid_bwd<BATCH, false><<<tile_grid_a(n_tiles, p.tile_blocks), 512, 0, s>>>(
-        p, d.grid_pre, a.partial_adj, d.tile_act, d.node_tiles, d.counters + CNT_NODE_TILES, a.grid_adj, d.sdf, d.forces);
+    k_grid_bwd<BATCH><<<tile_grid_a(2u * n_tiles, p.tile_blocks), 512, 0, s>>>(
+        p, d.grid_pre, a.partial_adj, d.tile_act, d.act_tiles, d.counters, a.grid_adj, d.sdf, d.forces);
   k_p2g_bwd<BATCH><<<nblk, 256, 0, s>>>(p, d.rec, adj_out, d.materials, d.sorted, a.grid_adj);
 }
 

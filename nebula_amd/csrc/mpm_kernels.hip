@@ -15,9 +15,10 @@
 //         barrier-separated phases (every thread owns a distinct node in a
 //         phase: no atomics, fixed order) and written as a per-tile partial
 //         (replaces mpm_zero_grid + mpm_p2g.comp's node-centric gather)
-//   grid  k_grid: one block per node tile; sums the <= 8 partials covering each
-//         node in a fixed order, then velocity, cap, forces, walls, analytic
-//         colliders and the dense-SDF BC in registers
+//   grid  k_grid_tiles: per occupied tile, its nodes and those around it that no
+//         other takes (with noise forces k_grid: one block per node tile); sums
+//         the <= 8 partials covering each node in a fixed order, then velocity,
+//         cap, forces, walls, analytic colliders and the dense-SDF BC in registers
 //         (replaces mpm_grid_update.comp + mpm_nanovdb_bc.comp)
 //   G2P   k_g2p: one thread per particle in bin order; 27-node gather, F update,
 //         register SVD, return map, Hencky stress, guards, advection; also
@@ -988,7 +989,10 @@ __device__ __forceinline__ void node_update(const SubParams& p, const SceneGeo& 
   node_bc(p, g, nx, ny, nz, x.x, x.y, x.z, vx, vy, vz, sdf, cols);
 }
 
-template <bool FROM_PARTIALS, bool UPDATE, bool BATCH, bool NOISE>
+// The grid update node tile by node tile: of the grid's own contents
+// (FROM_PARTIALS false), and from the boxes with turbulence or noise, whose lattice
+// points the nodes of a tile share.
+template <bool FROM_PARTIALS, bool BATCH, bool NOISE>
 __global__ __launch_bounds__(512) void k_grid(SubParams p, const float4* __restrict__ partial,
                                               const int32_t* __restrict__ tile_act, const uint32_t* __restrict__ tiles,
                                               const uint32_t* __restrict__ count, float4* __restrict__ grid_node,
@@ -1018,7 +1022,7 @@ __global__ __launch_bounds__(512) void k_grid(SubParams p, const float4* __restr
     }
     if (covered && grid_pre)
       grid_pre[nid] = mass < 1e-10f ? make_float4(0.f, 0.f, 0.f, mass) : make_float4(mx / mass, my / mass, mz / mass, mass);
-    const bool live = covered && UPDATE && !(mass < 1e-10f);
+    const bool live = covered && !(mass < 1e-10f);
     // massless nodes keep their momentum (shaders/mpm_grid_update.comp:109-110)
     if (covered && !live) grid_node[nid] = make_float4(mx, my, mz, mass);
     if constexpr (NOISE) {
@@ -1039,6 +1043,48 @@ __global__ __launch_bounds__(512) void k_grid(SubParams p, const float4* __restr
       }
     } else if (live) {
       float vx = mx / mass, vy = my / mass, vz = mz / mass, ox, oy, oz;
+      node_update(p, g, nx, ny, nz, vx, vy, vz, ox, oy, oz, sdf, cols, forces);
+      if (p.write_old) grid_old[nid] = make_float4(ox, oy, oz, 0.f);
+      grid_node[nid] = make_float4(vx, vy, vz, mass);
+    }
+  }
+}
+
+// The grid update from the boxes, per occupied tile (see NeighbourTiles).
+template <bool UPDATE, bool BATCH>
+__global__ __launch_bounds__(512) void k_grid_tiles(SubParams p, const float4* __restrict__ partial,
+                                                    const int32_t* __restrict__ tile_act,
+                                                    const uint32_t* __restrict__ act_tiles,
+                                                    const uint32_t* __restrict__ counters, float4* __restrict__ grid_node,
+                                                    float4* __restrict__ grid_old, float4* __restrict__ grid_pre,
+                                                    const float* __restrict__ sdf, const nb_collider* __restrict__ cols,
+                                                    const nb_force* __restrict__ forces) {
+  __shared__ NeighbourTiles s_near;
+  const uint32_t na = counters[CNT_ACTIVE];
+  const bool split = na <= kGridSplitTiles;
+  for (uint32_t w = blockIdx.x; w < (split ? 2u * na : na); w += gridDim.x) {
+    const uint32_t T = act_tiles[w < na ? w : w - na];
+    const SceneGeo g = tile_geo<BATCH>(p, T);
+    int tx, ty, tz;
+    tile_coords(g, T, tx, ty, tz);
+    load_neighbours(g, tx, ty, tz, tile_act, s_near);
+    const int last = s_near.open && (!split || w >= na) ? 1 : 0;
+#pragma unroll 1
+    for (int shell = w < na ? 0 : 1; shell <= last; shell++) {
+      int bx, by, bz;
+      float4 m;
+      if (!box_node(shell != 0, bx, by, bz) || !sum_boxes(s_near, shell != 0, bx, by, bz, partial, m)) continue;
+      const int nx = tx * 8 + bx - 1, ny = ty * 8 + by - 1, nz = tz * 8 + bz - 1;
+      const size_t nid = node_id(g, uint32_t(nx), uint32_t(ny), uint32_t(nz));
+      const float mass = m.w;
+      if (grid_pre)
+        grid_pre[nid] = mass < 1e-10f ? make_float4(0.f, 0.f, 0.f, mass) : make_float4(m.x / mass, m.y / mass, m.z / mass, mass);
+      // massless nodes keep their momentum (shaders/mpm_grid_update.comp:109-110)
+      if (!UPDATE || mass < 1e-10f) {
+        grid_node[nid] = m;
+        continue;
+      }
+      float vx = m.x / mass, vy = m.y / mass, vz = m.z / mass, ox, oy, oz;
       node_update(p, g, nx, ny, nz, vx, vy, vz, ox, oy, oz, sdf, cols, forces);
       if (p.write_old) grid_old[nid] = make_float4(ox, oy, oz, 0.f);
       grid_node[nid] = make_float4(vx, vy, vz, mass);
@@ -2332,27 +2378,27 @@ void launch_grid(const DevState& d, const SubParams& p, uint32_t n_tiles, bool f
                  const uint32_t* tiles, const uint32_t* count, hipStream_t s, Prof* pf) {
   ProfScope ps(pf, 6, s);
   const uint32_t g = tile_grid(n_tiles, p.tile_blocks);
-#define NB_GRID_LAUNCH(FP, UP, BT, NZ)                                                                       \
-  k_grid<FP, UP, BT, NZ><<<g, 512, 0, s>>>(p, d.partial, d.tile_act, tiles, count, d.grid_node, d.grid_old, \
+#define NB_GRID_LAUNCH(FP, BT, NZ)                                                                       \
+  k_grid<FP, BT, NZ><<<g, 512, 0, s>>>(p, d.partial, d.tile_act, tiles, count, d.grid_node, d.grid_old, \
                                            d.grid_pre, d.sdf, d.colliders, d.forces)
-  const bool nz = p.noise_forces != 0;
-  if (p.n_scenes > 0) {
-    if (from_partials && update) {
-      if (nz) NB_GRID_LAUNCH(true, true, true, true); else NB_GRID_LAUNCH(true, true, true, false);
-    } else if (from_partials) {
-      NB_GRID_LAUNCH(true, false, true, false);
+#define NB_GRID_TILES(UP, BT)                                                                                             \
+  k_grid_tiles<UP, BT><<<tile_grid(2u * n_tiles, p.tile_blocks), 512, 0, s>>>(p, d.partial, d.tile_act, d.act_tiles, d.counters, d.grid_node, d.grid_old,     \
+                                         d.grid_pre, d.sdf, d.colliders, d.forces)
+  const bool nz = p.noise_forces != 0 && update, bt = p.n_scenes > 0;
+  if (from_partials && !nz) {
+    if (bt) {
+      if (update) NB_GRID_TILES(true, true); else NB_GRID_TILES(false, true);
     } else {
-      if (nz) NB_GRID_LAUNCH(false, true, true, true); else NB_GRID_LAUNCH(false, true, true, false);
+      if (update) NB_GRID_TILES(true, false); else NB_GRID_TILES(false, false);
     }
+  } else if (bt) {
+    if (from_partials) NB_GRID_LAUNCH(true, true, true);
+    else if (nz) NB_GRID_LAUNCH(false, true, true); else NB_GRID_LAUNCH(false, true, false);
   } else {
-    if (from_partials && update) {
-      if (nz) NB_GRID_LAUNCH(true, true, false, true); else NB_GRID_LAUNCH(true, true, false, false);
-    } else if (from_partials) {
-      NB_GRID_LAUNCH(true, false, false, false);
-    } else {
-      if (nz) NB_GRID_LAUNCH(false, true, false, true); else NB_GRID_LAUNCH(false, true, false, false);
-    }
+    if (from_partials) NB_GRID_LAUNCH(true, false, true);
+    else if (nz) NB_GRID_LAUNCH(false, false, true); else NB_GRID_LAUNCH(false, false, false);
   }
+#undef NB_GRID_TILES
 #undef NB_GRID_LAUNCH
 }
 

@@ -142,6 +142,102 @@ __device__ __forceinline__ void tile_coords(const SceneGeo& g, uint32_t T, int& 
 __device__ __forceinline__ uint32_t tile_id(const SceneGeo& g, int tx, int ty, int tz) {
   return (g.key_base >> kTileBits) + morton3(uint32_t(tx), uint32_t(ty), uint32_t(tz));
 }
+// The nodes of the grid, tile by occupied tile.  A node lies in some particle's
+// stencil when an occupied tile's 10^3 box covers it.  The block of an occupied
+// tile takes its tile's 512 nodes (thread t the t-th in Morton order), then those
+// of the 488 nodes around them whose own tile is not occupied and that no occupied
+// tile before it (z, y, x ascending) covers: each covered node once.  A block per
+// tile that any box reaches (k_grid) spends most of its threads on nodes that none
+// covers, and read the covering boxes one after the other.  Bound by the latency of
+// a tile's list entries and boxes, then by memory: 43 -> 20 us for the 1,279
+// occupied tiles of 64 small scenes, 47 -> 36 for 2,385 of a terrain (4.19 M
+// particles), 18 -> 12 for 300 of 16 scenes (backward 20 -> 11).  Up to
+// kGridSplitTiles tiles, where blocks are few, a tile's own nodes and those around
+// it are two blocks: 7.6 -> 6.2 us at 128 tiles, even at 1,279 (20.3 / 21.5), 36 ->
+// 40 at 2,385.
+constexpr uint32_t kGridSplitTiles = 512;
+struct NeighbourTiles {
+  int32_t act[27];  // index of the occupied tile, -1: not occupied, -2: outside the cube
+  uint32_t open;    // some neighbour is not occupied
+};
+
+// Called by the whole block; n is in LDS.
+__device__ __forceinline__ void load_neighbours(const SceneGeo& g, int tx, int ty, int tz,
+                                                const int32_t* __restrict__ tile_act, NeighbourTiles& n) {
+  __syncthreads();
+  if (threadIdx.x < 64u) {
+    int32_t v = -2;
+    if (threadIdx.x < 27u) {
+      const int e = int(threadIdx.x), td = int(g.tile_dim);
+      const int sx = tx + e % 3 - 1, sy = ty + (e / 3) % 3 - 1, sz = tz + e / 9 - 1;
+      if (uint32_t(sx) < uint32_t(td) && uint32_t(sy) < uint32_t(td) && uint32_t(sz) < uint32_t(td))
+        v = max(tile_act[tile_id(g, sx, sy, sz)], -1);
+      n.act[e] = v;
+    }
+    const bool open = __any(v == -1);
+    if (threadIdx.x == 0u) n.open = open;
+  }
+  __syncthreads();
+}
+
+// Box coordinates of the node this thread takes: its tile's own (shell = false) or
+// one around it; false when it takes none.
+__device__ __forceinline__ bool box_node(bool shell, int& bx, int& by, int& bz) {
+  const int t = int(threadIdx.x);
+  if (!shell) {
+    bx = int(morton_compact(threadIdx.x)) + 1;
+    by = int(morton_compact(threadIdx.x >> 1)) + 1;
+    bz = int(morton_compact(threadIdx.x >> 2)) + 1;
+    return true;
+  }
+  if (t < 200) {  // the layers z = 0 and z = 9
+    bz = t < 100 ? 0 : 9;
+    by = (t % 100) / 10;
+    bx = t % 10;
+    return true;
+  }
+  const int r = (t - 200) % 36;  // the rings between them
+  bz = 1 + (t - 200) / 36;
+  by = r < 10 ? 0 : (r < 20 ? 9 : 1 + (r - 20) % 8);
+  bx = r < 20 ? r % 10 : (r < 28 ? 0 : 9);
+  return t < 488;
+}
+
+// Sum of the boxes that cover the node at box coordinates (bx, by, bz) of the tile
+// whose neighbours are n, tile by tile (z, y, x ascending); false when the node is
+// another block's.  The boxes' loads are independent: all are in flight together.
+__device__ __forceinline__ bool sum_boxes(const NeighbourTiles& n, bool shell, int bx, int by, int bz,
+                                          const float4* __restrict__ boxes, float4& sum) {
+  const int b[3] = {bx, by, bz};
+  int lo[3], own = 13;
+  bool two[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {  // covered by the tiles lo and, near a face, lo + 1 of the axis
+    lo[a] = b[a] <= 1 ? -1 : 0;
+    two[a] = b[a] <= 1 || b[a] >= 8;
+    own += (b[a] == 0 ? -1 : (b[a] == 9 ? 1 : 0)) * (a == 0 ? 1 : (a == 1 ? 3 : 9));
+  }
+  bool mine = !shell || n.act[own] == -1;
+  float4 q[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    q[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const bool in = (!(k & 1) || two[0]) && (!(k & 2) || two[1]) && (!(k & 4) || two[2]);
+    const int ox = lo[0] + (k & 1), oy = lo[1] + ((k >> 1) & 1), oz = lo[2] + (k >> 2);
+    const int32_t a = in ? n.act[(oz + 1) * 9 + (oy + 1) * 3 + ox + 1] : -1;
+    if (a >= 0) {
+      // a tile before this one covers the node
+      if (shell && (oz < 0 || (oz == 0 && (oy < 0 || (oy == 0 && ox < 0))))) mine = false;
+      if (mine) q[k] = boxes[size_t(a) * kBoxNodes + ((bz - 8 * oz) * kBox + by - 8 * oy) * kBox + bx - 8 * ox];
+    }
+  }
+  sum = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    sum.x += q[k].x; sum.y += q[k].y; sum.z += q[k].z; sum.w += q[k].w;
+  }
+  return mine;
+}
 // index of node (x, y, z) of the scene in the Morton-ordered node arrays
 __device__ __forceinline__ uint32_t node_id(const SceneGeo& g, uint32_t x, uint32_t y, uint32_t z) {
   return g.key_base + morton3(x, y, z);
