@@ -346,9 +346,16 @@ __device__ __forceinline__ float3 noise_hash33(float x, float y, float z) {  // 
   const float a = x * 127.1f + y * 311.7f + z * 74.7f;
   const float b = x * 269.5f + y * 183.3f + z * 246.1f;
   const float c = x * 113.5f + y * 271.9f + z * 124.6f;
-  return make_float3(-1.f + 2.f * gl_fract(hash_sin(a) * 43758.5453123f),
-                     -1.f + 2.f * gl_fract(hash_sin(b) * 43758.5453123f),
-                     -1.f + 2.f * gl_fract(hash_sin(c) * 43758.5453123f));
+  // one sine after the other: three side by side take the registers of the kernel
+  float h[3];
+#pragma unroll 1
+  for (int k = 0; k < 3; k++) {
+    const float v = -1.f + 2.f * gl_fract(hash_sin(k == 0 ? a : (k == 1 ? b : c)) * 43758.5453123f);
+    h[0] = k == 0 ? v : h[0];
+    h[1] = k == 1 ? v : h[1];
+    h[2] = v;
+  }
+  return make_float3(h[0], h[1], h[2]);
 }
 // value noise at (px, py, pz); grad(ox, oy, oz) is the gradient at the corner
 // (floor p) + (ox, oy, oz), o in {0, 1}
@@ -368,7 +375,9 @@ __device__ __forceinline__ float noise_value3_of(float px, float py, float pz, G
   const float nx01 = gl_mix(n[4], n[5], ux), nx11 = gl_mix(n[6], n[7], ux);
   return gl_mix(gl_mix(nx00, nx10, uy), gl_mix(nx01, nx11, uy), uz);
 }
-__device__ inline float noise_value3(float px, float py, float pz) {
+// (a call: inlined, its 24 sines would fill the instruction cache of the kernels that
+// have it for the lattice ranges that no table holds)
+__device__ __attribute__((noinline)) float noise_value3(float px, float py, float pz) {
 #pragma clang fp contract(off)
   const float ix = floorf(px), iy = floorf(py), iz = floorf(pz);
   return noise_value3_of(px, py, pz, [&](int ox, int oy, int oz) {
@@ -408,7 +417,9 @@ __device__ inline void apply_forces(float& vx, float& vy, float& vz, const nb_fo
 // so every value has the bits the node-by-node form gives.  An octave whose
 // lattice range does not fit the table (a high frequency on a coarse grid)
 // is hashed node by node.  On 57,001 sand particles (96^3, turbulence of three
-// octaves and noise of two) the grid update went from 233 to 39 us.
+// octaves and noise of two) the grid update went from 233 to 39 us, and to 29 with the
+// sines one after the other and the hashing of nodes out of line (38 registers spilled
+// and code beyond the instruction cache before).
 constexpr uint32_t kNoiseTab = 2048;    // lattice points held at a time
 constexpr uint32_t kNoisePhases = 16;   // (group of points, octave) pairs with a place in the table
 struct NoisePhase {
