@@ -887,71 +887,6 @@ __device__ __forceinline__ float4 grid_bwd_node(const SceneGeo& sg, int nx, int 
   return make_float4(gx * im, gy * im, gz * im, -(gx * u0x + gy * u0y + gz * u0z) * im);
 }
 
-// with turbulence or noise: a block per node tile, whose nodes share the noise's
-// lattice points
-template <bool BATCH>
-__global__ __launch_bounds__(512) void k_grid_bwd_noise(SubParams p, const float4* __restrict__ grid_pre,
-                                                  const float4* __restrict__ partial_adj,
-                                                  const int32_t* __restrict__ tile_act,
-                                                  const uint32_t* __restrict__ tiles, const uint32_t* __restrict__ count,
-                                                  float4* __restrict__ grid_adj, const float* __restrict__ sdf,
-                                                  const nb_force* __restrict__ forces) {
-  const uint32_t nb_tiles = *count;
-  const int lx = int(morton_compact(threadIdx.x)), ly = int(morton_compact(threadIdx.x >> 1)),
-            lz = int(morton_compact(threadIdx.x >> 2));
-  for (uint32_t b = blockIdx.x; b < nb_tiles; b += gridDim.x) {
-    const uint32_t N = tiles[b];
-    const SceneGeo sg = tile_geo<BATCH>(p, N);
-    const int td = int(sg.tile_dim);
-    int tx, ty, tz;
-    tile_coords(sg, N, tx, ty, tz);
-    const int nx = tx * 8 + lx, ny = ty * 8 + ly, nz = tz * 8 + lz;
-    const size_t nid = (size_t(N) << kTileBits) | threadIdx.x;
-    float gx = 0.f, gy = 0.f, gz = 0.f;
-    bool covered = false;
-    for (int dz = -1; dz <= 1; dz++) {
-      if ((dz < 0 && lz != 0) || (dz > 0 && lz != 7)) continue;
-      const int sz = tz + dz;
-      if (sz < 0 || sz >= td) continue;
-      for (int dy = -1; dy <= 1; dy++) {
-        if ((dy < 0 && ly != 0) || (dy > 0 && ly != 7)) continue;
-        const int sy = ty + dy;
-        if (sy < 0 || sy >= td) continue;
-        for (int dx = -1; dx <= 1; dx++) {
-          if ((dx < 0 && lx != 0) || (dx > 0 && lx != 7)) continue;
-          const int sx = tx + dx;
-          if (sx < 0 || sx >= td) continue;
-          const int32_t a = tile_act[tile_id(sg, sx, sy, sz)];
-          if (a < 0) continue;
-          const int bx = lx - 8 * dx + 1, by = ly - 8 * dy + 1, bz = lz - 8 * dz + 1;
-          const size_t e = size_t(a) * kBoxNodes + (bz * kBox + by) * kBox + bx;
-          const float4 g = partial_adj[e];
-          gx += g.x; gy += g.y; gz += g.z;
-          covered = true;
-        }
-      }
-    }
-    // the recorded forward's node state before the update: (momentum / mass, mass)
-    const float4 pre = covered ? grid_pre[nid] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float mass = pre.w;
-    const bool live = covered && !(mass < 1e-10f);
-    if (covered && !live) grid_adj[nid] = make_float4(0.f, 0.f, 0.f, 0.f);
-    // forward recompute (shaders/mpm_grid_update.comp:17-101, mpm_nanovdb_bc.comp:23-54)
-    const float u0x = pre.x, u0y = pre.y, u0z = pre.z;
-    const float sp = len3(u0x, u0y, u0z);
-    const bool capped = sp > 15.f;
-    float vx = u0x, vy = u0y, vz = u0z;
-    if (capped) { const float kk = 15.f / sp; vx *= kk; vy *= kk; vz *= kk; }
-    // forces add constants with respect to the state: they pass the adjoint
-    // through, but the flags below depend on the velocity they produce
-    __shared__ NoiseLds s_noise;
-    if (!__syncthreads_or(live)) continue;
-    tile_forces(vx, vy, vz, (float(nx) + 0.5f) * sg.h + sg.wmin[0], (float(ny) + 0.5f) * sg.h + sg.wmin[1],
-                (float(nz) + 0.5f) * sg.h + sg.wmin[2], live, forces, p.force_count, p.dt, s_noise);
-    if (live) grid_adj[nid] = grid_bwd_node(sg, nx, ny, nz, vx, vy, vz, pre, sp, gx, gy, gz, sdf);
-  }
-}
-
 // Per occupied tile, as the forward's k_grid_tiles.
 template <bool BATCH>
 __global__ __launch_bounds__(512) void k_grid_bwd(SubParams p, const float4* __restrict__ grid_pre,
@@ -993,6 +928,66 @@ __global__ __launch_bounds__(512) void k_grid_bwd(SubParams p, const float4* __r
       grid_adj[nid] = grid_bwd_node(sg, nx, ny, nz, vx, vy, vz, pre, sp, g.x, g.y, g.z, sdf);
     }
   }
+}
+
+// with turbulence or noise, as the forward's k_grid_noise
+template <uint32_t ROLES, bool BATCH>
+__device__ __forceinline__ void grid_bwd_noise(const SubParams& p, const float4* __restrict__ grid_pre,
+                                               const float4* __restrict__ partial_adj,
+                                               const int32_t* __restrict__ tile_act,
+                                               const uint32_t* __restrict__ act_tiles, uint32_t na,
+                                               float4* __restrict__ grid_adj, const float* __restrict__ sdf,
+                                               const nb_force* __restrict__ forces, NeighbourTiles& near, NoiseLds& lds,
+                                               uint64_t* s_live) {
+  constexpr uint32_t kNodes = kNoiseThreads / ROLES;
+  for (uint32_t w = blockIdx.x; w < noise_units<ROLES>() * na; w += gridDim.x) {
+    const uint32_t unit = w / na, T = act_tiles[w % na];
+    const SceneGeo sg = tile_geo<BATCH>(p, T);
+    int tx, ty, tz, b[3], lo[3], hi[3];
+    tile_coords(sg, T, tx, ty, tz);
+    load_neighbours(sg, tx, ty, tz, tile_act, near);
+    const bool shell = noise_shell<ROLES>(unit);
+    if (shell && !near.open) continue;
+    float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
+    const bool node = noise_unit_node<ROLES>(unit, int(threadIdx.x % kNodes), b, lo, hi);
+    const bool covered = node && threadIdx.x < kNodes && sum_boxes(near, shell, b[0], b[1], b[2], partial_adj, g);
+    const int nx = tx * 8 + b[0] - 1, ny = ty * 8 + b[1] - 1, nz = tz * 8 + b[2] - 1;
+    const size_t nid = covered ? node_id(sg, uint32_t(nx), uint32_t(ny), uint32_t(nz)) : 0;
+    const float4 pre = covered ? grid_pre[nid] : make_float4(0.f, 0.f, 0.f, 0.f);
+    bool live = covered && !(pre.w < 1e-10f), any;
+    if (covered && !live) grid_adj[nid] = make_float4(0.f, 0.f, 0.f, 0.f);
+    live = noise_live<ROLES>(live, s_live, any);
+    if (!any) continue;
+    // forward recompute, as in k_grid_bwd
+    const float sp = len3(pre.x, pre.y, pre.z);
+    float vx = pre.x, vy = pre.y, vz = pre.z;
+    if (sp > 15.f) { const float kk = 15.f / sp; vx *= kk; vy *= kk; vz *= kk; }
+    const float3 x = node_pos(sg, nx, ny, nz);
+    tile_forces<ROLES>(vx, vy, vz, x.x, x.y, x.z, live, node_pos(sg, tx * 8 + lo[0] - 1, ty * 8 + lo[1] - 1, tz * 8 + lo[2] - 1),
+                node_pos(sg, tx * 8 + hi[0] - 1, ty * 8 + hi[1] - 1, tz * 8 + hi[2] - 1), forces, p.force_count, p.dt,
+                lds);
+    if (live && threadIdx.x < kNodes)
+      grid_adj[nid] = grid_bwd_node(sg, nx, ny, nz, vx, vy, vz, pre, sp, g.x, g.y, g.z, sdf);
+  }}
+template <bool BATCH>
+__global__ __launch_bounds__(kNoiseThreads) void k_grid_bwd_noise(SubParams p, const float4* __restrict__ grid_pre,
+                                                                  const float4* __restrict__ partial_adj,
+                                                                  const int32_t* __restrict__ tile_act,
+                                                                  const uint32_t* __restrict__ act_tiles,
+                                                                  const uint32_t* __restrict__ counters,
+                                                                  float4* __restrict__ grid_adj,
+                                                                  const float* __restrict__ sdf,
+                                                                  const nb_force* __restrict__ forces) {
+  __shared__ NeighbourTiles s_near;
+  __shared__ NoiseLds s_noise;
+  __shared__ uint64_t s_live[2];
+  const uint32_t na = counters[CNT_ACTIVE];
+  if (na <= kNoiseSplitTiles)
+    grid_bwd_noise<4, BATCH>(p, grid_pre, partial_adj, tile_act, act_tiles, na, grid_adj, sdf, forces, s_near, s_noise,
+                             s_live);
+  else
+    grid_bwd_noise<1, BATCH>(p, grid_pre, partial_adj, tile_act, act_tiles, na, grid_adj, sdf, forces, s_near, s_noise,
+                             s_live);
 }
 
 // ---------------------------------------------------------------------------
@@ -1172,8 +1167,8 @@ static void adjoint_kernels(const DevState& d, const AdjState& a, const SubParam
 #undef NB_ADJ_CELLS
 #undef NB_ADJ_SCATTER
   if (p.noise_forces)
-    k_grid_bwd_noise<BATCH><<<tile_grid_a(n_tiles, p.tile_blocks), 512, 0, s>>>(
-        p, d.grid_pre, a.partial_adj, d.tile_act, d.node_tiles, d.counters + CNT_NODE_TILES, a.grid_adj, d.sdf, d.forces);
+    k_grid_bwd_noise<BATCH><<<tile_grid_a(noise_units<4>() * n_tiles, p.tile_blocks), kNoiseThreads, 0, s>>>(
+        p, d.grid_pre, a.partial_adj, d.tile_act, d.act_tiles, d.counters, a.grid_adj, d.sdf, d.forces);
   else
     k_grid_bwd<BATCH><<<tile_grid_a(2u * n_tiles, p.tile_blocks), 512, 0, s>>>(
         p, d.grid_pre, a.partial_adj, d.tile_act, d.act_tiles, d.counters, a.grid_adj, d.sdf, d.forces);

@@ -936,10 +936,6 @@ __device__ __forceinline__ void node_cap(float& vx, float& vy, float& vz) {
     vx *= k; vy *= k; vz *= k;
   }
 }
-__device__ __forceinline__ float3 node_pos(const SceneGeo& g, int nx, int ny, int nz) {
-  return make_float3((float(nx) + 0.5f) * g.h + g.wmin[0], (float(ny) + 0.5f) * g.h + g.wmin[1],
-                     (float(nz) + 0.5f) * g.h + g.wmin[2]);
-}
 // walls, analytic colliders and the dense SDF; (px, py, pz) is the node's position
 __device__ __forceinline__ void node_bc(const SubParams& p, const SceneGeo& g, int nx, int ny, int nz, float px,
                                         float py, float pz, float& vx, float& vy, float& vz,
@@ -989,60 +985,60 @@ __device__ __forceinline__ void node_update(const SubParams& p, const SceneGeo& 
   node_bc(p, g, nx, ny, nz, x.x, x.y, x.z, vx, vy, vz, sdf, cols);
 }
 
-// The grid update node tile by node tile: of the grid's own contents
-// (FROM_PARTIALS false), and from the boxes with turbulence or noise, whose lattice
-// points the nodes of a tile share.
-template <bool FROM_PARTIALS, bool BATCH, bool NOISE>
-__global__ __launch_bounds__(512) void k_grid(SubParams p, const float4* __restrict__ partial,
-                                              const int32_t* __restrict__ tile_act, const uint32_t* __restrict__ tiles,
+// node_update with turbulence or noise in the force list, and its stores, for a block
+// as tile_forces takes it
+template <uint32_t ROLES>
+__device__ __forceinline__ void grid_node_noise(const SubParams& p, const SceneGeo& g, int nx, int ny, int nz, size_t nid,
+                                                bool live, const float4 m, float3 first, float3 last,
+                                                float4* __restrict__ grid_node, float4* __restrict__ grid_old,
+                                                const float* __restrict__ sdf, const nb_collider* __restrict__ cols,
+                                                const nb_force* __restrict__ forces, NoiseLds& lds) {
+  const bool own = live && threadIdx.x < kNoiseThreads / ROLES;
+  float vx = 0.f, vy = 0.f, vz = 0.f;
+  if (own) {
+    vx = m.x / m.w; vy = m.y / m.w; vz = m.z / m.w;
+    node_cap(vx, vy, vz);
+    if (p.write_old) grid_old[nid] = make_float4(vx, vy, vz, 0.f);
+  }
+  const float3 x = node_pos(g, nx, ny, nz);
+  tile_forces<ROLES>(vx, vy, vz, x.x, x.y, x.z, live, first, last, forces, p.force_count, p.dt, lds);
+  if (own) {
+    node_bc(p, g, nx, ny, nz, x.x, x.y, x.z, vx, vy, vz, sdf, cols);
+    grid_node[nid] = make_float4(vx, vy, vz, m.w);
+  }
+}
+
+// The grid update of the grid's own contents, node tile by node tile.
+template <bool BATCH, bool NOISE>
+__global__ __launch_bounds__(512) void k_grid(SubParams p, const uint32_t* __restrict__ tiles,
                                               const uint32_t* __restrict__ count, float4* __restrict__ grid_node,
                                               float4* __restrict__ grid_old, float4* __restrict__ grid_pre,
                                               const float* __restrict__ sdf, const nb_collider* __restrict__ cols,
                                               const nb_force* __restrict__ forces) {
   const uint32_t nb_tiles = *count;
   // thread j holds the tile's j-th node in Morton order (contiguous in HBM)
-  const int lx = int(morton_compact(threadIdx.x)), ly = int(morton_compact(threadIdx.x >> 1)),
-            lz = int(morton_compact(threadIdx.x >> 2));
+  const uint32_t j = threadIdx.x;
   for (uint32_t b = blockIdx.x; b < nb_tiles; b += gridDim.x) {
     const uint32_t N = tiles[b];
     const SceneGeo g = tile_geo<BATCH>(p, N);
     int tx, ty, tz;
     tile_coords(g, N, tx, ty, tz);
-    const int nx = tx * 8 + lx, ny = ty * 8 + ly, nz = tz * 8 + lz;
-    const size_t nid = (size_t(N) << kTileBits) | threadIdx.x;
-    float mx = 0.f, my = 0.f, mz = 0.f, mass = 0.f;
-    // A node outside every occupied tile's box receives nothing and lies in
-    // no particle's stencil: it is not written (readers treat it as empty).
-    bool covered = true;
-    if (FROM_PARTIALS) {
-      covered = sum_partials(g, tx, ty, tz, lx, ly, lz, tile_act, partial, mx, my, mz, mass);
-    } else {
-      const float4 g4 = grid_node[nid];
-      mx = g4.x; my = g4.y; mz = g4.z; mass = g4.w;
-    }
-    if (covered && grid_pre)
-      grid_pre[nid] = mass < 1e-10f ? make_float4(0.f, 0.f, 0.f, mass) : make_float4(mx / mass, my / mass, mz / mass, mass);
-    const bool live = covered && !(mass < 1e-10f);
+    const int nx = tx * 8 + int(morton_compact(j)), ny = ty * 8 + int(morton_compact(j >> 1)),
+              nz = tz * 8 + int(morton_compact(j >> 2));
+    const size_t nid = (size_t(N) << kTileBits) | j;
+    const float4 m = grid_node[nid];
+    const float mass = m.w;
+    if (grid_pre)
+      grid_pre[nid] = mass < 1e-10f ? make_float4(0.f, 0.f, 0.f, mass) : make_float4(m.x / mass, m.y / mass, m.z / mass, mass);
     // massless nodes keep their momentum (shaders/mpm_grid_update.comp:109-110)
-    if (covered && !live) grid_node[nid] = make_float4(mx, my, mz, mass);
+    const bool live = !(mass < 1e-10f);
     if constexpr (NOISE) {
-      // the block's threads share the noise's lattice points (tile_forces)
       __shared__ NoiseLds s_noise;
       if (!__syncthreads_or(live)) continue;
-      float vx = 0.f, vy = 0.f, vz = 0.f;
-      if (live) {
-        vx = mx / mass; vy = my / mass; vz = mz / mass;
-        node_cap(vx, vy, vz);
-        if (p.write_old) grid_old[nid] = make_float4(vx, vy, vz, 0.f);
-      }
-      const float3 x = node_pos(g, nx, ny, nz);
-      tile_forces(vx, vy, vz, x.x, x.y, x.z, live, forces, p.force_count, p.dt, s_noise);
-      if (live) {
-        node_bc(p, g, nx, ny, nz, x.x, x.y, x.z, vx, vy, vz, sdf, cols);
-        grid_node[nid] = make_float4(vx, vy, vz, mass);
-      }
+      grid_node_noise<1>(p, g, nx, ny, nz, nid, live, m, node_pos(g, tx * 8, ty * 8, tz * 8),
+                      node_pos(g, tx * 8 + 7, ty * 8 + 7, tz * 8 + 7), grid_node, grid_old, sdf, cols, forces, s_noise);
     } else if (live) {
-      float vx = mx / mass, vy = my / mass, vz = mz / mass, ox, oy, oz;
+      float vx = m.x / mass, vy = m.y / mass, vz = m.z / mass, ox, oy, oz;
       node_update(p, g, nx, ny, nz, vx, vy, vz, ox, oy, oz, sdf, cols, forces);
       if (p.write_old) grid_old[nid] = make_float4(ox, oy, oz, 0.f);
       grid_node[nid] = make_float4(vx, vy, vz, mass);
@@ -1090,6 +1086,64 @@ __global__ __launch_bounds__(512) void k_grid_tiles(SubParams p, const float4* _
       grid_node[nid] = make_float4(vx, vy, vz, mass);
     }
   }
+}
+
+// The same with turbulence or noise.
+template <uint32_t ROLES, bool BATCH>
+__device__ __forceinline__ void grid_noise(const SubParams& p, const float4* __restrict__ partial,
+                                           const int32_t* __restrict__ tile_act, const uint32_t* __restrict__ act_tiles,
+                                           uint32_t na, float4* __restrict__ grid_node, float4* __restrict__ grid_old,
+                                           float4* __restrict__ grid_pre, const float* __restrict__ sdf,
+                                           const nb_collider* __restrict__ cols, const nb_force* __restrict__ forces,
+                                           NeighbourTiles& near, NoiseLds& lds, uint64_t* s_live) {
+  constexpr uint32_t kNodes = kNoiseThreads / ROLES;
+  for (uint32_t w = blockIdx.x; w < noise_units<ROLES>() * na; w += gridDim.x) {
+    const uint32_t unit = w / na, T = act_tiles[w % na];
+    const SceneGeo g = tile_geo<BATCH>(p, T);
+    int tx, ty, tz, b[3], lo[3], hi[3];
+    tile_coords(g, T, tx, ty, tz);
+    load_neighbours(g, tx, ty, tz, tile_act, near);
+    const bool shell = noise_shell<ROLES>(unit);
+    if (shell && !near.open) continue;
+    float4 m = make_float4(0.f, 0.f, 0.f, 0.f);
+    const bool node = noise_unit_node<ROLES>(unit, int(threadIdx.x % kNodes), b, lo, hi);
+    const bool covered = node && threadIdx.x < kNodes && sum_boxes(near, shell, b[0], b[1], b[2], partial, m);
+    const int nx = tx * 8 + b[0] - 1, ny = ty * 8 + b[1] - 1, nz = tz * 8 + b[2] - 1;
+    const size_t nid = covered ? node_id(g, uint32_t(nx), uint32_t(ny), uint32_t(nz)) : 0;
+    bool live = covered && !(m.w < 1e-10f), any;
+    if (covered && grid_pre)
+      grid_pre[nid] = live ? make_float4(m.x / m.w, m.y / m.w, m.z / m.w, m.w) : make_float4(0.f, 0.f, 0.f, m.w);
+    // massless nodes keep their momentum (shaders/mpm_grid_update.comp:109-110)
+    if (covered && !live) grid_node[nid] = m;
+    live = noise_live<ROLES>(live, s_live, any);
+    if (!any) continue;
+    grid_node_noise<ROLES>(p, g, nx, ny, nz, nid, live, m,
+                           node_pos(g, tx * 8 + lo[0] - 1, ty * 8 + lo[1] - 1, tz * 8 + lo[2] - 1),
+                           node_pos(g, tx * 8 + hi[0] - 1, ty * 8 + hi[1] - 1, tz * 8 + hi[2] - 1), grid_node, grid_old,
+                           sdf, cols, forces, lds);
+  }
+}
+template <bool BATCH>
+__global__ __launch_bounds__(kNoiseThreads) void k_grid_noise(SubParams p, const float4* __restrict__ partial,
+                                                              const int32_t* __restrict__ tile_act,
+                                                              const uint32_t* __restrict__ act_tiles,
+                                                              const uint32_t* __restrict__ counters,
+                                                              float4* __restrict__ grid_node,
+                                                              float4* __restrict__ grid_old,
+                                                              float4* __restrict__ grid_pre,
+                                                              const float* __restrict__ sdf,
+                                                              const nb_collider* __restrict__ cols,
+                                                              const nb_force* __restrict__ forces) {
+  __shared__ NeighbourTiles s_near;
+  __shared__ NoiseLds s_noise;
+  __shared__ uint64_t s_live[2];
+  const uint32_t na = counters[CNT_ACTIVE];
+  if (na <= kNoiseSplitTiles)
+    grid_noise<4, BATCH>(p, partial, tile_act, act_tiles, na, grid_node, grid_old, grid_pre, sdf, cols, forces, s_near,
+                         s_noise, s_live);
+  else
+    grid_noise<1, BATCH>(p, partial, tile_act, act_tiles, na, grid_node, grid_old, grid_pre, sdf, cols, forces, s_near,
+                         s_noise, s_live);
 }
 
 // ---------------------------------------------------------------------------
@@ -2378,25 +2432,29 @@ void launch_grid(const DevState& d, const SubParams& p, uint32_t n_tiles, bool f
                  const uint32_t* tiles, const uint32_t* count, hipStream_t s, Prof* pf) {
   ProfScope ps(pf, 6, s);
   const uint32_t g = tile_grid(n_tiles, p.tile_blocks);
-#define NB_GRID_LAUNCH(FP, BT, NZ)                                                                       \
-  k_grid<FP, BT, NZ><<<g, 512, 0, s>>>(p, d.partial, d.tile_act, tiles, count, d.grid_node, d.grid_old, \
-                                           d.grid_pre, d.sdf, d.colliders, d.forces)
-#define NB_GRID_TILES(UP, BT)                                                                                             \
-  k_grid_tiles<UP, BT><<<tile_grid(2u * n_tiles, p.tile_blocks), 512, 0, s>>>(p, d.partial, d.tile_act, d.act_tiles, d.counters, d.grid_node, d.grid_old,     \
-                                         d.grid_pre, d.sdf, d.colliders, d.forces)
+#define NB_GRID_LAUNCH(BT, NZ)                                                                                            \
+  k_grid<BT, NZ><<<g, 512, 0, s>>>(p, tiles, count, d.grid_node, d.grid_old, d.grid_pre, d.sdf, d.colliders, d.forces)
+#define NB_GRID_TILES(K, BLOCKS, THREADS)                                                                                 \
+  K<<<BLOCKS, THREADS, 0, s>>>(p, d.partial, d.tile_act, d.act_tiles, d.counters, d.grid_node, d.grid_old, d.grid_pre, \
+                               d.sdf, d.colliders, d.forces)
   const bool nz = p.noise_forces != 0 && update, bt = p.n_scenes > 0;
-  if (from_partials && !nz) {
+  if (from_partials && nz) {
+    const uint32_t gn = tile_grid(noise_units<4>() * n_tiles, p.tile_blocks);
+    if (bt) NB_GRID_TILES(k_grid_noise<true>, gn, kNoiseThreads);
+    else NB_GRID_TILES(k_grid_noise<false>, gn, kNoiseThreads);
+  } else if (from_partials) {
+    const uint32_t gt = tile_grid(2u * n_tiles, p.tile_blocks);
     if (bt) {
-      if (update) NB_GRID_TILES(true, true); else NB_GRID_TILES(false, true);
+      if (update) NB_GRID_TILES((k_grid_tiles<true, true>), gt, 512);
+      else NB_GRID_TILES((k_grid_tiles<false, true>), gt, 512);
     } else {
-      if (update) NB_GRID_TILES(true, false); else NB_GRID_TILES(false, false);
+      if (update) NB_GRID_TILES((k_grid_tiles<true, false>), gt, 512);
+      else NB_GRID_TILES((k_grid_tiles<false, false>), gt, 512);
     }
   } else if (bt) {
-    if (from_partials) NB_GRID_LAUNCH(true, true, true);
-    else if (nz) NB_GRID_LAUNCH(false, true, true); else NB_GRID_LAUNCH(false, true, false);
+    if (nz) NB_GRID_LAUNCH(true, true); else NB_GRID_LAUNCH(true, false);
   } else {
-    if (from_partials) NB_GRID_LAUNCH(true, false, true);
-    else if (nz) NB_GRID_LAUNCH(false, false, true); else NB_GRID_LAUNCH(false, false, false);
+    if (nz) NB_GRID_LAUNCH(false, true); else NB_GRID_LAUNCH(false, false);
   }
 #undef NB_GRID_TILES
 #undef NB_GRID_LAUNCH

@@ -238,6 +238,53 @@ __device__ __forceinline__ bool sum_boxes(const NeighbourTiles& n, bool shell, i
   }
   return mine;
 }
+// With turbulence or noise the nodes of a block share lattice points (tile_forces).
+// ROLES = 1: a block takes a tile's own nodes, or those around it, one a thread.
+// ROLES = 4: a quarter of its own (8 x 4 x 4), or one face of those around it, four
+// threads a node: ten blocks a tile, for scenes of few.  The unit's node t (box
+// coordinates, false: none) and the corners of the box its nodes lie in.
+constexpr uint32_t kNoiseThreads = 512;
+// A tile of a small scene has four quarters and about one face with nodes on it: five
+// blocks, on 256 CUs 51 tiles.  Frames of 20 substeps with ROLES 1 / 4, us: 8 tiles
+// 1777 / 1558, 12 tiles 1861 / 1653, 48 tiles (57,001 particles) 2116 / 1924, 64 tiles
+// 2316 / 2249 and, full, 2644 / 2874, 216 tiles 3881 / 4780.
+constexpr uint32_t kNoiseSplitTiles = 51;
+template <uint32_t ROLES>
+constexpr uint32_t noise_units() { return ROLES == 1u ? 2u : 10u; }
+template <uint32_t ROLES>
+__device__ __forceinline__ bool noise_shell(uint32_t unit) { return unit >= (ROLES == 1u ? 1u : 4u); }
+template <uint32_t ROLES>
+__device__ __forceinline__ bool noise_unit_node(uint32_t unit, int t, int (&n)[3], int (&first)[3], int (&last)[3]) {
+  if (ROLES == 1u) {
+    const bool shell = unit != 0u;
+    first[0] = first[1] = first[2] = shell ? 0 : 1;
+    last[0] = last[1] = last[2] = shell ? 9 : 8;
+    return box_node(shell, n[0], n[1], n[2]);
+  }
+  if (unit < 4u) {
+    const uint32_t m = unit * 128u + uint32_t(t);
+    const int hy = 4 * int(unit & 1u), hz = 4 * int(unit >> 1);
+    n[0] = int(morton_compact(m)) + 1; n[1] = int(morton_compact(m >> 1)) + 1; n[2] = int(morton_compact(m >> 2)) + 1;
+    first[0] = 1; first[1] = 1 + hy; first[2] = 1 + hz;
+    last[0] = 8; last[1] = 4 + hy; last[2] = 4 + hz;
+    return true;
+  }
+  const int side = (unit & 1u) ? 9 : 0;
+  if (unit < 6u) {  // z = 0, 9
+    n[0] = t % 10; n[1] = t / 10; n[2] = side;
+    first[0] = first[1] = 0; first[2] = last[2] = side; last[0] = last[1] = 9;
+    return t < 100;
+  }
+  if (unit < 8u) {  // y = 0, 9 between them
+    n[0] = t % 10; n[1] = side; n[2] = 1 + t / 10;
+    first[0] = 0; first[1] = last[1] = side; first[2] = 1; last[0] = 9; last[2] = 8;
+    return t < 80;
+  }
+  n[0] = side; n[1] = 1 + t % 8; n[2] = 1 + t / 8;  // x = 0, 9 between those
+  first[0] = last[0] = side; first[1] = first[2] = 1; last[1] = last[2] = 8;
+  return t < 64;
+}
+
 // index of node (x, y, z) of the scene in the Morton-ordered node arrays
 __device__ __forceinline__ uint32_t node_id(const SceneGeo& g, uint32_t x, uint32_t y, uint32_t z) {
   return g.key_base + morton3(x, y, z);
@@ -324,6 +371,12 @@ __device__ __forceinline__ void axis_stencil(float xp, float wmin, float h, floa
 __device__ __forceinline__ float sample_sdf(const float* sdf, const SceneGeo& g, int x, int y, int z) {
   if (x < 0 || y < 0 || z < 0 || x >= g.grid_res[0] || y >= g.grid_res[1] || z >= g.grid_res[2]) return 1e6f;
   return sdf[morton3(x, y, z)];
+}
+
+// position of node (nx, ny, nz)
+__device__ __forceinline__ float3 node_pos(const SceneGeo& g, int nx, int ny, int nz) {
+  return make_float3(fmaf(float(nx) + 0.5f, g.h, g.wmin[0]), fmaf(float(ny) + 0.5f, g.h, g.wmin[1]),
+                     fmaf(float(nz) + 0.5f, g.h, g.wmin[2]));
 }
 
 __device__ __forceinline__ float len3(float x, float y, float z) { return sqrtf(x * x + y * y + z * z); }
@@ -419,9 +472,12 @@ __device__ inline void apply_forces(float& vx, float& vy, float& vz, const nb_fo
 // is hashed node by node.  On 57,001 sand particles (96^3, turbulence of three
 // octaves and noise of two) the grid update went from 233 to 39 us, and to 29 with the
 // sines one after the other and the hashing of nodes out of line (38 registers spilled
-// and code beyond the instruction cache before).
+// and code beyond the instruction cache before).  What was left is a chain per node,
+// 38 values of noise: four threads share a node, one for each of the curl's four
+// points (ROLES = 4), and all forces' lattice points are hashed at once: 29 -> 19 us.
 constexpr uint32_t kNoiseTab = 2048;    // lattice points held at a time
-constexpr uint32_t kNoisePhases = 16;   // (group of points, octave) pairs with a place in the table
+constexpr uint32_t kNoisePhases = 32;   // (group of points, octave) pairs with a place in the table
+constexpr uint32_t kForcePhases = 16;   // of one force
 struct NoisePhase {
   float lo[3];       // first lattice point of the range
   int dim[3];        // lattice points per axis (0: not in the table)
@@ -431,8 +487,9 @@ struct NoiseLds {
   float4 grad[kNoiseTab];
   NoisePhase ph[kNoisePhases];
   uint32_t size[kNoisePhases];
-  float end[2][3];   // world position of the tile's first and last node
-  uint32_t total;
+  float part[3][4][kNoiseThreads];  // the curl's potentials: group, point, node
+  float end[2][3];   // world position of the block's first and last node
+  uint32_t total, upto;
 };
 
 // noise at p in a phase's lattice range (or hashed at once when it has none)
@@ -449,86 +506,129 @@ __device__ __forceinline__ float noise_value3_tab(float px, float py, float pz, 
   });
 }
 
-// apply_forces for a block that holds one tile's nodes, one a thread in
-// Morton order (thread 0 the first, the last thread the last); (x, y, z) is
-// the thread's node, live whether its velocity is wanted.  Every thread of
-// the block calls it.
-__device__ inline void tile_forces(float& vx, float& vy, float& vz, float x, float y, float z, bool live,
-                                   const nb_force* forces, uint32_t count, float dt, NoiseLds& L) {
+// A force's noise: groups 0 for none
+struct NoiseForm {
+  bool turb;
+  float fr, sd;
+  uint32_t oct, groups, phases;  // phases: octave by octave, the groups within
+};
+__device__ __forceinline__ NoiseForm noise_form(const nb_force& f) {
+  NoiseForm n;
+  n.turb = f.type == NB_FORCE_TURBULENCE;  // data: strength, frequency, octaves bits, seed; noise: dir xyz before them
+  n.fr = n.turb ? f.data[1] : f.data[4];
+  n.sd = n.turb ? f.data[3] : f.data[6];
+  const uint32_t oct = __float_as_uint(n.turb ? f.data[2] : f.data[5]);
+  n.oct = oct > 1u ? oct : 1u;
+  const bool on = (f.affect_mask == 0u || (f.affect_mask & 1u) != 0u) && (n.turb || f.type == NB_FORCE_NOISE);
+  n.groups = on ? (n.turb ? 3u : 1u) : 0u;
+  n.phases = on ? min(n.oct, kForcePhases / n.groups) * n.groups : 0u;
+  return n;
+}
+
+// apply_forces for a block of kNoiseThreads, ROLES a node: thread t holds node
+// t % (kNoiseThreads / ROLES); of the curl's four points it takes all (ROLES = 1) or
+// number t / (kNoiseThreads / ROLES) (ROLES = 4).  The nodes lie in the box from first to last (their
+// positions); (x, y, z) is the thread's node, live whether its velocity is wanted;
+// role 0 holds the velocity.  Every thread of the block calls it.
+template <uint32_t ROLES>
+__device__ inline void tile_forces(float& vx, float& vy, float& vz, float x, float y, float z, bool live, float3 first,
+                                   float3 last, const nb_force* forces, uint32_t count, float dt, NoiseLds& L) {
 #pragma clang fp contract(off)
   constexpr float kEps = 0.1f;                            // step of the curl's differences
   constexpr float kShift[3] = {19.1f, 47.3f, 71.7f};      // of the curl's three potentials, each along its own axis
-  if (threadIdx.x == 0u) { L.end[0][0] = x; L.end[0][1] = y; L.end[0][2] = z; }
-  if (threadIdx.x == blockDim.x - 1u) { L.end[1][0] = x; L.end[1][1] = y; L.end[1][2] = z; }
-  for (uint32_t fi = 0; fi < count; fi++) {
-    const nb_force f = forces[fi];
-    const uint32_t mask = f.affect_mask;
-    if (mask != 0u && (mask & 1u) == 0u) continue;
-    if (f.type == NB_FORCE_GRAVITY || f.type == NB_FORCE_CONSTANT_WIND) {
-      const float s = f.data[3];
-      vx += (f.data[0] * s) * dt;
-      vy += (f.data[1] * s) * dt;
-      vz += (f.data[2] * s) * dt;
-      continue;
-    }
-    const bool turb = f.type == NB_FORCE_TURBULENCE;  // data: strength, frequency, octaves bits, seed
-    if (!turb && f.type != NB_FORCE_NOISE) continue;  // data: dir xyz, strength, frequency, octaves bits, seed
-    const float fr = turb ? f.data[1] : f.data[4], sd = turb ? f.data[3] : f.data[6];
-    const uint32_t oct_ = __float_as_uint(turb ? f.data[2] : f.data[5]);
-    const uint32_t oct = oct_ > 1u ? oct_ : 1u;
-    const uint32_t groups = turb ? 3u : 1u;
-    const uint32_t phases = min(oct, kNoisePhases / groups) * groups;  // octave by octave, the groups within
-    __syncthreads();  // the ends are there; the last force's table is done with
-    if (threadIdx.x < phases) {
-      const uint32_t grp = threadIdx.x % groups;
-      float freq = 1.f;
-      for (uint32_t o = 0; o < threadIdx.x / groups; o++) freq *= 2.f;
+  constexpr uint32_t kNodes = kNoiseThreads / ROLES;
+  const uint32_t node = threadIdx.x % kNodes, role = threadIdx.x / kNodes;
+  if (threadIdx.x == 0u) {
+    L.end[0][0] = first.x; L.end[0][1] = first.y; L.end[0][2] = first.z;
+    L.end[1][0] = last.x; L.end[1][1] = last.y; L.end[1][2] = last.z;
+  }
+  // as many forces at a time as the phases and the table hold
+  for (uint32_t from = 0; from < count;) {
+    __syncthreads();  // the ends are there; the last table is done with
+    if (threadIdx.x < 64u) {
+      static_assert(kNoisePhases <= 64u && kForcePhases <= kNoisePhases, "a lane a phase");
+      uint32_t upto = from, used = 0u, mine = count, idx = 0u;
+      for (; upto < count; upto++) {
+        const uint32_t np = noise_form(forces[upto]).phases;
+        if (used + np > kNoisePhases) break;
+        if (threadIdx.x >= used && threadIdx.x < used + np) {
+          mine = upto;
+          idx = threadIdx.x - used;
+        }
+        used += np;
+      }
       NoisePhase ph;
-      float vol = 1.f;
-      bool ok = true;
-      for (int a = 0; a < 3; a++) {
-        // the nodes' coordinates lie between the ends', and rounding keeps
-        // that order through every step
-        const float p0 = L.end[0][a] * fr + sd, p1 = L.end[1][a] * fr + sd;
-        float lo = fminf(p0, p1), hi = fmaxf(p0, p1);
-        if (turb) {
-          if (uint32_t(a) == grp) {
-            lo = lo + kShift[a];
-            hi = hi + kShift[a];
-          } else {
-            lo = lo - kEps;
-            hi = hi + kEps;
+      ph.lo[0] = ph.lo[1] = ph.lo[2] = 0.f;
+      ph.dim[0] = ph.dim[1] = ph.dim[2] = 0;
+      uint32_t size = 0u;
+      if (mine < count) {
+        const NoiseForm f = noise_form(forces[mine]);
+        const uint32_t grp = idx % f.groups;
+        float freq = 1.f;
+        for (uint32_t o = 0; o < idx / f.groups; o++) freq *= 2.f;
+        float vol = 1.f;
+        bool ok = true;
+        for (int a = 0; a < 3; a++) {
+          // the nodes' coordinates lie between the ends', and rounding keeps
+          // that order through every step
+          const float p0 = L.end[0][a] * f.fr + f.sd, p1 = L.end[1][a] * f.fr + f.sd;
+          float lo = fminf(p0, p1), hi = fmaxf(p0, p1);
+          if (f.turb) {
+            if (uint32_t(a) == grp) {
+              lo = lo + kShift[a];
+              hi = hi + kShift[a];
+            } else {
+              lo = lo - kEps;
+              hi = hi + kEps;
+            }
           }
+          lo = floorf(lo * freq);
+          hi = floorf(hi * freq);
+          ok = ok && lo > -4194304.f && hi < 4194304.f && hi - lo < float(kNoiseTab);  // false for NaN too
+          ph.lo[a] = lo;
+          const float d = ok ? hi - lo + 2.f : 0.f;
+          ph.dim[a] = int(d);
+          vol *= d;
         }
-        lo = floorf(lo * freq);
-        hi = floorf(hi * freq);
-        ok = ok && lo > -4194304.f && hi < 4194304.f && hi - lo < float(kNoiseTab);  // false for NaN too
-        ph.lo[a] = lo;
-        const float d = ok ? hi - lo + 2.f : 0.f;
-        ph.dim[a] = int(d);
-        vol *= d;
+        ok = ok && vol <= float(kNoiseTab);
+        if (!ok) ph.dim[0] = ph.dim[1] = ph.dim[2] = 0;
+        size = ok ? uint32_t(vol) : 0u;
       }
-      ok = ok && vol <= float(kNoiseTab);
-      if (!ok) ph.dim[0] = ph.dim[1] = ph.dim[2] = 0;
-      ph.off = 0u;
-      L.ph[threadIdx.x] = ph;
-      L.size[threadIdx.x] = ok ? uint32_t(vol) : 0u;
+      // places in the table, force by force; a force that does not fit beside
+      // those before it waits for the next table
+      uint32_t at = 0u, slot = 0u;
+      for (uint32_t f = from; f < upto; f++) {
+        const uint32_t np = noise_form(forces[f]).phases;
+        uint32_t sum = 0u;
+        for (uint32_t i = 0; i < np; i++) sum += uint32_t(__shfl(int(size), int(slot + i)));
+        if (f > from && at + sum > kNoiseTab) {
+          upto = f;
+          break;
+        }
+        for (uint32_t i = 0; i < np; i++, slot++) {
+          uint32_t n = uint32_t(__shfl(int(size), int(slot)));
+          const bool fits = at + n <= kNoiseTab;
+          if (threadIdx.x == slot) {
+            if (!fits) {
+              ph.dim[0] = 0;
+              size = 0u;
+            }
+            ph.off = at;
+          }
+          at += fits ? n : 0u;
+        }
+      }
+      if (threadIdx.x < slot) {
+        L.ph[threadIdx.x] = ph;
+        L.size[threadIdx.x] = size;
+      }
+      if (threadIdx.x == 0u) {
+        L.total = at;
+        L.upto = upto;
+      }
     }
     __syncthreads();
-    if (threadIdx.x == 0u) {
-      uint32_t at = 0u;
-      for (uint32_t i = 0; i < phases; i++) {
-        if (at + L.size[i] > kNoiseTab) {
-          L.ph[i].dim[0] = 0;
-          L.size[i] = 0u;
-        }
-        L.ph[i].off = at;
-        at += L.size[i];
-      }
-      L.total = at;
-    }
-    __syncthreads();
-    const uint32_t total = L.total;
+    const uint32_t total = L.total, upto = L.upto;
     for (uint32_t e = threadIdx.x; e < total; e += blockDim.x) {
       uint32_t i = 0;
       while (e >= L.ph[i].off + L.size[i]) i++;
@@ -538,65 +638,104 @@ __device__ inline void tile_forces(float& vx, float& vy, float& vz, float x, flo
       L.grad[e] = make_float4(g.x, g.y, g.z, 0.f);
     }
     __syncthreads();
-    if (!live) continue;
-    const float px = x * fr + sd, py = y * fr + sd, pz = z * fr + sd;
-    // fBm (force_noise.glsl:40-50) at up to four points at a time, octave by octave
     NoisePhase none;
     none.dim[0] = 0;
-    if (turb) {
-      // the curl (force_noise.glsl:54-82): group g holds the potential shifted
-      // along axis g, at +-eps along the two other axes
-      float d[3][2];  // differences of group g along its first and second other axis
+    uint32_t base = 0u;  // of the force's phases
+    for (uint32_t fi = from; fi < upto; fi++) {
+      const nb_force f = forces[fi];
+      const uint32_t mask = f.affect_mask;
+      if (mask != 0u && (mask & 1u) == 0u) continue;
+      if (f.type == NB_FORCE_GRAVITY || f.type == NB_FORCE_CONSTANT_WIND) {
+        const float s = f.data[3];
+        vx += (f.data[0] * s) * dt;
+        vy += (f.data[1] * s) * dt;
+        vz += (f.data[2] * s) * dt;
+        continue;
+      }
+      const NoiseForm nf = noise_form(f);
+      if (nf.groups == 0u) continue;
+      const float px = x * nf.fr + nf.sd, py = y * nf.fr + nf.sd, pz = z * nf.fr + nf.sd;
+      // fBm (force_noise.glsl:40-50), octave by octave
+      if (nf.turb) {
+        // the curl (force_noise.glsl:54-82): group g holds the potential shifted
+        // along axis g, at +-eps along the two other axes
+        if (live) {
 #pragma unroll 1
-      for (uint32_t g = 0; g < 3u; g++) {
-        const float qx = g == 0u ? px + kShift[0] : px, qy = g == 1u ? py + kShift[1] : py;
-        const float qz = g == 2u ? pz + kShift[2] : pz;
-        // first other axis: y, x, x; second: z, z, y
-        const float ax = g == 0u ? 0.f : kEps, ay = g == 0u ? kEps : 0.f;
-        const float bz = g == 2u ? 0.f : kEps, by = g == 2u ? kEps : 0.f;
-        float s[4] = {0.f, 0.f, 0.f, 0.f};
-        float amp = 0.5f, freq = 1.f;
+          for (uint32_t g = 0; g < 3u; g++) {
+            const float qx = g == 0u ? px + kShift[0] : px, qy = g == 1u ? py + kShift[1] : py;
+            const float qz = g == 2u ? pz + kShift[2] : pz;
+            // first other axis: y, x, x; second: z, z, y
+            const float ax = g == 0u ? 0.f : kEps, ay = g == 0u ? kEps : 0.f;
+            const float bz = g == 2u ? 0.f : kEps, by = g == 2u ? kEps : 0.f;
+            float s[4 / ROLES] = {};
+            float amp = 0.5f, freq = 1.f;
 #pragma unroll 1
-        for (uint32_t o = 0; o < oct; o++) {
-          const uint32_t i = o * 3u + g;
-          const NoisePhase ph = i < phases ? L.ph[i] : none;
+            for (uint32_t o = 0; o < nf.oct; o++) {
+              const uint32_t i = o * 3u + g;
+              const NoisePhase ph = i < nf.phases ? L.ph[base + i] : none;
 #pragma unroll
-          for (int k = 0; k < 4; k++) {
-            float ux = qx, uy = qy, uz = qz;
-            if (k == 0) { ux = qx + ax; uy = qy + ay; }
-            if (k == 1) { ux = qx - ax; uy = qy - ay; }
-            if (k == 2) { uy = qy + by; uz = qz + bz; }
-            if (k == 3) { uy = qy - by; uz = qz - bz; }
-            s[k] += amp * noise_value3_tab(ux * freq, uy * freq, uz * freq, ph, L.grad);
+              for (uint32_t j = 0; j < 4u / ROLES; j++) {
+                const uint32_t k = ROLES == 1u ? j : role;
+                float ux = qx, uy = qy, uz = qz;
+                if (k == 0u) { ux = qx + ax; uy = qy + ay; }
+                if (k == 1u) { ux = qx - ax; uy = qy - ay; }
+                if (k == 2u) { uy = qy + by; uz = qz + bz; }
+                if (k == 3u) { uy = qy - by; uz = qz - bz; }
+                s[j] += amp * noise_value3_tab(ux * freq, uy * freq, uz * freq, ph, L.grad);
+              }
+              freq *= 2.f;
+              amp *= 0.5f;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 4u / ROLES; j++) L.part[g][ROLES == 1u ? j : role][node] = s[j];
           }
+        }
+        __syncthreads();
+        if (live && role == 0u) {
+          float d[3][2];  // differences of group g along its first and second other axis
+#pragma unroll
+          for (int g = 0; g < 3; g++) {
+            d[g][0] = L.part[g][0][node] - L.part[g][1][node];
+            d[g][1] = L.part[g][2][node] - L.part[g][3][node];
+          }
+          const float s2 = 2.f * kEps;
+          const float cx = d[2][1] / s2 - d[1][1] / s2, cy = d[0][1] / s2 - d[2][0] / s2, cz = d[1][0] / s2 - d[0][0] / s2;
+          vx += (cx * f.data[0]) * dt;
+          vy += (cy * f.data[0]) * dt;
+          vz += (cz * f.data[0]) * dt;
+        }
+        __syncthreads();
+      } else if (live && role == 0u) {
+        float s = 0.f, amp = 0.5f, freq = 1.f;
+#pragma unroll 1
+        for (uint32_t o = 0; o < nf.oct; o++) {
+          const NoisePhase ph = o < nf.phases ? L.ph[base + o] : none;
+          s += amp * noise_value3_tab(px * freq, py * freq, pz * freq, ph, L.grad);
           freq *= 2.f;
           amp *= 0.5f;
         }
-        const float d0 = s[0] - s[1], d1 = s[2] - s[3];
-        if (g == 0u) { d[0][0] = d0; d[0][1] = d1; }
-        if (g == 1u) { d[1][0] = d0; d[1][1] = d1; }
-        if (g == 2u) { d[2][0] = d0; d[2][1] = d1; }
+        const float k = (s * f.data[3]) * dt;
+        vx += f.data[0] * k;
+        vy += f.data[1] * k;
+        vz += f.data[2] * k;
       }
-      const float s2 = 2.f * kEps;
-      const float cx = d[2][1] / s2 - d[1][1] / s2, cy = d[0][1] / s2 - d[2][0] / s2, cz = d[1][0] / s2 - d[0][0] / s2;
-      vx += (cx * f.data[0]) * dt;
-      vy += (cy * f.data[0]) * dt;
-      vz += (cz * f.data[0]) * dt;
-    } else {
-      float s = 0.f, amp = 0.5f, freq = 1.f;
-#pragma unroll 1
-      for (uint32_t o = 0; o < oct; o++) {
-        const NoisePhase ph = o < phases ? L.ph[o] : none;
-        s += amp * noise_value3_tab(px * freq, py * freq, pz * freq, ph, L.grad);
-        freq *= 2.f;
-        amp *= 0.5f;
-      }
-      const float k = (s * f.data[3]) * dt;
-      vx += f.data[0] * k;
-      vy += f.data[1] * k;
-      vz += f.data[2] * k;
+      base += nf.phases;
     }
+    from = upto;
   }
+}
+
+// Whether a block's nodes are wanted, known by role 0 (live), for all roles; any: of
+// the block.
+template <uint32_t ROLES>
+__device__ __forceinline__ bool noise_live(bool live, uint64_t* s_live, bool& any) {
+  constexpr uint32_t kWaves = kNoiseThreads / ROLES / 64u;
+  any = __syncthreads_or(live);
+  if (ROLES == 1u) return live;
+  const uint64_t b = __ballot(live);
+  if (threadIdx.x < kWaves * 64u && (threadIdx.x & 63u) == 0u) s_live[threadIdx.x >> 6] = b;
+  __syncthreads();
+  return (s_live[(threadIdx.x >> 6) % kWaves] >> (threadIdx.x & 63u)) & 1u;
 }
 
 // applyColliderBC — shaders/collider_common.glsl:62-73

@@ -74,3 +74,33 @@ def test_one_block_a_tile_equals_two(gpu_lib):
         e.adjointEnd()
     assert np.array_equal(got[0][1].view(np.uint32), got[1][1].view(np.uint32))
     assert np.array_equal(got[0][2].view(np.uint32), got[1][2].view(np.uint32))
+
+
+def test_noise_four_threads_a_node_equal_one(gpu_lib):
+    """A scene of at most 27 tiles alone and in a batch of more than 51; forces
+    whose lattice points take several tables, one beyond any table."""
+    rng = np.random.default_rng(4)
+    a = _scene(24, 500, "anywhere")
+    fill = [falling_box(f"f{i}", 48, 3000, 2e4, 0.3, MaterialModel.ELASTIC, rng, corrected_svd=True) for i in range(12)]
+    a.forces = [mpm.GravityForce((0.0, 1.0, 0.0), -9.8), mpm.TurbulenceForce(strength=2.0, frequency=3.0, octaves=5, seed=1.0),
+                mpm.TurbulenceForce(strength=1.0, frequency=7.0, octaves=4, seed=0.3),
+                mpm.NoiseForce((0.0, 1.0, 0.0), 0.5, 5.0, 6, 0.7, 0.1), mpm.NoiseForce((1.0, 0.0, 0.0), 0.5, 900.0, 2, 0.7, 0.1)]
+    W = rng.standard_normal((8, a.n, 4)).astype(np.float32)
+    W[1, :, 3] = 0.0
+    got = []
+    for e, total in ((make_engine(a), a.n), (make_batch_engine([a] + fill), a.n + sum(s.n for s in fill))):
+        e.substep(a.dt, 2)
+        tiles = e.activeTileCount()
+        e.adjointBegin(2, 2)
+        e.forwardRecorded(a.dt)
+        full = np.zeros((8, total, 4), np.float32)
+        full[:, :a.n] = W
+        e.setAdjoint(full)
+        e.backward()
+        state = e.getState()[:, :a.n].copy()
+        state[1, :, 3] = 0.0  # the batch's material ids are offset
+        got.append((tiles, state, e.getAdjoint()[:, :a.n].copy()))
+        e.adjointEnd()
+    assert got[0][0] <= 27 and got[1][0] > 51
+    assert np.array_equal(got[0][1].view(np.uint32), got[1][1].view(np.uint32))
+    assert np.array_equal(got[0][2].view(np.uint32), got[1][2].view(np.uint32))
