@@ -13,10 +13,11 @@
 //         128-byte record each) and sums their 27 node contributions in
 //         registers; the sums are merged into the tile's 10^3 LDS node box in 27
 //         barrier-separated phases (every thread owns a distinct node in a
-//         phase: no atomics, fixed order) and written as a per-tile partial
+//         phase: no atomics, fixed order) and written as a per-tile partial;
+//         small scenes: k_p2g_items walks the cells, k_p2g merges
 //         (replaces mpm_zero_grid + mpm_p2g.comp's node-centric gather)
 //   grid  k_grid_tiles: per occupied tile, its nodes and those around it that no
-//         other takes (with noise forces k_grid: one block per node tile); sums
+//         other takes (with noise forces k_grid_noise, in smaller units); sums
 //         the <= 8 partials covering each node in a fixed order, then velocity,
 //         cap, forces, walls, analytic colliders and the dense-SDF BC in registers
 //         (replaces mpm_grid_update.comp + mpm_nanovdb_bc.comp)
@@ -2070,12 +2071,12 @@ __global__ __launch_bounds__(256) void k_bin_compact(const uint8_t* __restrict__
 // kG2PUnit particles of one occupied tile (a tile's particles are one
 // contiguous range of the bin order; k_bin_tile_offsets lists the units).
 // The block builds the tile's 10^3 node box in LDS from the partials (the
-// same sums and node update as k_grid, bit for bit), stores each node's
+// same sums and node update as k_grid_tiles, bit for bit), stores each node's
 // G2P view (velocity, or zero for a node that does not take part, and FLIP's
 // saved velocity), then runs G2P for the unit's particles gathering from
 // LDS.  A particle whose stencil leaves the box (its position lies outside
 // the grid) reads the box with a range check: the nodes outside it are
-// outside the grid too.  Results equal k_grid + k_g2p bit for bit; the
+// outside the grid too.  Results equal k_grid_tiles + k_g2p bit for bit; the
 // grid itself is not written (the last substep of a call runs unfused, so the
 // exported grid stays that of the last substep).
 template <bool FLIP, bool BATCH>
@@ -2110,7 +2111,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
       const int nx = tx * 8 - 1 + bx, ny = ty * 8 - 1 + by, nz = tz * 8 - 1 + bz;
       float4 v = make_float4(0.f, 0.f, 0.f, 0.f), o = make_float4(0.f, 0.f, 0.f, 0.f);
       if (nx >= 0 && nx < g.grid_res[0] && ny >= 0 && ny < g.grid_res[1] && nz >= 0 && nz < g.grid_res[2]) {
-        // the node's own tile and its place in it, as k_grid sees the node
+        // the node's own tile and its place in it, as the grid update sees the node
         const int ntx = nx >> 3, nty = ny >> 3, ntz = nz >> 3;
         float mx, my, mz, mass;
         (void)sum_partials(g, ntx, nty, ntz, nx & 7, ny & 7, nz & 7, tile_act, partial, mx, my, mz, mass);
@@ -2462,7 +2463,7 @@ void launch_grid(const DevState& d, const SubParams& p, uint32_t n_tiles, bool f
 
 // The fused grid update + G2P (k_g2p_tile) over the work units the bin listed
 // (not with turbulence or noise forces: their noise code would halve the
-// kernel's occupancy; those substeps run k_grid + k_g2p).
+// kernel's occupancy; those substeps run k_grid_noise + k_g2p).
 void launch_g2p_fused(const DevState& d, const SubParams& p, uint32_t n_tiles, hipStream_t s, Prof* pf) {
   // units <= occupied tiles + n / kG2PUnit; blocks stride over them
   const uint32_t max_units = n_tiles + p.n / kG2PUnit + 1u;

@@ -147,8 +147,8 @@ __device__ __forceinline__ uint32_t tile_id(const SceneGeo& g, int tx, int ty, i
 // tile takes its tile's 512 nodes (thread t the t-th in Morton order), then those
 // of the 488 nodes around them whose own tile is not occupied and that no occupied
 // tile before it (z, y, x ascending) covers: each covered node once.  A block per
-// tile that any box reaches (k_grid) spends most of its threads on nodes that none
-// covers, and read the covering boxes one after the other.  Bound by the latency of
+// tile that any box reaches spent most of its threads on nodes that none covers, and
+// read the covering boxes one after the other.  Now bound by the latency of
 // a tile's list entries and boxes, then by memory: 43 -> 20 us for the 1,279
 // occupied tiles of 64 small scenes, 47 -> 36 for 2,385 of a terrain (4.19 M
 // particles), 18 -> 12 for 300 of 16 scenes (backward 20 -> 11).  Up to
