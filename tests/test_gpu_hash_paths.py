@@ -56,3 +56,17 @@ def test_cells_beyond_a_wave_with_and_without_their_list(gpu_lib, res, many):
     p = p[rng.permutation(len(p))]
     cnt, _, _ = _check(f"{many} cells of 257", p, None, (0, 0, 0), 1.0 / res, (res, res, res))
     assert np.sum(cnt > 256) == many
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 5000])
+@pytest.mark.parametrize("order", ["runs", "mixed"])
+def test_places_kept_from_the_count(gpu_lib, n, order):
+    """Beyond 2^18 cells the count keeps the particles' places: runs of equal cells
+    within and across waves, unused slots between them, and no order at all."""
+    rng = np.random.default_rng(n)
+    cells = np.repeat(rng.choice(128 ** 3, n, replace=False), rng.integers(1, 90, n))[:n]
+    p = _points(cells, np.ones(n, int), 128, rng)
+    if order == "mixed":
+        p = p[rng.permutation(n)]
+    tf = np.where(rng.random(n) < 0.2, 6, 0).astype(np.uint32)
+    _check(f"{order} {n}", p, tf, (0, 0, 0), 1.0 / 128, (128, 128, 128))
