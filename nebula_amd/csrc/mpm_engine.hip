@@ -350,6 +350,16 @@ struct TapeIO {
   const DevState* bins = nullptr;  // bin buffers to use instead of the engine's
 };
 
+// What an unfused substep leaves: its bins, its grid and, if its G2P counted them,
+// the particles' tile counts.
+void substep_done(nb_mpm* h, bool old_written, bool counted) {
+  h->bins_valid = true;
+  h->keys_valid = true;
+  h->counted = h->counts_dirty = counted;
+  h->grid_mode = GridMode::SPARSE;
+  h->old_valid = old_written;
+}
+
 // One substep.  last: the call's last, so the FP64 fallback's queue is worked
 // off at its end (the next substep's bin does it otherwise); if the caller may
 // write the state before the next call, its particles are not counted for a
@@ -394,11 +404,7 @@ int enqueue_substep(nb_mpm* h, float dt, Prof* pf, bool last, const TapeIO& io =
   launch_g2p(dv, p, true, count, h->stream, pf, io.rec_out);
   if (last) launch_g2p_fb(dv, p, io.rec_out ? io.rec_out : dv.rec, h->stream, pf);
   NB_HIP(hipGetLastError());
-  h->bins_valid = true;
-  h->keys_valid = true;
-  h->counted = h->counts_dirty = count;
-  h->grid_mode = GridMode::SPARSE;
-  h->old_valid = flip;
+  substep_done(h, flip, count);
   return NB_OK;
 }
 
@@ -843,6 +849,7 @@ int nb_mpm_graph_substeps(nb_mpm* h, float dt_sub, uint32_t n) {
     for (uint32_t i = 0; i < n; i++) NB_HIP(hipGraphLaunch(h->graph_exec, h->stream));
     launch_g2p_fb(dv, p, dv.rec, h->stream, nullptr);
     NB_HIP(hipGetLastError());
+    substep_done(h, p.write_old != 0u, true);  // a replay of an earlier capture has run none of the host's code
   }
   if (rc == NB_OK) rc = sync_out(h);
   return rc;
