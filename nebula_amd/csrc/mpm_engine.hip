@@ -1214,13 +1214,14 @@ int nb_mpm_set_collider_mesh(nb_mpm* h, const float* tris, uint32_t n_tris, int 
   if (n_tris && !tris) return fail(NB_ERR_ARG, "null triangles");
   int rc = ensure_sdf(h);
   if (rc != NB_OK) return rc;
-  float* d_tris = nullptr;  // the triangles, then a float4 of scratch for each
-  const size_t bytes = std::max<size_t>(size_t(n_tris) * (12 * 4 + sizeof(float4)), 4);
+  float* d_tris = nullptr;  // the triangles, then the scratch
+  const size_t bytes = std::max<size_t>(size_t(n_tris) * (12 * 4 + kMeshScratch), 4);
   NB_HIP(hipMalloc(&d_tris, bytes));
   rc = n_tris ? upload(h, d_tris, tris, size_t(n_tris) * 12 * 4) : NB_OK;
   if (rc == NB_OK) {
     const int32_t res[3] = {int32_t(h->grid_res[0]), int32_t(h->grid_res[1]), int32_t(h->grid_res[2])};
-    launch_mesh_sdf(d_tris, reinterpret_cast<float4*>(d_tris + size_t(n_tris) * 12), n_tris, res, h->cube_res, h->cfg.cell_size, exact != 0, h->d.sdf, h->stream);
+    launch_mesh_sdf(d_tris, d_tris + size_t(n_tris) * 12, n_tris, res, h->cube_res, h->cfg.cell_size, exact != 0,
+                    h->d.sdf, h->stream);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) rc = fail(NB_ERR_HIP, "mesh SDF build failed: %s", hipGetErrorString(e));

@@ -2524,16 +2524,16 @@ void launch_g2p(const DevState& d, const SubParams& p, bool use_sorted, bool cou
 // host.
 //
 // A cell's result is the minimum over all triangles, but few of them can hold
-// it: a block takes one 8^3 brick of cells, bounds the distance any of its
-// cells can have (U: the nearest centroid's distance to the brick's centre plus
-// the brick's radius) and keeps, in index order, the triangles whose own lower
-// bound does not exceed U; each wave then bounds its 4^3 sub-brick the same way
-// over that list with true distances, holds for each a linear lower bound (a
-// distance to a triangle is convex), measures the nearest one and then only
-// those whose bound is not above some lane's best.  A triangle dropped is
-// farther than the result from every cell it is dropped for, with slack above
-// rounding, so neither a minimum nor a tie: values and signs have the bits of
-// the pass over all triangles.  On 128^3 cells and 3,360 triangles a cell
+// it: a block takes one 8^3 brick of cells, measures the triangle of the nearest
+// centroid from each (U: the largest of these distances) and keeps, in index
+// order, the triangles whose own lower bound does not exceed U; each wave then
+// does the same for its 4^3 sub-brick over that list, holds for each triangle a
+// linear lower bound (a distance to a triangle is convex), measures the nearest
+// one and then only those whose bound is not above some lane's best.  What is
+// compared with a bound is always a distance measured, and a bound is lowered by
+// what rounding can take from the distance that would be measured (mesh_error),
+// so a triangle dropped is neither a minimum nor a tie: values and signs have the
+// bits of the pass over all triangles.  On 128^3 cells and 3,360 triangles a cell
 // measures about 26 distances instead of 3,360 and the build takes 0.67 ms
 // instead of 10.1 (VALU-bound; 0.98 with the wave's bound alone).
 // ---------------------------------------------------------------------------
@@ -2582,13 +2582,25 @@ constexpr uint32_t kMeshThreads = 512;       // cells of a brick
 constexpr uint32_t kMeshList = 2048;         // triangles a block holds at a time
 constexpr int kMeshHeld = 8;                 // of them, those a lane holds bounds of at a time
 constexpr float kMeshSlack = 1e-3f;          // of the lengths in a bound: far above their rounding
+// What rounding can do to a distance.  With l the triangle's longest edge, N its
+// cross product, k = l^2 / |N| (longest edge over height), R the distance to its
+// farthest vertex and u = 2^-24: the dot products of tri_closest are off by up to 6 u
+// l R and the barycentric numerators of a point within about l of the triangle
+// sideways by some 24 u l^3 R.  A point up to 48 u k^2 R beside the triangle may so be
+// taken to lie over it, which takes that much at most from its distance: from there on
+// the closest point lies in the plane, wherever.  The closest point of a point over
+// the triangle moves within the plane, by 3.4 u k^2 R at most in 8e7 tries over k of 1.2
+// to 90 and R / l of 0.3 to 10^4.  All this while the error is below the triangle's
+// size; beyond, a distance may be anything down to that to the plane, and the triangle
+// is measured everywhere.
+constexpr float kMeshError = 2.9e-6f;  // 48 u
 
-// Centroid and radius of each triangle.  A triangle so thin that the rounding
-// of its closest point is not bounded by the slack (height below a hundredth
-// of its longest edge), or not finite, gets a negative radius: it bounds
-// nothing and is never dropped.
+// Centroid and radius of each triangle, and its kMeshError k^2.  A triangle of no
+// height (below a hundredth of its longest edge), not finite or beyond the range
+// where its products are gets a negative radius: it bounds nothing and is never
+// dropped.
 __global__ __launch_bounds__(256) void k_mesh_spheres(const float* __restrict__ tris, uint32_t n_tris,
-                                                      float4* __restrict__ sph) {
+                                                      float4* __restrict__ sph, float* __restrict__ err) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n_tris) return;
   const float* t = tris + size_t(i) * 12;
@@ -2601,8 +2613,16 @@ __global__ __launch_bounds__(256) void k_mesh_spheres(const float* __restrict__ 
   const float cx = bx - ax, cy = by - ay, cz = bz - az;
   const float l2 = fmaxf(fmaxf(ax * ax + ay * ay + az * az, bx * bx + by * by + bz * bz), cx * cx + cy * cy + cz * cz);
   const float n2 = nx * nx + ny * ny + nz * nz;
-  const bool good = n2 > 1e-4f * l2 * l2 && n2 < 1e30f && l2 < 1e15f && fabsf(gx) + fabsf(gy) + fabsf(gz) < 1e15f;
+  const bool good = n2 > 1e-4f * l2 * l2 && n2 > 1e-30f && l2 < 1e14f && fabsf(gx) + fabsf(gy) + fabsf(gz) < 1e15f;
   sph[i] = make_float4(gx, gy, gz, good ? r * (1.f + kMeshSlack) : -1.f);
+  err[i] = good ? kMeshError * (l2 * l2 / n2) : 0.f;
+}
+
+// What rounding can take from a distance to a triangle of radius rad none of whose
+// vertices is farther than R; INFINITY where that is not bounded.
+__device__ __forceinline__ float mesh_error(float err, float rad, float R) {
+  const float e = err * R;
+  return e <= rad ? e : INFINITY;
 }
 
 // Whether some point of the ball (centre (cx, cy, cz), radius r) can lie in the
@@ -2629,12 +2649,12 @@ __device__ __forceinline__ bool mesh_edge_slab(const float* __restrict__ t, floa
 
 // Whether triangle t, its centroid's distance dg and its radius rad from the
 // centre (cx, cy, cz) of a ball of radius r known, may hold the minimum of a
-// point of the ball when no such point is farther than U from the mesh.
+// point of the ball when a distance of at most U is known for each.
 template <bool EXACT>
-__device__ __forceinline__ bool mesh_may_hold(const float* __restrict__ t, float dg, float rad, float cx, float cy,
-                                              float cz, float r, float U) {
+__device__ __forceinline__ bool mesh_may_hold(const float* __restrict__ t, float dg, float rad, float err, float cx,
+                                              float cy, float cz, float r, float U) {
   if (!(rad >= 0.f)) return true;
-  const float slack = kMeshSlack * (dg + rad + r);
+  const float R = dg + rad + r, slack = kMeshSlack * R + mesh_error(err, rad, R);
   if (!(dg - rad - r > U + slack)) return true;
   return !EXACT && mesh_edge_slab(t, cx, cy, cz, r, slack, U);
 }
@@ -2643,14 +2663,15 @@ __device__ __forceinline__ bool mesh_may_hold(const float* __restrict__ t, float
 // thread in Morton order, so that each wave holds a 4^3 sub-brick.
 template <bool EXACT>
 __global__ __launch_bounds__(kMeshThreads) void k_mesh_sdf(const float* __restrict__ tris,
-                                                           const float4* __restrict__ sph, uint32_t n_tris, int rx,
+                                                           const float4* __restrict__ sph,
+                                                           const float* __restrict__ err, uint32_t n_tris, int rx,
                                                            int ry, int rz, uint32_t nc, uint32_t first_brick, float cs,
                                                            float* __restrict__ sdf) {
 #pragma clang fp contract(off)
   constexpr uint32_t kWaves = kMeshThreads / 64;
   __shared__ uint32_t s_list[kMeshList];
-  __shared__ float s_min[kWaves];
-  __shared__ uint32_t s_cnt[kWaves];
+  __shared__ float s_min[kWaves], s_max[kWaves];
+  __shared__ uint32_t s_arg[kWaves], s_cnt[kWaves];
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   const uint32_t m = (first_brick + blockIdx.x) * kMeshThreads + threadIdx.x;
   const int ix = int(morton_compact(m)), iy = int(morton_compact(m >> 1)), iz = int(morton_compact(m >> 2));
@@ -2661,40 +2682,70 @@ __global__ __launch_bounds__(kMeshThreads) void k_mesh_sdf(const float* __restri
     return;
   }
   const float px = (float(ix) + 0.5f) * cs, py = (float(iy) + 0.5f) * cs, pz = (float(iz) + 0.5f) * cs;
-  auto wave_min = [](float v) {
+  // the least distance measured so far and its triangle (a cell outside the grid
+  // wants none)
+  float best = valid ? 1e9f : -INFINITY;
+  uint32_t best_j = 0u;
+  bool outer = true;
+  auto measure = [&](uint32_t j) {
+    const float* t = tris + size_t(j) * 12;
+    const float3 q = tri_closest<EXACT>(t, px, py, pz);
+    const float dx = px - q.x, dy = py - q.y, dz = pz - q.z;
+    const float d = sqrtf((dx * dx + dy * dy) + dz * dz);
+    if (d < best || (d == best && j < best_j)) {
+      best = d;
+      best_j = j;
+      outer = (dx * t[0] + dy * t[1]) + dz * t[2] >= 0.f;
+    }
+  };
+  auto wave_max = [](float v) {
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fminf(v, __shfl_xor(v, d));
+    for (int d = 32; d >= 1; d >>= 1) v = fmaxf(v, __shfl_xor(v, d));
     return v;
   };
-  // the brick's ball, and the bound on its cells' distances
+  // the brick's ball; the triangle of the nearest centroid, and the largest of its
+  // distances from the brick's cells
   const float bcx = float(bx + 4) * cs, bcy = float(by + 4) * cs, bcz = float(bz + 4) * cs;
   const float br = 6.0622f * cs * (1.f + kMeshSlack);  // 3.5 sqrt(3) cells
   float u = INFINITY;
+  uint32_t u_j = 0u;
   for (uint32_t i = threadIdx.x; i < n_tris; i += kMeshThreads) {
     const float4 g = sph[i];
-    if (g.w >= 0.f) u = fminf(u, len3(g.x - bcx, g.y - bcy, g.z - bcz));
+    const float d = len3(g.x - bcx, g.y - bcy, g.z - bcz);
+    if (g.w >= 0.f && d < u) { u = d; u_j = i; }
   }
-  u = wave_min(u);
-  if (lane == 0u) s_min[wave] = u;
-  __syncthreads();
 #pragma unroll
-  for (uint32_t w = 0; w < kWaves; w++) u = fminf(u, s_min[w]);
-  const float U = (u + br) * (1.f + kMeshSlack);
+  for (int d = 32; d >= 1; d >>= 1) {
+    const float v = __shfl_xor(u, d);
+    const uint32_t j = uint32_t(__shfl_xor(int(u_j), d));
+    if (v < u || (v == u && j < u_j)) { u = v; u_j = j; }
+  }
+  if (lane == 0u) { s_min[wave] = u; s_arg[wave] = u_j; }
+  __syncthreads();
+  u = s_min[0];
+  u_j = s_arg[0];
+#pragma unroll
+  for (uint32_t w = 1; w < kWaves; w++)
+    if (s_min[w] < u) { u = s_min[w]; u_j = s_arg[w]; }
+  if (n_tris) measure(uint32_t(__builtin_amdgcn_readfirstlane(int(u_j))));  // one triangle for all
+  const float most = wave_max(best);
+  if (lane == 0u) s_max[wave] = most;
+  __syncthreads();
+  float U = -INFINITY;
+#pragma unroll
+  for (uint32_t w = 0; w < kWaves; w++) U = fmaxf(U, s_max[w]);
 
-  float best = 1e9f;
-  uint32_t best_j = 0u;
-  bool outer = true;
   const int wx = ix & ~3, wy = iy & ~3, wz = iz & ~3;
   const float wcx = float(wx + 2) * cs, wcy = float(wy + 2) * cs, wcz = float(wz + 2) * cs;
   const float wr = 2.5981f * cs * (1.f + kMeshSlack);  // 1.5 sqrt(3) cells
-  float wu = INFINITY;  // nearest true distance to the sub-brick's centre so far
   uint32_t count = 0;
   for (uint32_t base = 0; base < n_tris; base += kMeshThreads) {
     const uint32_t i = base + threadIdx.x;
     bool keep = false;
     if (i < n_tris) {
       const float4 g = sph[i];
-      keep = mesh_may_hold<EXACT>(tris + size_t(i) * 12, len3(g.x - bcx, g.y - bcy, g.z - bcz), g.w, bcx, bcy, bcz, br, U);
+      keep = mesh_may_hold<EXACT>(tris + size_t(i) * 12, len3(g.x - bcx, g.y - bcy, g.z - bcz), g.w, err[i], bcx, bcy, bcz,
+                                  br, U);
     }
     const uint64_t kept = __ballot(keep);
     __syncthreads();  // the last round's counts are read, its list entries used
@@ -2712,7 +2763,8 @@ __global__ __launch_bounds__(kMeshThreads) void k_mesh_sdf(const float* __restri
     for (uint32_t c0 = 0; c0 < count; c0 += 64u * kMeshHeld) {
       // a lane's triangles of this part of the list: distance from the
       // sub-brick's centre and its gradient there.  The distance to a triangle
-      // is convex, so d + g . (p - centre) bounds it from below at any p; a
+      // is convex, so d + g . (p - centre) bounds it from below at any p, less
+      // what rounding does to d, to g and to the distance measured; a
       // triangle that bounds nothing there holds g = 0 and d = 0 (the missing
       // edge region makes the distance jump; too thin; the centre lies on it).
       float hd[kMeshHeld], hx[kMeshHeld], hy[kMeshHeld], hz[kMeshHeld], hs[kMeshHeld];
@@ -2730,34 +2782,27 @@ __global__ __launch_bounds__(kMeshThreads) void k_mesh_sdf(const float* __restri
             const float3 q = tri_closest<true>(t, wcx, wcy, wcz);
             const float gx = wcx - q.x, gy = wcy - q.y, gz = wcz - q.z, d = len3(gx, gy, gz);
             if (d < near) { near = d; near_k = k; }
-            if (d > 0.25f * wr && (EXACT || !mesh_edge_slab(t, wcx, wcy, wcz, wr, kMeshSlack * (d + rad + wr), INFINITY))) {
+            const float R = d + 2.f * rad + wr, e_d = mesh_error(err[j], rad, R);
+            if (d > 0.25f * wr && e_d < 0.25f * d &&
+                (EXACT || !mesh_edge_slab(t, wcx, wcy, wcz, wr, kMeshSlack * R + e_d, INFINITY))) {
               hd[k] = d;
               hx[k] = gx / d; hy[k] = gy / d; hz[k] = gz / d;
-              hs[k] = 4.f * kMeshSlack * (d + wr);
+              hs[k] = 4.f * kMeshSlack * (d + wr) + e_d * (2.f + 3.f * wr / d);
             }
           }
         }
       }
       // the wave's nearest triangle first (any order gives the same result:
       // equal distances go to the lower index), then the others in turn
-      wu = fminf(wu, wave_min(near));
-      const uint64_t at_min = __ballot(near <= wu && near < INFINITY);
-      auto measure = [&](uint32_t j) {
-        const float* t = tris + size_t(j) * 12;
-        const float3 q = tri_closest<EXACT>(t, px, py, pz);
-        const float dx = px - q.x, dy = py - q.y, dz = pz - q.z;
-        const float d = sqrtf((dx * dx + dy * dy) + dz * dz);
-        if (d < best || (d == best && j < best_j)) {
-          best = d;
-          best_j = j;
-          outer = (dx * t[0] + dy * t[1]) + dz * t[2] >= 0.f;
-        }
-      };
+      float nearest = near;
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1) nearest = fminf(nearest, __shfl_xor(nearest, d));
+      const uint64_t at_min = __ballot(near == nearest && near < INFINITY);
       if (at_min) {
         const int l = __ffsll((unsigned long long)at_min) - 1;
         measure(s_list[c0 + uint32_t(__builtin_amdgcn_readlane(near_k, l)) * 64u + uint32_t(l)]);
       }
-      const float W = fminf((wu + wr) * (1.f + kMeshSlack), U);
+      const float W = wave_max(best);
 #pragma unroll
       for (int k = 0; k < kMeshHeld; k++) {
         const uint32_t e0 = c0 + uint32_t(k) * 64u;
@@ -2778,20 +2823,23 @@ __global__ __launch_bounds__(kMeshThreads) void k_mesh_sdf(const float* __restri
   if (m < nc) sdf[m] = valid ? (outer ? best : -best) : 1e9f;
 }
 
-// sph: n_tris float4 of scratch
-void launch_mesh_sdf(const float* tris, float4* sph, uint32_t n_tris, const int32_t res[3], uint32_t cube, float cs,
+// scratch: kMeshScratch bytes a triangle
+void launch_mesh_sdf(const float* tris, void* scratch, uint32_t n_tris, const int32_t res[3], uint32_t cube, float cs,
                      bool exact, float* sdf, hipStream_t s) {
   const uint32_t nc = cube * cube * cube, bricks = cdiv(nc, kMeshThreads);
-  if (n_tris) k_mesh_spheres<<<cdiv(n_tris, 256), 256, 0, s>>>(tris, n_tris, sph);
+  static_assert(kMeshScratch == sizeof(float4) + sizeof(float), "centroid, radius and error");
+  float4* sph = static_cast<float4*>(scratch);
+  float* err = reinterpret_cast<float*>(sph + n_tris);
+  if (n_tris) k_mesh_spheres<<<cdiv(n_tris, 256), 256, 0, s>>>(tris, n_tris, sph, err);
   // so that no launch runs long on a large mesh: at most 2^31 triangle tests
   // (a brick against a triangle) to a launch
   const uint32_t step = std::max(1u, uint32_t((uint64_t(1) << 31) / std::max(n_tris, 1u)));
   for (uint32_t b0 = 0; b0 < bricks; b0 += step) {
     const uint32_t nb = std::min(step, bricks - b0);
     if (exact)
-      k_mesh_sdf<true><<<nb, kMeshThreads, 0, s>>>(tris, sph, n_tris, res[0], res[1], res[2], nc, b0, cs, sdf);
+      k_mesh_sdf<true><<<nb, kMeshThreads, 0, s>>>(tris, sph, err, n_tris, res[0], res[1], res[2], nc, b0, cs, sdf);
     else
-      k_mesh_sdf<false><<<nb, kMeshThreads, 0, s>>>(tris, sph, n_tris, res[0], res[1], res[2], nc, b0, cs, sdf);
+      k_mesh_sdf<false><<<nb, kMeshThreads, 0, s>>>(tris, sph, err, n_tris, res[0], res[1], res[2], nc, b0, cs, sdf);
   }
 }
 
