@@ -61,10 +61,11 @@ typedef struct nb_hash_grid {
  * predP; w unused), type_flag (n uint32, or NULL: no particle skipped),
  * cell_count and cell_offset (hash_cells uint32 each), sorted (n uint32).
  * Enqueued on hip_stream (a hipStream_t; NULL = the default stream) and
- * asynchronous.  Scratch: none for hashes of up to 2^18 cells (with n >=
- * hash_cells / 4096); else 1.25 MiB and 4 bytes per particle (without the
- * latter where they cannot be had) taken from the stream-ordered allocator
- * (hipMallocAsync) and returned to it in the same call.  n = 0 gives zero counts and offsets. */
+ * asynchronous.  Nothing of sorted past its first m entries is written.
+ * Scratch: none for hashes of up to 2^18 cells; else 1.25 MiB and 4 bytes per
+ * particle (without the latter where they cannot be had) taken from the
+ * stream-ordered allocator (hipMallocAsync) and returned to it in the same
+ * call.  n = 0 gives zero counts and offsets. */
 int nb_hash_build(const nb_hash_grid* grid, const float* pred_pos4, const uint32_t* type_flag, uint32_t n,
                   uint32_t* cell_count, uint32_t* cell_offset, uint32_t* sorted, void* hip_stream);
 

@@ -134,8 +134,12 @@ __device__ __forceinline__ void load_items(const uint32_t* __restrict__ c, uint3
   }
 }
 
+// The chunk's sum into out[b], or (OWN) for each later chunk j into out[j kChunk + b]:
+// out is then cell_offset, and the sums that a block of k_hash_offsets reads lie in the
+// part that it alone writes.
+template <bool OWN>
 __global__ __launch_bounds__(kThreads) void k_hash_chunk_sums(const uint32_t* __restrict__ cell_count, uint32_t nc,
-                                                              uint32_t* __restrict__ scratch) {
+                                                              uint32_t* __restrict__ out) {
   __shared__ uint32_t s_wave[kThreads / 64 + 1];
   uint32_t v[kItems];
   load_items(cell_count, nc, blockIdx.x * kChunk + threadIdx.x * kItems, v);
@@ -144,7 +148,11 @@ __global__ __launch_bounds__(kThreads) void k_hash_chunk_sums(const uint32_t* __
   for (uint32_t k = 0; k < kItems; k++) s += v[k];
   uint32_t tot;
   (void)nb::block_exclusive_scan<kThreads>(s, s_wave, tot);
-  if (threadIdx.x == 0) scratch[blockIdx.x] = tot;
+  if (OWN) {
+    for (uint32_t j = blockIdx.x + 1u + threadIdx.x; j < gridDim.x; j += kThreads) out[size_t(j) * kChunk + blockIdx.x] = tot;
+  } else if (threadIdx.x == 0) {
+    out[blockIdx.x] = tot;
+  }
 }
 
 // exclusive scan of the chunk sums in place, one block of 1024 threads
@@ -166,8 +174,10 @@ __global__ __launch_bounds__(1024) void k_hash_chunk_scan(uint32_t* __restrict__
 // START offsets (END: END offsets): the chunk's base plus the prefix inside the chunk.
 // SUMS: scratch holds the chunks' sums and each block adds up those before its
 // own, which saves the scan's launch (a whole kernel is 2-5 us of stream time)
-// and reads at most kSumChunks words a block; else it holds their scan.
-template <bool SUMS, bool END>
+// and reads at most kSumChunks words a block; OWN: these sums stand in the block's
+// own part of cell_off; SCAN: scratch holds the sums' scan.
+enum class Base { SCAN, SUMS, OWN };
+template <Base FROM, bool END>
 __global__ __launch_bounds__(kThreads) void k_hash_offsets(const uint32_t* __restrict__ cell_count, uint32_t nc,
                                                            const uint32_t* __restrict__ scratch,
                                                            uint32_t* __restrict__ cell_off) {
@@ -180,10 +190,11 @@ __global__ __launch_bounds__(kThreads) void k_hash_offsets(const uint32_t* __res
   for (uint32_t k = 0; k < kItems; k++) s += v[k];
   uint32_t tot;
   uint32_t base;
-  if (SUMS) {
+  if (FROM != Base::SCAN) {
     uint32_t b = 0;
-    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kThreads) b += scratch[i];
-    (void)nb::block_exclusive_scan<kThreads>(b, s_wave, base);
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kThreads)
+      b += FROM == Base::OWN ? cell_off[size_t(blockIdx.x) * kChunk + i] : scratch[i];
+    (void)nb::block_exclusive_scan<kThreads>(b, s_wave, base);  // its barriers part these reads from the writes below
   } else {
     base = scratch[blockIdx.x];
   }
@@ -468,15 +479,14 @@ int validate_hash_build(const nb_hash_grid* grid, const float* pred_pos4, uint32
   return NB_OK;
 }
 
-// Whether a build needs no scratch: the chunk sums fit `sorted`, which is free
-// until the scatter, and the crowded pass finds its cells by itself (a sweep
-// of at most 1 MB of counts).  Taking scratch from the stream-ordered
+// Whether a build needs no scratch: the chunks' sums stand in cell_offset until the
+// offsets do (at most 64 of them, and a chunk that has another before it is whole,
+// hash_cells being a power of two), and the crowded pass finds its cells by itself (a
+// sweep of at most 1 MB of counts).  Taking scratch from the stream-ordered
 // allocator and giving it back costs 25 us of host time, as much as all of a
 // small build: 32,768 particles in 64^3 cells took 48 us with it and take
 // 27 without.
-bool hash_needs_no_scratch(const nb_hash_grid* grid, uint32_t n) {
-  return grid->hash_cells <= (1u << 18) && n >= (grid->hash_cells + nbh::kChunk - 1u) / nbh::kChunk;
-}
+bool hash_needs_no_scratch(const nb_hash_grid* grid) { return grid->hash_cells <= (1u << 18); }
 
 // Enqueues a validated hash build with the given scratch (hash_scratch_words()
 // uint32 of device memory; null when hash_needs_no_scratch) and, or null, n words
@@ -496,7 +506,6 @@ int enqueue_hash_build(const nb_hash_grid* grid, const float* pred_pos4, const u
   const uint32_t nchunks = (nc + kChunk - 1u) / kChunk;
   const uint32_t pblocks = uint32_t((uint64_t(n) + kThreads - 1u) / kThreads);
   const bool sums = nchunks <= kSumChunks;
-  uint32_t* chunk_sums = scratch ? scratch : sorted;
   // four cells a thread where most cells are empty and their counts are
   // bandwidth (16.8 M cells, 2 M particles: 22 us against 38); in a small hash
   // the four turns of a thread are latency (262,144 cells, 32,768 particles: 9.8
@@ -509,15 +518,20 @@ int enqueue_hash_build(const nb_hash_grid* grid, const float* pred_pos4, const u
     hipLaunchKernelGGL(k_hash_count<true>, dim3(pblocks), dim3(kThreads), 0, s, g, pred, type_flag, n, cell_count, rank);
   else if (n)
     hipLaunchKernelGGL(k_hash_count<false>, dim3(pblocks), dim3(kThreads), 0, s, g, pred, type_flag, n, cell_count, rank);
-  hipLaunchKernelGGL(k_hash_chunk_sums, dim3(nchunks), dim3(kThreads), 0, s, cell_count, nc, chunk_sums);
-  if (!sums) hipLaunchKernelGGL(k_hash_chunk_scan, dim3(1), dim3(1024), 0, s, chunk_sums, nchunks);
-#define NB_OFFSETS(SM, EN)                                                                                       \
-  hipLaunchKernelGGL((k_hash_offsets<SM, EN>), dim3(nchunks), dim3(kThreads), 0, s, cell_count, nc, chunk_sums, \
+  if (scratch)
+    hipLaunchKernelGGL(k_hash_chunk_sums<false>, dim3(nchunks), dim3(kThreads), 0, s, cell_count, nc, scratch);
+  else if (nchunks > 1u)
+    hipLaunchKernelGGL(k_hash_chunk_sums<true>, dim3(nchunks), dim3(kThreads), 0, s, cell_count, nc, cell_offset);
+  if (!sums) hipLaunchKernelGGL(k_hash_chunk_scan, dim3(1), dim3(1024), 0, s, scratch, nchunks);
+#define NB_OFFSETS(FR, EN)                                                                                            \
+  hipLaunchKernelGGL((k_hash_offsets<Base::FR, EN>), dim3(nchunks), dim3(kThreads), 0, s, cell_count, nc, scratch, \
                      cell_offset)
-  if (sums) {
-    if (rank) NB_OFFSETS(true, true); else NB_OFFSETS(true, false);
+  if (!scratch) {
+    NB_OFFSETS(OWN, false);
+  } else if (sums) {
+    if (rank) NB_OFFSETS(SUMS, true); else NB_OFFSETS(SUMS, false);
   } else {
-    if (rank) NB_OFFSETS(false, true); else NB_OFFSETS(false, false);
+    if (rank) NB_OFFSETS(SCAN, true); else NB_OFFSETS(SCAN, false);
   }
 #undef NB_OFFSETS
   if (n) {
@@ -548,7 +562,7 @@ extern "C" int nb_hash_build(const nb_hash_grid* grid, const float* pred_pos4, c
   const int v = nb::validate_hash_build(grid, pred_pos4, n, cell_count, cell_offset, sorted);
   if (v != NB_OK) return v;
   hipStream_t s = static_cast<hipStream_t>(hip_stream);
-  if (nb::hash_needs_no_scratch(grid, n))
+  if (nb::hash_needs_no_scratch(grid))
     return nb::enqueue_hash_build(grid, pred_pos4, type_flag, n, cell_count, cell_offset, sorted, nullptr, nullptr, s);
   void* scratch = nullptr;
   // with room for the particles' places in their cells, or, where there is none,
@@ -624,7 +638,7 @@ extern "C" int nb_hash_build_noalloc(const nb_hash_grid* grid, const float* pred
   if (grid->hash_cells > NB_HASH_MAX_CELLS)
     return nb::set_error(NB_ERR_ARG, "nb_hash_build_noalloc: hash_cells = %u exceeds the scratch array's %u",
                          grid->hash_cells, NB_HASH_MAX_CELLS);
-  if (nb::hash_needs_no_scratch(grid, n))
+  if (nb::hash_needs_no_scratch(grid))
     return nb::enqueue_hash_build(grid, pred_pos4, type_flag, n, cell_count, cell_offset, sorted, nullptr, nullptr,
                                   static_cast<hipStream_t>(hip_stream));
   uint32_t* s = nullptr;
