@@ -122,6 +122,7 @@ struct nb_mpm {
   bool keys_valid = false;
   bool counted = false;
   bool counts_dirty = false;
+  bool fb_pending = false;  // the last G2P left the FP64 fallback's queue to the next bin
   GridMode grid_mode = GridMode::NONE;
   bool old_valid = false;
   std::vector<void*> allocs;
@@ -316,7 +317,15 @@ void bin(nb_mpm* h, const DevState& dv, const SubParams& p, Prof* pf) {
   const BinFrom from = !h->keys_valid ? BinFrom::RECORDS : (h->counted ? BinFrom::COUNTED : BinFrom::KEYS);
   if (from != BinFrom::COUNTED && h->counts_dirty) launch_clear_counts(dv, h->NT, h->stream);
   launch_bin(dv, p, h->NT, from, h->stream, pf);
-  h->counted = h->counts_dirty = false;
+  h->counted = h->counts_dirty = h->fb_pending = false;
+}
+
+// After a run of substeps (of dt): the fallback's queue, where the last G2P left it to a
+// next bin or the run ended early, worked off on rec, or dropped (null).  The queue has room for one G2P's entries and they are of the state
+// that it left, so none stay behind when a call returns.
+void settle_queue(nb_mpm* h, float4* rec, float dt) {
+  if (h->fb_pending) launch_g2p_fb(h->dev(), h->params(dt, false), rec, h->stream, nullptr);
+  h->fb_pending = false;
 }
 
 // one substep on the records (the caller brackets a run of them with
@@ -377,7 +386,7 @@ int enqueue_substep(nb_mpm* h, float dt, Prof* pf, bool last, const TapeIO& io =
     bin(h, dv, p, pf);
     launch_p2g(dv, p, h->NT, h->stream, pf);
     launch_g2p_fused(dv, p, h->NT, h->stream, pf);
-    if (last) launch_g2p_fb(dv, p, dv.rec, h->stream, pf);
+    h->fb_pending = p.svd_fp64 != 0u;
     NB_HIP(hipGetLastError());
     h->bins_valid = true;
     h->keys_valid = h->counted = h->counts_dirty = true;
@@ -403,6 +412,7 @@ int enqueue_substep(nb_mpm* h, float dt, Prof* pf, bool last, const TapeIO& io =
   const bool count = !(last && h->ptr_exported);
   launch_g2p(dv, p, true, count, h->stream, pf, io.rec_out);
   if (last) launch_g2p_fb(dv, p, io.rec_out ? io.rec_out : dv.rec, h->stream, pf);
+  h->fb_pending = !last && p.svd_fp64 != 0u;
   NB_HIP(hipGetLastError());
   substep_done(h, flip, count);
   return NB_OK;
@@ -418,8 +428,51 @@ int run_substeps(nb_mpm* h, float dt, uint32_t n, Prof* pf) {
   // last substep's, as after the reference's step
   for (uint32_t i = 0; i < n && rc == NB_OK; i++)
     rc = enqueue_substep(h, dt, pf, i + 1 == n, TapeIO{}, h->fuse_g2p && i + 1 < n);
+  settle_queue(h, h->d.rec, dt);
   if (rc == NB_OK) rc = sync_out(h);
   return rc;
+}
+
+// n substeps as replays of one captured substep
+int replay_substeps(nb_mpm* h, float dt_sub, uint32_t n) {
+  int rc = sync_in(h, true);
+  // the captured substep starts from the keys and counts the previous G2P left
+  // and leaves the same, and the fallback's queue, to the next
+  if (rc == NB_OK && !(h->keys_valid && h->counted)) {
+    rc = enqueue_substep(h, dt_sub, nullptr, n == 1);
+    n--;
+  }
+  if (rc != NB_OK || n == 0) return rc;
+  const SubParams p = h->params(dt_sub, h->knobs.flip_ratio > 0.01f);
+  const DevState dv = h->dev();
+  if (!h->graph_exec || std::memcmp(&p, &h->graph_p, sizeof(p)) != 0 ||
+      std::memcmp(&dv, &h->graph_d, sizeof(dv)) != 0) {
+    if (h->graph_exec) {
+      (void)hipGraphExecDestroy(h->graph_exec);
+      h->graph_exec = nullptr;
+    }
+    NB_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
+    rc = enqueue_substep(h, dt_sub, nullptr, false);
+    hipGraph_t g = nullptr;
+    const hipError_t e = hipStreamEndCapture(h->stream, &g);
+    if (rc != NB_OK || e != hipSuccess) {
+      if (g) (void)hipGraphDestroy(g);
+      return rc != NB_OK ? rc : fail(NB_ERR_HIP, "hipStreamEndCapture failed: %s", hipGetErrorString(e));
+    }
+    const hipError_t ei = hipGraphInstantiate(&h->graph_exec, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    if (ei != hipSuccess) {
+      h->graph_exec = nullptr;
+      return fail(NB_ERR_HIP, "hipGraphInstantiate failed: %s", hipGetErrorString(ei));
+    }
+    h->graph_p = p;
+    h->graph_d = dv;
+  }
+  // a replay of an earlier capture runs none of the host's code
+  substep_done(h, p.write_old != 0u, true);
+  h->fb_pending = p.svd_fp64 != 0u;
+  for (uint32_t i = 0; i < n; i++) NB_HIP(hipGraphLaunch(h->graph_exec, h->stream));
+  return NB_OK;
 }
 
 }  // namespace
@@ -813,44 +866,9 @@ int nb_mpm_set_tuning(nb_mpm* h, const nb_mpm_tuning* t) {
 int nb_mpm_graph_substeps(nb_mpm* h, float dt_sub, uint32_t n) {
   if (!h) return fail(NB_ERR_ARG, "null handle");
   if (n == 0 || h->n_live == 0) return NB_OK;
-  int rc = sync_in(h, true);
-  // the captured substep starts from the keys and counts the previous G2P left
-  // and leaves the same, and the fallback's queue, to the next
-  if (rc == NB_OK && !(h->keys_valid && h->counted)) {
-    rc = enqueue_substep(h, dt_sub, nullptr, n == 1);
-    n--;
-  }
-  if (rc == NB_OK && n) {
-    const SubParams p = h->params(dt_sub, h->knobs.flip_ratio > 0.01f);
-    const DevState dv = h->dev();
-    if (!h->graph_exec || std::memcmp(&p, &h->graph_p, sizeof(p)) != 0 ||
-        std::memcmp(&dv, &h->graph_d, sizeof(dv)) != 0) {
-      if (h->graph_exec) {
-        (void)hipGraphExecDestroy(h->graph_exec);
-        h->graph_exec = nullptr;
-      }
-      NB_HIP(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-      rc = enqueue_substep(h, dt_sub, nullptr, false);
-      hipGraph_t g = nullptr;
-      const hipError_t e = hipStreamEndCapture(h->stream, &g);
-      if (rc != NB_OK || e != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        return rc != NB_OK ? rc : fail(NB_ERR_HIP, "hipStreamEndCapture failed: %s", hipGetErrorString(e));
-      }
-      const hipError_t ei = hipGraphInstantiate(&h->graph_exec, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      if (ei != hipSuccess) {
-        h->graph_exec = nullptr;
-        return fail(NB_ERR_HIP, "hipGraphInstantiate failed: %s", hipGetErrorString(ei));
-      }
-      h->graph_p = p;
-      h->graph_d = dv;
-    }
-    for (uint32_t i = 0; i < n; i++) NB_HIP(hipGraphLaunch(h->graph_exec, h->stream));
-    launch_g2p_fb(dv, p, dv.rec, h->stream, nullptr);
-    NB_HIP(hipGetLastError());
-    substep_done(h, p.write_old != 0u, true);  // a replay of an earlier capture has run none of the host's code
-  }
+  int rc = replay_substeps(h, dt_sub, n);
+  settle_queue(h, h->d.rec, dt_sub);
+  NB_HIP(hipGetLastError());
   if (rc == NB_OK) rc = sync_out(h);
   return rc;
 }
@@ -941,6 +959,7 @@ int nb_mpm_autotune(nb_mpm* h, float dt_sub, uint32_t trial_substeps, uint32_t f
     if (!(t_best < 0.99f * t_start)) best = start, best_ms = 0.5f * t_start;
     else best_ms = 0.5f * t_best;
   }
+  settle_queue(h, nullptr, 0.f);  // of a trial that failed
   restore();
   release();
   if (!ok) {
@@ -1864,6 +1883,7 @@ int nb_mpm_forward_recorded(nb_mpm* h, float dt_sub) {
   h->keys_valid = h->counted = false;  // the first substep writes its keys into the first key slot
   for (uint32_t s = 0; s < A.n && rc == NB_OK; s++)
     rc = enqueue_substep(h, dt_sub, nullptr, s + 1 == A.n, tape_io(h, s, adj_next(h, s), key_next(h, s)));
+  settle_queue(h, nullptr, 0.f);
   h->grid_mode = GridMode::NONE;  // the grids went to the tape
   h->bins_valid = false;          // and the bins to the tape's bin buffers
   if (rc == NB_OK) rc = sync_out(h);
@@ -1943,6 +1963,7 @@ int nb_mpm_backward(nb_mpm* h, float* d_params, uint32_t params_cap) {
       std::swap(in, out);
     }
   }
+  settle_queue(h, nullptr, 0.f);
   if (rc != NB_OK) return rc;
   launch_adjoint_params(A.a, h->n_live, h->material_count, h->stream);
   NB_HIP(hipGetLastError());

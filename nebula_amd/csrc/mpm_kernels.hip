@@ -2485,11 +2485,11 @@ void launch_g2p_fused(const DevState& d, const SubParams& p, uint32_t n_tiles, h
 }
 
 // The FP64 fallback's fix-up after a call's last G2P, which leaves its queue
-// empty (nothing to do when it is off).
+// empty (nothing to do when it is off); without records it only empties it.
 void launch_g2p_fb(const DevState& d, const SubParams& p, float4* rec, hipStream_t s, Prof* pf) {
   if (!p.svd_fp64) return;
   ProfScope ps(pf, 9, s);
-  launch_fb_entries(d, p, rec, s);
+  if (rec) launch_fb_entries(d, p, rec, s);
   k_g2p_fb_reset<<<1, 64, 0, s>>>(p.fb_ctl);
 }
 

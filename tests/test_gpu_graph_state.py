@@ -49,3 +49,23 @@ def test_bins_and_grid_after_a_replay(gpu_lib, name, flip_ratio):
     for what, a, b in zip(("keys", "sorted", "count", "end"), eager.getBins(), graph.getBins()):
         assert np.array_equal(a, b), what
     assert np.array_equal(eager.getState().view(np.uint32), graph.getState().view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [1, 2, 5])
+def test_fallback_queue_is_worked_off_within_the_call(gpu_lib, n):
+    """Every particle takes the FP64 fallback (equal singular values): a replayed run's
+    last queue is settled with that run's time step, and nothing of it is left for the
+    standalone G2P, whose own entries need the whole queue."""
+    sc = _scenes()[2]
+    sc.fields[2:5, :, :3] = (np.eye(3) * (0.98, 0.95, 0.98))[:, None]
+    eager, graph = make_engine(sc), make_engine(sc)
+    for e, run in ((eager, eager.substep), (graph, graph.graphSubstep)):
+        e.setSvdFallback(count_stats=True)
+        e.svdFallbackStats(reset=True)
+        for dt in (sc.dt, 0.5 * sc.dt):
+            run(dt, n)
+            e.runBin()
+            e.runG2P(dt)
+    assert eager.svdFallbackStats() == graph.svdFallbackStats()
+    assert eager.svdFallbackStats()["fp64_return_map_lanes"] >= sc.n
+    assert np.array_equal(eager.getState().view(np.uint32), graph.getState().view(np.uint32))
