@@ -5,7 +5,8 @@
 // hash_scan_local, hash_scan_global, hash_add_base, hash_sort) over
 // engine-owned buffers.  Here:
 //   k_hash_clear      zero cell_count (and the scratch counter)
-//   k_hash_count      cell of every particle, one atomic count per run of lanes
+//   k_hash_count      cell of every particle, one atomic count per run of lanes (in
+//                     few cells: per cell of a wave)
 //   k_hash_chunk_sums / k_hash_chunk_scan / k_hash_offsets
 //                     exclusive prefix of the counts in two levels (4096 cells
 //                     per block; no group-count limit; the scan kernel only
@@ -15,11 +16,12 @@
 //                     atomicAdd(START of the cell) -> cell_offset ends as END
 //                     offsets, as after hash_sort
 //   k_hash_stabilize  every cell's slice of `sorted` put in ascending particle
-//                     order: cells of <= 16 in registers by a sorting network,
-//                     of <= 256 by their wave, more crowded cells listed for
-//                     k_hash_crowded
-//   k_hash_crowded    one block per crowded cell: bitonic sort in LDS (up to
-//                     16384 particles) or in place in global memory
+//                     order: cells of <= 16 in registers by a sorting network, of
+//                     <= 512 by a wave (in larger hashes, many: listed), more
+//                     crowded ones left for k_hash_crowded
+//   k_hash_crowded    listed cells of <= 512 by a wave each, larger ones by a
+//                     block each: bitonic sort in LDS (up to 16384 particles) or
+//                     in place in global memory
 // Per-particle work reads the 16-byte predP (and typeFlag).  The result does not depend on the order of the
 // atomics, so it is deterministic.
 #include <hip/hip_runtime.h>
@@ -43,7 +45,9 @@ constexpr uint32_t kSmall = 16;                         // cells up to this size
 constexpr uint32_t kLdsSort = 16384;                    // crowded cells up to this size: sorted in LDS
 constexpr uint32_t kCrowdThreads = 512;
 constexpr uint32_t kSumChunks = 4096;                   // up to this many chunks: no scan kernel
-constexpr uint32_t kWaveSort = 256;                     // crowded cells up to this size: sorted by their wave
+constexpr uint32_t kWaveSort = 512;                     // crowded cells up to this size: sorted by one wave
+constexpr uint32_t kWaveCells = 4;                      // so many of them the wave that meets them sorts at once
+constexpr uint32_t kBigStep = 256;                      // every cell of more than kWaveSort has a multiple of it
 constexpr uint32_t kCrowdCap = 65536;                   // listed crowded cells; beyond: a dense sweep
 // scratch layout (uint32 words)
 constexpr uint32_t kOffCrowdCount = kMaxChunks;         // after the chunk sums
@@ -65,26 +69,53 @@ __device__ __forceinline__ uint32_t hash_cell(const Geo& g, const float4 p) {
   return nb::morton3(uint32_t(lx), uint32_t(ly), uint32_t(lz));
 }
 
-// Adds one per valid lane to counters[key], one atomic per run of equal keys in
-// neighbouring lanes; returns the value before the run's add plus the lane's
-// place in it.  Call from uniform control flow.  (Grouping all equal keys of a
-// wave takes one turn of a loop per distinct key, 64 in particles stored in no
-// spatial order: 94 us for the count of 2,000,003 such particles and 148 for
-// their scatter, against 83 and 128 this way, bound by the cells'
-// lines then, one moved by each atomic; for 32,768 of them 11 and 12 us against
-// 4.6 and 5.1.  Particles in spatial order have few runs a wave either way.)
-__device__ __forceinline__ uint32_t wave_run_add(uint32_t* __restrict__ counters, uint32_t key, bool valid) {
+// Adds one per valid lane to counters[key]; returns the value before the lane's
+// atomic's add plus the lane's place among the lanes it covers.  Call from uniform
+// control flow.
+// One atomic per run of equal keys in neighbouring lanes: particles stored in no
+// spatial order have 64 runs a wave, and a loop that groups all equal keys takes a turn
+// for each (94 us for the count of 2,000,003 such particles in 256 x 128 x 200 cells
+// and 148 for their scatter, against 83 and 128 by runs, bound by the cells' lines
+// then, one moved by each atomic; 32,768 in 64^3 cells: 11 and 12 us against 4.6 and
+// 5.1).  In few cells the atomics themselves meet: 200,000 particles in 4^3 cells took
+// 287 us by runs and 63 in groups.  Equal keys in different runs tell the two apart,
+// looked for at four of the wave's lanes (32,768 particles in 8^3 cells: 11 and 15 us;
+// two waves in five find a pair there, nearly all do in 4^3 cells).
+__device__ __forceinline__ uint32_t wave_add(uint32_t* __restrict__ counters, uint32_t key, bool valid) {
   const uint32_t lane = threadIdx.x & 63u;
+  const uint64_t below = (1ull << lane) - 1ull;
   const uint32_t k = valid ? key : 0xFFFFFFFFu;  // no cell has this key
   const uint32_t before = uint32_t(__shfl_up(int(k), 1));
   const uint64_t heads = __ballot(lane == 0u || before != k);
-  const uint32_t head = 63u - uint32_t(__clzll((long long)(heads & (~0ull >> (63u - lane)))));
-  uint32_t base = 0;
-  if (valid && head == lane) {
-    const uint64_t after = lane == 63u ? 0ull : heads >> (lane + 1u);
-    base = atomicAdd(&counters[key], after ? uint32_t(__ffsll((unsigned long long)after)) : 64u - lane);
+  auto in_runs = [&](int l) {
+    const uint32_t kl = uint32_t(__builtin_amdgcn_readlane(int(k), l));
+    const uint64_t peers = __ballot(k == kl) & heads;
+    return kl != 0xFFFFFFFFu && (peers & (peers - 1ull)) != 0ull;
+  };
+  uint32_t leader, place, count = 0, base = 0;
+  if (!(in_runs(0) || in_runs(16) || in_runs(32) || in_runs(48))) {
+    leader = 63u - uint32_t(__clzll((long long)(heads & (below | (1ull << lane)))));
+    place = lane - leader;
+    const uint64_t after = heads & ~(below | (1ull << lane));
+    count = (after ? uint32_t(__ffsll((unsigned long long)after)) - 1u : 64u) - lane;
+  } else {
+    leader = lane;
+    place = 0;
+    uint64_t pending = __ballot(valid);
+    while (pending) {
+      const int l = __ffsll((unsigned long long)pending) - 1;
+      const bool mine = k == uint32_t(__builtin_amdgcn_readlane(int(k), l));
+      const uint64_t peers = __ballot(mine);
+      if (mine) {
+        leader = uint32_t(l);
+        place = uint32_t(__popcll(peers & below));
+        count = uint32_t(__popcll(peers));
+      }
+      pending &= ~peers;
+    }
   }
-  return uint32_t(__shfl(int(base), int(head))) + (lane - head);
+  if (valid && leader == lane) base = atomicAdd(&counters[key], count);
+  return uint32_t(__shfl(int(base), int(leader))) + place;
 }
 
 __global__ __launch_bounds__(kThreads) void k_hash_clear(uint32_t* __restrict__ cell_count, uint32_t nc,
@@ -114,7 +145,7 @@ __global__ __launch_bounds__(kThreads) void k_hash_count(Geo g, const float4* __
     if (type_flag != nullptr && type_flag[i] == NB_HASH_TYPE_UNUSED) valid = false;
     else key = hash_cell(g, pred[i]);
   }
-  const uint32_t r = wave_run_add(cell_count, key, valid);
+  const uint32_t r = wave_add(cell_count, key, valid);
   if (RANKED && valid) rank[i] = r;
 }
 
@@ -226,7 +257,7 @@ __global__ __launch_bounds__(kThreads) void k_hash_scatter(Geo g, const float4* 
     if (type_flag != nullptr && type_flag[i] == NB_HASH_TYPE_UNUSED) valid = false;
     else key = hash_cell(g, pred[i]);
   }
-  const uint32_t slot = wave_run_add(cell_off, key, valid);
+  const uint32_t slot = wave_add(cell_off, key, valid);
   if (valid) sorted[slot] = i;
 }
 
@@ -310,15 +341,67 @@ __device__ __forceinline__ void wave_sort_cell(uint32_t* __restrict__ seg, uint3
     if (64u * e + lane < cnt) seg[64u * e + lane] = v[e];
 }
 
+// a crowded cell of up to kWaveSort particles, by its wave
+__device__ __forceinline__ void wave_sort_cell_of(uint32_t* __restrict__ seg, uint32_t cnt) {
+  if (cnt <= 64u) wave_sort_cell<1>(seg, cnt);
+  else if (cnt <= 256u) wave_sort_cell<4>(seg, cnt);
+  else wave_sort_cell<8>(seg, cnt);
+}
+
+// Without a list the crowded cells are found from `sorted` itself: a cell of more than
+// `step` particles has some at a multiple of step, the first of which is its own, so
+// one lane a multiple looks its particle's cell up.  That deals the cells out by the
+// particles they hold, whatever part of the grid is crowded.  (A place read while its
+// cell is being sorted holds some particle of the same cell.)  Count, cell and start of
+// the cell whose first multiple of step the place `at` is, else 0.
+__device__ __forceinline__ uint32_t crowded_at(const Geo& g, const float4* __restrict__ pred,
+                                               const uint32_t* __restrict__ cell_count,
+                                               const uint32_t* __restrict__ cell_off, const uint32_t* sorted,
+                                               uint64_t at, uint32_t used, uint32_t step, uint32_t& c, uint32_t& start) {
+  c = start = 0u;
+  if (at >= used) return 0u;
+  c = hash_cell(g, pred[sorted[at]]);
+  const uint32_t cnt = cell_count[c];
+  start = cell_off[c] - cnt;
+  return at - start < step ? cnt : 0u;
+}
+// the cells of kSmall to kWaveSort at the lanes' places, one after the other by the wave
+__device__ __forceinline__ void sort_crowded_at(const Geo& g, const float4* __restrict__ pred,
+                                                const uint32_t* __restrict__ cell_count,
+                                                const uint32_t* __restrict__ cell_off, uint32_t* sorted, uint64_t at,
+                                                uint32_t used) {
+  uint32_t c, start;
+  const uint32_t cnt = crowded_at(g, pred, cell_count, cell_off, sorted, at, used, kSmall, c, start);
+  uint64_t mid = __ballot(cnt > kSmall && cnt <= kWaveSort);
+  while (mid) {
+    const int l = __ffsll((unsigned long long)mid) - 1;
+    mid &= mid - 1ull;
+    wave_sort_cell_of(sorted + uint32_t(__builtin_amdgcn_readlane(int(start), l)),
+                      uint32_t(__builtin_amdgcn_readlane(int(cnt), l)));
+  }
+}
+
 // One thread per cell, or per V = 4 consecutive cells where most are empty:
 // the counts then come in 16-byte loads and the offsets are read only beside a
-// cell that needs them.
-template <uint32_t V>
-__global__ __launch_bounds__(kThreads) void k_hash_stabilize(const uint32_t* __restrict__ cell_count,
+// cell that needs them.  Crowded cells of up to kWaveSort particles: with a list, a
+// wave sorts the few it meets itself, one after the other, and lists more; without, the
+// waves of the launch's first find_blocks blocks find them, `lanes` lanes of each at a
+// multiple of kSmall.  (Sorted by the wave that meets them, however many: 165 us for
+// 200,000 particles of which the cells hold 37 each, 120 for 8^3 cells of 64, 64 for
+// 2,000 particles in 4^3 cells.)
+template <uint32_t V, bool LIST>
+__global__ __launch_bounds__(kThreads) void k_hash_stabilize(Geo g, const float4* __restrict__ pred,
+                                                             const uint32_t* __restrict__ cell_count,
                                                              const uint32_t* __restrict__ cell_off, uint32_t nc,
-                                                             uint32_t* __restrict__ sorted,
-                                                             uint32_t* __restrict__ scratch) {
-  const uint32_t c0 = (blockIdx.x * kThreads + threadIdx.x) * V;
+                                                             uint32_t* sorted, uint32_t* __restrict__ scratch,
+                                                             uint32_t find_blocks, uint32_t lanes) {
+  if (!LIST && blockIdx.x < find_blocks) {
+    const uint32_t lane = threadIdx.x & 63u, wave = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+    const uint64_t at = lane < lanes ? (uint64_t(wave) * lanes + lane) * kSmall : ~0ull;
+    sort_crowded_at(g, pred, cell_count, cell_off, sorted, at, cell_off[nc - 1u]);
+    return;
+  }
+  const uint32_t c0 = ((LIST ? blockIdx.x : blockIdx.x - find_blocks) * kThreads + threadIdx.x) * V;
   uint32_t n[V];
   if (V == 4u && c0 + 4u <= nc && (reinterpret_cast<uintptr_t>(cell_count) & 15u) == 0u) {
     const uint4 q = *reinterpret_cast<const uint4*>(cell_count + c0);
@@ -332,19 +415,24 @@ __global__ __launch_bounds__(kThreads) void k_hash_stabilize(const uint32_t* __r
     const uint32_t cnt = n[k];
     if (!__any(cnt >= 2u)) continue;
     const uint32_t start = cnt >= 2u ? cell_off[c0 + k] - cnt : 0u;
-    if (scratch != nullptr && cnt > kWaveSort) {
-      const uint32_t slot = atomicAdd(&scratch[kOffCrowdCount], 1u);
-      if (slot < kCrowdCap) scratch[kOffCrowdList + slot] = c0 + k;
-    }
-    // cells of 17..256, one after the other by the whole wave
-    uint64_t mid = __ballot(cnt > kSmall && cnt <= kWaveSort);
-    while (mid) {
-      const int l = __ffsll((unsigned long long)mid) - 1;
-      mid &= mid - 1ull;
-      const uint32_t m = uint32_t(__builtin_amdgcn_readlane(int(cnt), l));
-      uint32_t* seg = sorted + uint32_t(__builtin_amdgcn_readlane(int(start), l));
-      if (m <= 64u) wave_sort_cell<1>(seg, m);
-      else wave_sort_cell<4>(seg, m);
+    if (LIST) {
+      uint64_t mid = __ballot(cnt > kSmall && cnt <= kWaveSort);
+      const bool few = uint32_t(__popcll(mid)) <= kWaveCells / V;
+      const bool listed = cnt > kWaveSort || (!few && cnt > kSmall);
+      const uint64_t list = __ballot(listed);
+      if (list) {
+        const uint32_t lane = threadIdx.x & 63u, first = uint32_t(__ffsll((unsigned long long)list)) - 1u;
+        uint32_t at = 0;
+        if (lane == first) at = atomicAdd(&scratch[kOffCrowdCount], uint32_t(__popcll(list)));
+        at = uint32_t(__builtin_amdgcn_readlane(int(at), int(first))) + uint32_t(__popcll(list & ((1ull << lane) - 1ull)));
+        if (listed && at < kCrowdCap) scratch[kOffCrowdList + at] = c0 + k;
+      }
+      while (few && mid) {
+        const int l = __ffsll((unsigned long long)mid) - 1;
+        mid &= mid - 1ull;
+        wave_sort_cell_of(sorted + uint32_t(__builtin_amdgcn_readlane(int(start), l)),
+                          uint32_t(__builtin_amdgcn_readlane(int(cnt), l)));
+      }
     }
     const bool small = cnt >= 2u && cnt <= kSmall;
     // network width: the widest small cell of the wave
@@ -407,41 +495,51 @@ __device__ void sort_crowded(uint32_t* __restrict__ sorted, const uint32_t* __re
   __syncthreads();
 }
 
-// The crowded cells listed by k_hash_stabilize, one per block; when the list
-// overflowed, every block sweeps its share of all cells instead.  Without a
-// list (scratch null) block b looks at the cells b, b + gridDim.x, ..., so that
-// neighbouring crowded cells fall to different blocks.
-__global__ __launch_bounds__(kCrowdThreads) void k_hash_crowded(const uint32_t* __restrict__ cell_count,
+// The crowded cells that are left.  LIST: those k_hash_stabilize listed, up to
+// kWaveSort particles one per wave, larger ones one per block.  Without a list the
+// larger ones alone, and all of them when the list overflowed: a block takes a stretch
+// of places and the cells that crowded_at finds there.
+template <bool LIST>
+__global__ __launch_bounds__(kCrowdThreads) void k_hash_crowded(Geo g, const float4* __restrict__ pred,
+                                                                const uint32_t* __restrict__ cell_count,
                                                                 const uint32_t* __restrict__ cell_off, uint32_t nc,
-                                                                uint32_t* __restrict__ sorted,
-                                                                const uint32_t* __restrict__ scratch) {
+                                                                uint32_t* sorted, const uint32_t* __restrict__ scratch) {
   __shared__ uint32_t s_buf[kLdsSort];
   __shared__ uint32_t s_list[kCrowdThreads];
   __shared__ uint32_t s_n;
-  if (scratch == nullptr) {
-    for (uint32_t c0 = blockIdx.x; c0 < nc; c0 += gridDim.x * kCrowdThreads) {
-      if (threadIdx.x == 0) s_n = 0;
-      __syncthreads();
-      const uint64_t c = c0 + uint64_t(threadIdx.x) * gridDim.x;
-      if (c < nc && cell_count[c] > kWaveSort) s_list[atomicAdd(&s_n, 1u)] = uint32_t(c);
-      __syncthreads();
-      const uint32_t k = s_n;
-      for (uint32_t e = 0; e < k; e++) sort_crowded(sorted, cell_count, cell_off, s_list[e], s_buf);
-      __syncthreads();
+  static_assert(kWaveSort >= kBigStep && kBigStep % kSmall == 0u, "a multiple of the step in each");
+  if (LIST) {
+    const uint32_t m = scratch[kOffCrowdCount];
+    if (m <= kCrowdCap) {
+      for (uint32_t e = blockIdx.x + (threadIdx.x >> 6) * gridDim.x; e < m; e += (kCrowdThreads / 64) * gridDim.x) {
+        const uint32_t c = uint32_t(__builtin_amdgcn_readfirstlane(int(scratch[kOffCrowdList + e]))), cnt = cell_count[c];
+        if (cnt <= kWaveSort) wave_sort_cell_of(sorted + (cell_off[c] - cnt), cnt);
+      }
+      for (uint32_t e = blockIdx.x; e < m; e += gridDim.x) {
+        const uint32_t c = scratch[kOffCrowdList + e];
+        if (cell_count[c] > kWaveSort) sort_crowded(sorted, cell_count, cell_off, c, s_buf);
+      }
+      return;
     }
-    return;
   }
-  const uint32_t m = scratch[kOffCrowdCount];
-  if (m <= kCrowdCap) {
-    for (uint32_t e = blockIdx.x; e < m; e += gridDim.x) sort_crowded(sorted, cell_count, cell_off,
-                                                                      scratch[kOffCrowdList + e], s_buf);
-    return;
+  const uint32_t used = cell_off[nc - 1u];
+  const uint32_t steps = used / kBigStep + (used % kBigStep ? 1u : 0u), per = (steps + gridDim.x - 1u) / gridDim.x;
+  const uint64_t first = uint64_t(blockIdx.x) * per * kBigStep;
+  if (LIST) {
+    for (uint64_t x = threadIdx.x & ~63u; x < uint64_t(per) * (kBigStep / kSmall); x += kCrowdThreads) {
+      const uint64_t y = x + (threadIdx.x & 63u);
+      sort_crowded_at(g, pred, cell_count, cell_off, sorted,
+                      y < uint64_t(per) * (kBigStep / kSmall) ? first + y * kSmall : ~0ull, used);
+    }
   }
-  for (uint32_t base = blockIdx.x * kCrowdThreads; base < nc; base += gridDim.x * kCrowdThreads) {
-    if (threadIdx.x == 0) s_n = 0;
+  for (uint32_t w = 0; w < per; w += kCrowdThreads) {
+    if (threadIdx.x == 0u) s_n = 0u;
     __syncthreads();
-    const uint32_t c = base + threadIdx.x;
-    if (c < nc && cell_count[c] > kWaveSort) s_list[atomicAdd(&s_n, 1u)] = c;
+    uint32_t c, start;
+    const uint32_t v = w + threadIdx.x;
+    const uint32_t cnt = crowded_at(g, pred, cell_count, cell_off, sorted, v < per ? first + uint64_t(v) * kBigStep : ~0ull,
+                                    used, kBigStep, c, start);
+    if (cnt > kWaveSort) s_list[atomicAdd(&s_n, 1u)] = c;
     __syncthreads();
     const uint32_t k = s_n;
     for (uint32_t e = 0; e < k; e++) sort_crowded(sorted, cell_count, cell_off, s_list[e], s_buf);
@@ -481,8 +579,8 @@ int validate_hash_build(const nb_hash_grid* grid, const float* pred_pos4, uint32
 
 // Whether a build needs no scratch: the chunks' sums stand in cell_offset until the
 // offsets do (at most 64 of them, and a chunk that has another before it is whole,
-// hash_cells being a power of two), and the crowded pass finds its cells by itself (a
-// sweep of at most 1 MB of counts).  Taking scratch from the stream-ordered
+// hash_cells being a power of two), and the crowded pass finds its cells by itself (its
+// counts, 1 MB at most, stay in the L2s).  Taking scratch from the stream-ordered
 // allocator and giving it back costs 25 us of host time, as much as all of a
 // small build: 32,768 particles in 64^3 cells took 48 us with it and take
 // 27 without.
@@ -540,15 +638,28 @@ int enqueue_hash_build(const nb_hash_grid* grid, const float* pred_pos4, const u
                          sorted);
     else
       hipLaunchKernelGGL(k_hash_scatter, dim3(pblocks), dim3(kThreads), 0, s, g, pred, type_flag, n, cell_offset, sorted);
-    if (vec == 4u)
-      hipLaunchKernelGGL(k_hash_stabilize<4>, dim3(cblocks), dim3(kThreads), 0, s, cell_count, cell_offset, nc, sorted,
-                         scratch);
-    else
-      hipLaunchKernelGGL(k_hash_stabilize<1>, dim3(cblocks), dim3(kThreads), 0, s, cell_count, cell_offset, nc, sorted,
-                         scratch);
-    // 64 KB of LDS a block: two fit a CU, so 512 blocks are all that run at once
-    hipLaunchKernelGGL(k_hash_crowded, dim3(512), dim3(kCrowdThreads), 0, s, cell_count, cell_offset, nc, sorted,
-                       scratch);
+    // few lanes a wave while there are waves to spare
+    const uint32_t lanes = n <= (1u << 16) ? 4u : (n <= (1u << 18) ? 16u : 64u);
+    const uint32_t find_blocks = scratch ? 0u : (n - 1u) / (nbh::kThreads / 64u * lanes * kSmall) + 1u;
+#define NB_STABILIZE(VC, LI)                                                                                           \
+  hipLaunchKernelGGL((k_hash_stabilize<VC, LI>), dim3(cblocks + find_blocks), dim3(kThreads), 0, s, g, pred, cell_count, \
+                     cell_offset, nc, sorted, scratch, find_blocks, lanes)
+    // 64 KB of LDS a block: two fit a CU, so 512 blocks run at once; twice as many
+    // where most cells are large, so that each is alone in a block's stretch (2,000,003
+    // particles in 8^3 cells: 102 us against 150; else the empty ones cost 2 us)
+    const uint32_t crowd_blocks = std::min((n - 1u) / kWaveSort + 1u, !scratch && n / kWaveSort >= nc ? 1024u : 512u);
+#define NB_CROWDED(LI)                                                                                              \
+  hipLaunchKernelGGL(k_hash_crowded<LI>, dim3(crowd_blocks), dim3(kCrowdThreads), 0, s, g, pred, cell_count,        \
+                     cell_offset, nc, sorted, scratch)
+    if (!scratch) {
+      NB_STABILIZE(1, false);
+      NB_CROWDED(false);
+    } else {
+      if (vec == 4u) NB_STABILIZE(4, true); else NB_STABILIZE(1, true);
+      NB_CROWDED(true);
+    }
+#undef NB_STABILIZE
+#undef NB_CROWDED
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(NB_ERR_HIP, "nb_hash_build: launch failed: %s", hipGetErrorString(e));
