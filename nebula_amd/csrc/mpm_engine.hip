@@ -1234,7 +1234,7 @@ int nb_mpm_set_collider_mesh(nb_mpm* h, const float* tris, uint32_t n_tris, int 
   int rc = ensure_sdf(h);
   if (rc != NB_OK) return rc;
   float* d_tris = nullptr;  // the triangles, then the scratch
-  const size_t bytes = std::max<size_t>(size_t(n_tris) * (12 * 4 + kMeshScratch), 4);
+  const size_t bytes = size_t(n_tris) * 12 * 4 + mesh_scratch(n_tris);
   NB_HIP(hipMalloc(&d_tris, bytes));
   rc = n_tris ? upload(h, d_tris, tris, size_t(n_tris) * 12 * 4) : NB_OK;
   if (rc == NB_OK) {

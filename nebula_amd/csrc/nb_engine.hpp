@@ -250,8 +250,8 @@ void launch_g2p(const DevState& d, const SubParams& p, bool use_sorted, bool cou
                 float4* rec_out = nullptr);
 void launch_sdf_sphere(float* sdf, const SubParams& p, float r, float cx, float cy, float cz, hipStream_t s);
 // the Morton SDF of a triangle mesh (n x 12 floats: normal, v0, v1, v2) on a grid of res cells of size cs
-// (scratch: kMeshScratch bytes a triangle, 16-byte aligned)
-constexpr size_t kMeshScratch = 20;
+// (scratch: mesh_scratch(n_tris) bytes, 16-byte aligned)
+inline size_t mesh_scratch(uint32_t n_tris) { return size_t(n_tris) * (sizeof(float4) + sizeof(float)) + sizeof(uint32_t); }
 void launch_mesh_sdf(const float* tris, void* scratch, uint32_t n_tris, const int32_t res[3], uint32_t cube, float cs,
                      bool exact, float* sdf, hipStream_t s);
 void launch_fill_identity(uint32_t* a, uint32_t rows, uint32_t n, hipStream_t s);
