@@ -736,7 +736,7 @@ int engine_alloc(nb_mpm* h, void* hip_stream) {
   c.add(&d.cell_count, cells);
   c.add(&d.cell_end, cells);
   c.add(&d.bucket, h->cap);
-  c.add(&d.tile_cnt, h->NT);
+  c.add(&d.tile_cnt, tile_slots(h->NT));
   c.add(&d.tile_mark, h->NT);
   c.add(&d.tile_sums, (h->NT + 255) / 256 + 1);
   c.add(&d.tile_act, h->NT);
@@ -773,7 +773,7 @@ int engine_alloc(nb_mpm* h, void* hip_stream) {
 
   auto zero = [&](void* p, size_t bytes) { return hipMemsetAsync(p, 0, bytes, h->stream); };
   if (zero(d.cell_count, cells * 4) != hipSuccess || zero(d.cell_end, cells * 4) != hipSuccess ||
-      zero(d.tile_cnt, size_t(h->NT) * 4) != hipSuccess || zero(d.counters, CNT_SLOTS * 4) != hipSuccess ||
+      zero(d.tile_cnt, size_t(tile_slots(h->NT)) * 4) != hipSuccess || zero(d.counters, CNT_SLOTS * 4) != hipSuccess ||
       zero(d.grid_node, cells * 16) != hipSuccess || zero(d.grid_old, cells * 16) != hipSuccess ||
       zero(d.materials, size_t(h->max_materials()) * 64) != hipSuccess ||
       zero(d.colliders, NB_MAX_COLLIDERS * 64) != hipSuccess || zero(d.forces, NB_MAX_FORCES * 32) != hipSuccess ||

@@ -105,7 +105,7 @@ __device__ __forceinline__ uint32_t count_in_tile(uint32_t key, uint32_t* __rest
     pending &= ~peers;
   }
   uint32_t base = 0;
-  if (place == 0u) base = atomicAdd(&tile_cnt[tile], cnt);
+  if (place == 0u) base = atomicAdd(&tile_cnt[tile_slot(tile)], cnt);
   return uint32_t(__shfl(int(base), leader_of)) + place;
 }
 
@@ -168,10 +168,10 @@ __device__ __forceinline__ void scatter_one(uint32_t n, uint32_t i, const uint32
 // offsets (the reference's cellOffset).  The counts of different waves arrive
 // in any order, so a particle's place in its cell is the number of smaller
 // indices there, counted in LDS (a cell holds about 8; lanes of one cell read
-// the same words).  A tile beyond the LDS stage places its particles in memory
-// and orders cell by cell: up to 64 particles by the cell's wave (a bitonic
-// sort across its lanes), larger cells by the block in LDS, and cells beyond
-// that by an insertion sort of their thread.
+// the same words).  A tile beyond the LDS stage places its particles in memory,
+// and 4, 16 or 64 lanes sort a cell of up to 32, 128 or 512 in registers; larger cells
+// are the block's, in LDS or in memory.  (1,048,576 particles of 16 / 32 / 64 a cell:
+// 20 / 44 / 124 us; a wave's cells one after the other 77 / 101 / 614.)
 constexpr uint32_t kSortThreads = 512;
 constexpr uint32_t kSortStage = 6144;  // particles of a tile sorted in LDS
 
@@ -194,18 +194,15 @@ __global__ __launch_bounds__(kSortThreads) void k_bin_sort(uint32_t n, const uin
   __shared__ uint32_t s_cur[kTileCells], s_start[kTileCells + 1];
   __shared__ uint32_t s_wave[kSortThreads / 64 + 1];
   __shared__ uint64_t s_wave64[kSortThreads / 64 + 1];
-  __shared__ uint16_t s_big[kTileCells];
   __shared__ uint32_t s_nbig;
   static_assert(kSortThreads == uint32_t(kTileCells), "one thread per cell");
-  const uint32_t lane = threadIdx.x & 63u;
   // the FP64 fallback's queue, worked off beside the scatter, is empty again
   if (fb_ctl != nullptr && blockIdx.x == 0u && threadIdx.x < kFbSlots) fb_ctl[threadIdx.x * kFbCtlStride] = 0u;
   const uint32_t na = counters[CNT_ACTIVE];
+  bool dense = false;
   for (uint32_t a = blockIdx.x; a < na; a += gridDim.x) {
     const uint32_t first = tile_start[a], tot = min(tile_total[a], n - min(first, n));
-    const bool staged = tot <= kSortStage;
     s_cur[threadIdx.x] = 0u;
-    if (threadIdx.x == 0u) s_nbig = 0u;
     // the first four entries of a thread (2048 of the tile) stay in registers
     typename E::T held[4];
 #pragma unroll
@@ -255,72 +252,96 @@ __global__ __launch_bounds__(kSortThreads) void k_bin_sort(uint32_t n, const uin
       for (uint32_t e = n_items + threadIdx.x; e < tot; e += kSortThreads) items[first + e] = make_uint4(0u, 0u, 0u, 0u);
     }
     __syncthreads();
-    if (staged) {
-      each([&](typename E::T u) {
-        const uint32_t c = E::cell(u), at = atomicAdd(&s_cur[c], 1u);
-        s_idx[at] = E::index(u);
-        s_cell[at] = uint16_t(c);
-      });
-      __syncthreads();
-      for (uint32_t e = threadIdx.x; e < tot; e += kSortThreads) {
-        const uint32_t v = s_idx[e], c = s_cell[e], b = s_start[c], m = s_start[c + 1u];
-        uint32_t r = b;
-        for (uint32_t j = b; j < m; j += 4u) {  // four reads in flight
-          const uint32_t w0 = s_idx[j], w1 = s_idx[j + 1u], w2 = s_idx[j + 2u], w3 = s_idx[j + 3u];
-          r += (w0 < v ? 1u : 0u) + (j + 1u < m && w1 < v ? 1u : 0u) + (j + 2u < m && w2 < v ? 1u : 0u) +
-               (j + 3u < m && w3 < v ? 1u : 0u);
-        }
-        sorted[first + r] = v;
-      }
-      __syncthreads();
+    if (tot > kSortStage) {
+      dense = true;
       continue;
     }
-    each([&](typename E::T u) { sorted[first + atomicAdd(&s_cur[E::cell(u)], 1u)] = E::index(u); });
-    __threadfence_block();
+    each([&](typename E::T u) {
+      const uint32_t c = E::cell(u), at = atomicAdd(&s_cur[c], 1u);
+      s_idx[at] = E::index(u);
+      s_cell[at] = uint16_t(c);
+    });
     __syncthreads();
-    const uint32_t start = first + ex;
-    uint64_t mid = __ballot(cnt >= 2u && cnt <= 64u);
-    while (mid) {
-      const int l = __ffsll((unsigned long long)mid) - 1;
-      mid &= mid - 1ull;
-      const uint32_t m = uint32_t(__shfl(int(cnt), l));
-      uint32_t* seg = sorted + uint32_t(__shfl(int(start), l));
-      uint32_t v = lane < m ? seg[lane] : 0xFFFFFFFFu;
-      for (uint32_t k = 2; k <= 64u; k <<= 1)
-        for (uint32_t j = k >> 1; j >= 1u; j >>= 1) {
-          const uint32_t o = uint32_t(__shfl_xor(int(v), int(j)));
-          v = ((lane & k) == 0u) == ((lane & j) == 0u) ? min(v, o) : max(v, o);
-        }
-      if (lane < m) seg[lane] = v;
-    }
-    if (cnt > 64u && cnt <= kSortStage) {
-      s_big[atomicAdd(&s_nbig, 1u)] = uint16_t(threadIdx.x);
-    } else if (cnt > kSortStage) {
-      for (uint32_t k = start + 1; k < start + cnt; k++) {
-        const uint32_t v = sorted[k];
-        uint32_t j = k;
-        while (j > start && sorted[j - 1] > v) {
-          sorted[j] = sorted[j - 1];
-          j--;
-        }
-        sorted[j] = v;
+    for (uint32_t e = threadIdx.x; e < tot; e += kSortThreads) {
+      const uint32_t v = s_idx[e], c = s_cell[e], b = s_start[c], m = s_start[c + 1u];
+      uint32_t r = b;
+      for (uint32_t j = b; j < m; j += 4u) {  // four reads in flight
+        const uint32_t w0 = s_idx[j], w1 = s_idx[j + 1u], w2 = s_idx[j + 2u], w3 = s_idx[j + 3u];
+        r += (w0 < v ? 1u : 0u) + (j + 1u < m && w1 < v ? 1u : 0u) + (j + 2u < m && w2 < v ? 1u : 0u) +
+             (j + 3u < m && w3 < v ? 1u : 0u);
       }
+      sorted[first + r] = v;
     }
     __syncthreads();
+  }
+  if (!dense) return;
+  // (after the others: in one loop with them its registers cost every tile a sixth)
+  for (uint32_t a = blockIdx.x; a < na; a += gridDim.x) {
+    const uint32_t first = tile_start[a], tot = min(tile_total[a], n - min(first, n));
+    if (tot <= kSortStage) continue;
+    const size_t key = (size_t(act_tiles[a]) << kTileBits) + threadIdx.x;
+    const uint32_t cnt = cell_count[key], ex = cell_end[key] - cnt - first;
+    __syncthreads();
+    s_cur[threadIdx.x] = ex;
+    s_start[threadIdx.x] = ex;
+    if (threadIdx.x == 0u) {
+      s_start[kTileCells] = tot;
+      s_nbig = 0u;
+    }
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < tot; e += 4u * kSortThreads) {  // four loads in flight
+      typename E::T u[4];
+#pragma unroll
+      for (uint32_t r = 0; r < 4u; r++)
+        if (e + r * kSortThreads < tot) u[r] = bucket[first + e + r * kSortThreads];
+#pragma unroll
+      for (uint32_t r = 0; r < 4u; r++)
+        if (e + r * kSortThreads < tot) sorted[first + atomicAdd(&s_cur[E::cell(u[r])], 1u)] = E::index(u[r]);
+    }
+    __syncthreads();
+    // the wave's cells by the lanes that sort one, smallest first
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t below = (1ull << lane) - 1ull;
+    const uint64_t m4 = __ballot(cnt >= 2u && cnt <= 32u), m16 = __ballot(cnt > 32u && cnt <= 128u);
+    const uint64_t m64 = __ballot(cnt > 128u && cnt <= 512u);
+    const uint32_t e4 = uint32_t(__popcll(m4)), e16 = e4 + uint32_t(__popcll(m16)), e64 = e16 + uint32_t(__popcll(m64));
+    uint16_t* order = s_cell + (threadIdx.x & ~63u);
+    uint16_t* big = s_cell + kTileCells;
+    if (cnt > 512u) {
+      big[atomicAdd(&s_nbig, 1u)] = uint16_t(threadIdx.x);
+    } else if (cnt >= 2u) {
+      order[cnt <= 32u ? uint32_t(__popcll(m4 & below))
+                       : (cnt <= 128u ? e4 + uint32_t(__popcll(m16 & below)) : e16 + uint32_t(__popcll(m64 & below)))] =
+          uint16_t(threadIdx.x);
+    }
+    __syncthreads();
+    auto sort_cells = [&](auto lanes, uint32_t i, uint32_t stop) {
+      constexpr uint32_t G = decltype(lanes)::value;
+      for (; i < stop; i += 64u / G) {
+        const uint32_t at = i + lane / G;
+        const uint32_t c = at < stop ? order[at] : 0u, b = s_start[c];
+        group_sort_segment<G, 8>(sorted + first + b, at < stop ? s_start[c + 1u] - b : 0u);
+      }
+    };
+    sort_cells(std::integral_constant<uint32_t, 4u>{}, 0u, e4);
+    sort_cells(std::integral_constant<uint32_t, 16u>{}, e4, e16);
+    sort_cells(std::integral_constant<uint32_t, 64u>{}, e16, e64);
     const uint32_t nbig = s_nbig;
     for (uint32_t q = 0; q < nbig; q++) {
-      const uint32_t c = s_big[q], bs = first + s_start[c], bm = s_start[c + 1u] - s_start[c];
-      for (uint32_t e = threadIdx.x; e < bm; e += kSortThreads) s_idx[e] = sorted[bs + e];
-      __syncthreads();
-      for (uint32_t e = threadIdx.x; e < bm; e += kSortThreads) {
-        const uint32_t v = s_idx[e];
-        uint32_t r = 0;
-        for (uint32_t j = 0; j < bm; j++) r += s_idx[j] < v ? 1u : 0u;
-        sorted[bs + r] = v;
+      const uint32_t c = big[q], m = s_start[c + 1u] - s_start[c];
+      uint32_t* seg = sorted + first + s_start[c];
+      uint32_t P = 1u;
+      while (P < m) P <<= 1;
+      if (P > kSortStage) {
+        block_bitonic(seg, m, P);
+        continue;
       }
+      for (uint32_t e = threadIdx.x; e < P; e += kSortThreads) s_idx[e] = e < m ? seg[e] : 0xFFFFFFFFu;
+      __syncthreads();
+      block_bitonic(s_idx, P, P);
+      for (uint32_t e = threadIdx.x; e < m; e += kSortThreads) seg[e] = s_idx[e];
       __syncthreads();
     }
-    __syncthreads();
   }
 }
 
@@ -1840,12 +1861,12 @@ __global__ __launch_bounds__(1024) void k_bin_tiles(SubParams p, uint32_t* __res
     const uint32_t T = t0 + k;
     cnt[k] = 0u;
     if (k < c && T < nt) {
-      cnt[k] = tile_cnt[T];
+      cnt[k] = tile_cnt[tile_slot(T)];
       g = tile_geo<BATCH>(p, T);  // neighbours stay inside the tile's scene
       tile_coords(g, T, at3[k][0], at3[k][1], at3[k][2]);
       td[k] = int(g.tile_dim);
       s_occ[0][T] = cnt[k] ? 1 : 0;
-      if (cnt[k]) tile_cnt[T] = 0u;  // ready for the next count
+      if (cnt[k]) tile_cnt[tile_slot(T)] = 0u;  // ready for the next count
     }
   }
   // occupied in the 3x3x3 neighbourhood, axis by axis
@@ -1934,13 +1955,13 @@ __global__ __launch_bounds__(256) void k_bin_mark(SubParams p, float4* rec, cons
     int tx, ty, tz;
     tile_coords(g, T, tx, ty, tz);
     const int td = int(g.tile_dim);
-    cnt = tile_cnt[T];
+    cnt = tile_cnt[tile_slot(T)];
     uint32_t any = 0;
 #pragma unroll
     for (int o = 0; o < 27; o++) {  // all loads in flight together
       const int x = tx + o % 3 - 1, y = ty + (o / 3) % 3 - 1, z = tz + o / 9 - 1;
       const bool in = uint32_t(x) < uint32_t(td) && uint32_t(y) < uint32_t(td) && uint32_t(z) < uint32_t(td);
-      any |= in ? tile_cnt[tile_id(g, in ? x : tx, in ? y : ty, in ? z : tz)] : 0u;
+      any |= in ? tile_cnt[tile_slot(tile_id(g, in ? x : tx, in ? y : ty, in ? z : tz))] : 0u;
     }
     m = (cnt ? 1u : 0u) | (any ? 2u : 0u);
     tile_mark[T] = uint8_t(m);
@@ -2037,7 +2058,7 @@ __global__ __launch_bounds__(256) void k_bin_compact(const uint8_t* __restrict__
     tot.cls[0] = uint32_t(v[6]); tot.cls[1] = uint32_t(v[6] >> 32); tot.cls[2] = uint32_t(v[7]); tot.cls[3] = uint32_t(v[7] >> 32);
   }
   const uint32_t T = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t m = T < nt ? tile_mark[T] : 0u, cnt = (m & 1u) ? tile_cnt[T] : 0u;
+  const uint32_t m = T < nt ? tile_mark[T] : 0u, cnt = (m & 1u) ? tile_cnt[tile_slot(T)] : 0u;
   const uint32_t q = tile_class(cnt);
   const uint64_t own[3] = {uint64_t(m & 1u) | (uint64_t(m >> 1) << 32), uint64_t(cnt) | (uint64_t(tile_units(cnt)) << 32),
                            cnt ? uint64_t(1) << (16u * q) : uint64_t(0)};
@@ -2056,7 +2077,7 @@ __global__ __launch_bounds__(256) void k_bin_compact(const uint8_t* __restrict__
 #pragma unroll
       for (uint32_t k = 0; k < 4u; k++) at += k < q ? tot.cls[k] : (k == q ? pre.cls[k] : 0u);
       tile_order[at] = oa;
-      tile_cnt[T] = 0u;  // ready for the next count
+      tile_cnt[tile_slot(T)] = 0u;  // ready for the next count
     }
     if (m & 2u) node_tiles[uint32_t(l0 >> 32)] = T;
   }
@@ -2320,7 +2341,7 @@ static void launch_fb_entries(const DevState& d, const SubParams& p, float4* rec
 }
 
 void launch_clear_counts(const DevState& d, uint32_t n_tiles, hipStream_t s) {
-  k_zero<<<cdiv(n_tiles, 256), 256, 0, s>>>(d.tile_cnt, n_tiles);
+  k_zero<<<cdiv(tile_slots(n_tiles), 256), 256, 0, s>>>(d.tile_cnt, tile_slots(n_tiles));
 }
 
 void launch_bin(const DevState& d, const SubParams& p, uint32_t n_tiles, BinFrom from, hipStream_t s, Prof* pf) {

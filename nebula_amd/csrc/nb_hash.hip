@@ -301,51 +301,11 @@ __device__ __forceinline__ void sort_small(uint32_t* __restrict__ seg, uint32_t 
     if (k < cnt) seg[k] = v[k];
 }
 
-// ascending sort of 64 E values, E a lane, value e of lane l at place 64 e + l
-// (bitonic: a step of 64 or more pairs values of one lane)
-template <uint32_t E>
-__device__ __forceinline__ void wave_sort(uint32_t (&v)[E]) {
-  const uint32_t lane = threadIdx.x & 63u;
-#pragma unroll
-  for (uint32_t k = 2; k <= 64u * E; k <<= 1) {
-#pragma unroll
-    for (uint32_t j = k >> 1; j >= 1u; j >>= 1) {
-#pragma unroll
-      for (uint32_t e = 0; e < E; e++) {
-        const uint32_t at = 64u * e + lane;
-        const bool up = (at & k) == 0u;
-        if (j >= 64u) {
-          const uint32_t f = e ^ (j / 64u);
-          if (f > e) {
-            const uint32_t lo = min(v[e], v[f]), hi = max(v[e], v[f]);
-            v[e] = up ? lo : hi;
-            v[f] = up ? hi : lo;
-          }
-        } else {
-          const uint32_t o = uint32_t(__shfl_xor(int(v[e]), int(j)));
-          v[e] = up == ((at & j) == 0u) ? min(v[e], o) : max(v[e], o);
-        }
-      }
-    }
-  }
-}
-template <uint32_t E>
-__device__ __forceinline__ void wave_sort_cell(uint32_t* __restrict__ seg, uint32_t cnt) {
-  const uint32_t lane = threadIdx.x & 63u;
-  uint32_t v[E];
-#pragma unroll
-  for (uint32_t e = 0; e < E; e++) v[e] = 64u * e + lane < cnt ? seg[64u * e + lane] : 0xFFFFFFFFu;
-  wave_sort<E>(v);
-#pragma unroll
-  for (uint32_t e = 0; e < E; e++)
-    if (64u * e + lane < cnt) seg[64u * e + lane] = v[e];
-}
-
 // a crowded cell of up to kWaveSort particles, by its wave
 __device__ __forceinline__ void wave_sort_cell_of(uint32_t* __restrict__ seg, uint32_t cnt) {
-  if (cnt <= 64u) wave_sort_cell<1>(seg, cnt);
-  else if (cnt <= 256u) wave_sort_cell<4>(seg, cnt);
-  else wave_sort_cell<8>(seg, cnt);
+  if (cnt <= 64u) nb::group_sort_segment<64, 1>(seg, cnt);
+  else if (cnt <= 256u) nb::group_sort_segment<64, 4>(seg, cnt);
+  else nb::group_sort_segment<64, 8>(seg, cnt);
 }
 
 // Without a list the crowded cells are found from `sorted` itself: a cell of more than
@@ -446,38 +406,6 @@ __global__ __launch_bounds__(kThreads) void k_hash_stabilize(Geo g, const float4
   }
 }
 
-// Bitonic sort (ascending) of a[0, cnt) over the padded length P (a power of
-// two >= cnt), every merge in its "flip" form so that all compare-exchanges put
-// the smaller value first: partners at or past cnt hold +inf and are skipped.
-// Block-cooperative; a is LDS or global memory of this block alone.
-__device__ __forceinline__ void cas(uint32_t* a, uint32_t i, uint32_t l, uint32_t cnt) {
-  if (l < cnt) {
-    const uint32_t x = a[i], y = a[l];
-    if (x > y) {
-      a[i] = y;
-      a[l] = x;
-    }
-  }
-}
-__device__ void block_bitonic(uint32_t* a, uint32_t cnt, uint32_t P) {
-  const uint32_t half = P >> 1;
-  for (uint32_t k = 2; k <= P; k <<= 1) {
-    const uint32_t hk = k >> 1;
-    for (uint32_t t = threadIdx.x; t < half; t += blockDim.x) {
-      const uint32_t b = (t / hk) * k, o = t % hk;
-      cas(a, b + o, b + k - 1u - o, cnt);
-    }
-    __syncthreads();
-    for (uint32_t j = k >> 2; j >= 1u; j >>= 1) {
-      for (uint32_t t = threadIdx.x; t < half; t += blockDim.x) {
-        const uint32_t i = (t / j) * (2u * j) + (t % j);
-        cas(a, i, i + j, cnt);
-      }
-      __syncthreads();
-    }
-  }
-}
-
 __device__ void sort_crowded(uint32_t* __restrict__ sorted, const uint32_t* __restrict__ cell_count,
                              const uint32_t* __restrict__ cell_off, uint32_t c, uint32_t* s_buf) {
   const uint32_t cnt = cell_count[c];
@@ -487,10 +415,10 @@ __device__ void sort_crowded(uint32_t* __restrict__ sorted, const uint32_t* __re
   if (cnt <= kLdsSort) {
     for (uint32_t k = threadIdx.x; k < P; k += blockDim.x) s_buf[k] = k < cnt ? seg[k] : 0xFFFFFFFFu;
     __syncthreads();
-    block_bitonic(s_buf, P, P);
+    nb::block_bitonic(s_buf, P, P);
     for (uint32_t k = threadIdx.x; k < cnt; k += blockDim.x) seg[k] = s_buf[k];
   } else {
-    block_bitonic(seg, cnt, P);
+    nb::block_bitonic(seg, cnt, P);
   }
   __syncthreads();
 }

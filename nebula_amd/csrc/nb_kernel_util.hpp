@@ -95,6 +95,75 @@ __device__ __forceinline__ void block_exclusive_scan3(const uint64_t (&v)[3], ui
   }
 }
 
+// Ascending sort of seg[0, cnt), cnt <= G E, by G neighbouring lanes (a power of two),
+// E registers each: value e in register e / G of the group's lane e % G.  Bitonic: a step
+// of G or more pairs values of one lane.  All groups of a wave call it together (cnt 0:
+// none).
+template <uint32_t G, uint32_t E>
+__device__ __forceinline__ void group_sort_segment(uint32_t* seg, uint32_t cnt) {
+  const uint32_t lane = threadIdx.x & (G - 1u);
+  uint32_t v[E];
+#pragma unroll
+  for (uint32_t e = 0; e < E; e++) v[e] = G * e + lane < cnt ? seg[G * e + lane] : 0xFFFFFFFFu;
+#pragma unroll
+  for (uint32_t k = 2; k <= G * E; k <<= 1) {
+#pragma unroll
+    for (uint32_t j = k >> 1; j >= 1u; j >>= 1) {
+#pragma unroll
+      for (uint32_t e = 0; e < E; e++) {
+        const uint32_t at = G * e + lane;
+        const bool up = (at & k) == 0u;
+        if (j >= G) {
+          const uint32_t f = e ^ (j / G);
+          if (f > e) {
+            const uint32_t lo = min(v[e], v[f]), hi = max(v[e], v[f]);
+            v[e] = up ? lo : hi;
+            v[f] = up ? hi : lo;
+          }
+        } else {
+          const uint32_t o = uint32_t(__shfl_xor(int(v[e]), int(j)));
+          v[e] = up == ((at & j) == 0u) ? min(v[e], o) : max(v[e], o);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (uint32_t e = 0; e < E; e++)
+    if (G * e + lane < cnt) seg[G * e + lane] = v[e];
+}
+
+// Bitonic sort (ascending) of a[0, cnt) over the padded length P (a power of
+// two >= cnt), every merge in its "flip" form so that all compare-exchanges put
+// the smaller value first: partners at or past cnt hold +inf and are skipped.
+// Block-cooperative; a is LDS or global memory of this block alone.
+__device__ __forceinline__ void compare_exchange(uint32_t* a, uint32_t i, uint32_t l, uint32_t cnt) {
+  if (l < cnt) {
+    const uint32_t x = a[i], y = a[l];
+    if (x > y) {
+      a[i] = y;
+      a[l] = x;
+    }
+  }
+}
+__device__ inline void block_bitonic(uint32_t* a, uint32_t cnt, uint32_t P) {
+  const uint32_t half = P >> 1;
+  for (uint32_t k = 2; k <= P; k <<= 1) {
+    const uint32_t hk = k >> 1;
+    for (uint32_t t = threadIdx.x; t < half; t += blockDim.x) {
+      const uint32_t b = (t / hk) * k, o = t % hk;
+      compare_exchange(a, b + o, b + k - 1u - o, cnt);
+    }
+    __syncthreads();
+    for (uint32_t j = k >> 2; j >= 1u; j >>= 1) {
+      for (uint32_t t = threadIdx.x; t < half; t += blockDim.x) {
+        const uint32_t i = (t / j) * (2u * j) + (t % j);
+        compare_exchange(a, i, i + j, cnt);
+      }
+      __syncthreads();
+    }
+  }
+}
+
 // Workgroups are dealt to the 8 XCDs (each with its own L2) round-robin by
 // id.  Block b is given chunk xcd_chunk(b, nb) of the work, so that each XCD
 // walks one contiguous eighth of the chunks: neighbouring particles, and the
