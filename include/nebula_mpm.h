@@ -442,12 +442,16 @@ int nb_mpm_set_grid(nb_mpm* h, const float* mom4, const float* mass, const float
 /* ---- measurement ----
  * Run n substeps of dt_sub, recording HIP events around every kernel launch on
  * the engine's stream.  kernel_ms[i] receives the summed duration of kernel i,
- * names are written (comma separated) into names (capacity names_cap). */
+ * names are written (comma separated) into names (capacity names_cap).
+ * The FP64 fallback's work on what G2P queued (g2p_fb) is launched by itself
+ * here, before the next substep's bin and after the last substep; outside this
+ * call it runs within a launch of the bin, beside its work, so the sum of the
+ * kernels is a little more than a substep takes. */
 int nb_mpm_profile_substeps(nb_mpm* h, float dt_sub, uint32_t n, float* kernel_ms, uint32_t kernel_cap,
                             uint32_t* n_kernels, char* names, uint32_t names_cap);
 /* Launches of each kernel in the last nb_mpm_profile_substeps (same order as
- * its names): a call's substeps but the last run the grid update inside G2P
- * (g2p_grid), the last one runs grid_update and g2p. */
+ * its names).  With nb_mpm_set_fused_g2p a call's substeps but the last run the
+ * grid update inside G2P (g2p_grid), the last one runs grid_update and g2p. */
 int nb_mpm_profile_calls(const nb_mpm* h, uint32_t* calls, uint32_t cap);
 /* Calibration for HBM byte counters: copies `bytes` (rounded down to 16) from
  * one scratch buffer to another with a plain float4 copy kernel (k_copy),

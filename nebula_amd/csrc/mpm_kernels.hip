@@ -2347,6 +2347,15 @@ void launch_clear_counts(const DevState& d, uint32_t n_tiles, hipStream_t s) {
 void launch_bin(const DevState& d, const SubParams& p, uint32_t n_tiles, BinFrom from, hipStream_t s, Prof* pf) {
   const uint32_t tg = tile_grid(n_tiles, p.tile_blocks);
   const bool batch = p.n_scenes > 0;
+  // The fallback's queue of the G2P before.  Large cubes: beside k_bin_mark.  Small
+  // ones: beside the scatter, while that is short (262,144 particles: 14.7 us together,
+  // 5 + 14 apart); beyond 2^20 particles its registers would slow the scatter (4.19 M:
+  // 39 against 20 + 16).  By itself when timed, to be booked under its own name.
+  const bool small = n_tiles <= kSmallTiles, apart = pf != nullptr || (small && p.n > (1u << 20));
+  if (apart && p.svd_fp64) {
+    ProfScope ps(pf, 9, s);
+    launch_fb_entries(d, p, d.rec, s);
+  }
   if (from != BinFrom::COUNTED) {
     ProfScope ps(pf, 0, s);
     const uint32_t nb = cdiv(p.n, 256);
@@ -2359,21 +2368,21 @@ void launch_bin(const DevState& d, const SubParams& p, uint32_t n_tiles, BinFrom
   }
   {
     ProfScope ps(pf, 1, s);
-    if (n_tiles <= kSmallTiles) {
+    if (small) {
 #define NB_TILES(BT)                                                                                             \
   k_bin_tiles<BT><<<1, 1024, 0, s>>>(p, d.tile_cnt, d.tile_act, d.act_tiles, d.node_tiles, d.tile_total,         \
                                      d.tile_start, d.tile_order, d.counters, d.units, n_tiles)
       if (batch) NB_TILES(true); else NB_TILES(false);
 #undef NB_TILES
     } else {
-      const uint32_t tb = cdiv(n_tiles, 256), g = tb + fb_blocks(p, 256);
+      const uint32_t tb = cdiv(n_tiles, 256), g = tb + (apart ? 0u : fb_blocks(p, 256));
       if (batch)
         k_bin_mark<true><<<g, 256, 0, s>>>(p, d.rec, d.materials, d.tile_cnt, d.tile_mark, d.tile_sums, n_tiles, tb);
       else
         k_bin_mark<false><<<g, 256, 0, s>>>(p, d.rec, d.materials, d.tile_cnt, d.tile_mark, d.tile_sums, n_tiles, tb);
     }
   }
-  if (n_tiles > kSmallTiles) {
+  if (!small) {
     ProfScope ps(pf, 2, s);
     const uint32_t tb = cdiv(n_tiles, 256);
 #define NB_COMPACT(SC)                                                                                            \
@@ -2389,12 +2398,7 @@ void launch_bin(const DevState& d, const SubParams& p, uint32_t n_tiles, BinFrom
   }
   {
     ProfScope ps(pf, 3, s);
-    // small cubes: the fallback's queue beside the scatter, while that is
-    // short (262,144 particles: 14.7 us together, 5 + 14 apart); beyond 2^20
-    // particles its registers would slow the scatter (4.19 M: 39 against 20 + 16)
-    const bool apart = p.n > (1u << 20);
-    const uint32_t nb = cdiv(p.n, 256), fb = n_tiles <= kSmallTiles && !apart ? fb_blocks(p, 256) : 0u;
-    if (n_tiles <= kSmallTiles && apart) launch_fb_entries(d, p, d.rec, s);
+    const uint32_t nb = cdiv(p.n, 256), fb = small && !apart ? fb_blocks(p, 256) : 0u;
 #define NB_SCATTER_FB(PK, BT)                                                                                   \
   k_bin_scatter_fb<PK, BT><<<nb + fb, 256, 0, s>>>(p, d.rec, d.materials, d.keys, d.rank, d.tile_act, d.tile_start, \
                                                    d.bucket, fb)
