@@ -202,7 +202,12 @@ void nb_mpm_config_default(nb_mpm_config* cfg);
 void nb_mpm_knobs_default(nb_mpm_knobs* knobs);
 
 /* MPMEngine::init (src/engine/MPMEngine.cpp:34-156).  hip_stream: a hipStream_t
- * to enqueue on, or NULL for an engine-owned stream of default priority. */
+ * to enqueue on, or NULL for an engine-owned stream of default priority.
+ * Device memory: 356 B per particle of capacity and 448 B more for up to 262,144
+ * of them (the work items of small scenes; a batch of more than 16 scenes or
+ * 262,144 particles, which never takes them, has none), 42 B per cell of the
+ * grid's power-of-two cube and 16 KB per tile of 8^3 cells (per particle, where
+ * there are fewer). */
 int nb_mpm_create(const nb_mpm_config* cfg, void* hip_stream, nb_mpm** out);
 /* MPMEngine::cleanup (src/engine/MPMEngine.cpp:160-163). */
 int nb_mpm_destroy(nb_mpm* h);

@@ -748,11 +748,16 @@ int engine_alloc(nb_mpm* h, void* hip_stream) {
   c.add(&d.tile_order, h->NT);
   c.add(&d.counters, CNT_SLOTS);
   c.add(&d.partial, size_t(h->cap_tiles) * kBoxNodes);
-  d.item_cap = std::min(h->cap, kItemParticles);
-  c.add(&d.items, d.item_cap);
-  c.add(&d.cell_item, cells);
-  c.add(&d.tile_items, h->NT);
-  c.add(&d.item_sum, size_t(27) * d.item_cap);
+  // the buffers of P2G's items and the adjoint's cells, unless the engine can never take
+  // those forms (a batch's particle count is fixed)
+  const bool by_item = !h->batch() || (h->n_scenes <= kItemScenes && h->cap <= kItemParticles);
+  d.item_cap = by_item ? std::min(h->cap, kItemParticles) : 0u;
+  if (by_item) {
+    c.add(&d.items, d.item_cap);
+    c.add(&d.cell_item, cells);
+    c.add(&d.tile_items, h->NT);
+    c.add(&d.item_sum, size_t(27) * d.item_cap);
+  }
   c.add(&d.grid_node, cells);
   c.add(&d.grid_old, cells);
   c.add(&d.materials, h->max_materials());

@@ -202,7 +202,7 @@ struct DevState {
   uint16_t* cell_item;    // NT*512: a cell's first item among its tile's | items << 11
   uint32_t* tile_items;   // NT: items of an occupied tile | chunk layers << 16
   float4* item_sum;       // 27 * item_cap: sums per offset and item (in the adjoint: per offset and cell)
-  uint32_t item_cap;      // particles the item buffers hold
+  uint32_t item_cap;      // particles the item buffers hold; 0: there are none
   uint32_t item_pad;
   float4* grid_node;      // NT*512
   float4* grid_old;       // NT*512
