@@ -1439,29 +1439,39 @@ int nb_mpm_get_bins(nb_mpm* h, uint32_t* keys, uint32_t* sorted, uint32_t* cell_
   if (h->batch()) return fail(NB_ERR_UNSUPPORTED, "%s: not available on a batch of scenes", __func__);
   if (!h->bins_valid) return fail(NB_ERR_STATE, "no bins: call nb_mpm_run_bin first");
   const uint32_t n = h->n_live;
-  int rc = NB_OK;
-  if (keys && n) rc = download(h, keys, h->d.keys, size_t(n) * 4);
-  if (rc == NB_OK && sorted && n) rc = download(h, sorted, h->d.sorted, size_t(n) * 4);
-  if (rc != NB_OK) return rc;
-  if (cell_count || cell_end) {
-    std::vector<uint32_t> cnt(h->NC), dev_end(h->NC);
+  hipError_t e = hipSuccess;
+  auto copy = [&](void* dst, const void* src, size_t count) {
+    if (e == hipSuccess && dst && n) e = hipMemcpyAsync(dst, src, count * 4, hipMemcpyDefault, h->stream);
+  };
+  const bool cells = cell_count || cell_end;
+  std::vector<uint32_t> own(cells && !cell_count ? h->NC : 0);
+  std::vector<int32_t> act(cells ? h->NT : 0);
+  uint32_t* cnt = cell_count ? cell_count : own.data();
+  copy(keys, h->d.keys, n);
+  copy(sorted, h->d.sorted, n);
+  if (cells) {
+    copy(cnt, h->d.cell_count, h->NC);
+    copy(cell_end, h->d.cell_end, h->NC);
+    copy(act.data(), h->d.tile_act, h->NT);
+  }
+  const hipError_t waited = hipStreamSynchronize(h->stream);
+  if (e == hipSuccess) e = waited;
+  if (e != hipSuccess) return fail(NB_ERR_HIP, "nb_mpm_get_bins: copy failed: %s", hipGetErrorString(e));
+  if (cells) {
     if (n) {
-      if ((rc = download(h, cnt.data(), h->d.cell_count, size_t(h->NC) * 4)) != NB_OK) return rc;
-      if ((rc = download(h, dev_end.data(), h->d.cell_end, size_t(h->NC) * 4)) != NB_OK) return rc;
       // the device's counts are those of the occupied tiles only
-      std::vector<int32_t> act(h->NT);
-      if ((rc = download(h, act.data(), h->d.tile_act, size_t(h->NT) * 4)) != NB_OK) return rc;
-      for (uint32_t c = 0; c < h->NC; c++)
-        if (act[c >> kTileBits] < 0) cnt[c] = 0u;
+      for (uint32_t t = 0; t < h->NT; t++)
+        if (act[t] < 0) std::fill(cnt + (t << kTileBits), cnt + std::min((t + 1u) << kTileBits, h->NC), 0u);
+    } else {
+      std::fill(cnt, cnt + h->NC, 0u);
     }
-    if (cell_count) std::memcpy(cell_count, cnt.data(), size_t(h->NC) * 4);
     if (cell_end) {
       // dense END offsets: occupied cells carry the device value; an empty cell
       // holds the running prefix (the reference's cellOffset for count 0)
       uint32_t acc = 0;
       for (uint32_t c = 0; c < h->NC; c++) {
         acc += cnt[c];
-        cell_end[c] = cnt[c] ? dev_end[c] : acc;
+        if (!cnt[c]) cell_end[c] = acc;
       }
     }
   }
