@@ -2090,7 +2090,7 @@ __global__ __launch_bounds__(256) void k_bin_compact(const uint8_t* __restrict__
 
 // Grid update and G2P fused, one block per work unit: a unit is up to
 // kG2PUnit particles of one occupied tile (a tile's particles are one
-// contiguous range of the bin order; k_bin_tile_offsets lists the units).
+// contiguous range of the bin order; the bin's tile pass lists the units).
 // The block builds the tile's 10^3 node box in LDS from the partials (the
 // same sums and node update as k_grid_tiles, bit for bit), stores each node's
 // G2P view (velocity, or zero for a node that does not take part, and FLIP's
@@ -2559,8 +2559,8 @@ void launch_g2p(const DevState& d, const SubParams& p, bool use_sorted, bool cou
 // what rounding can take from the distance that would be measured (mesh_error),
 // so a triangle dropped is neither a minimum nor a tie: values and signs have the
 // bits of the pass over all triangles.  On 128^3 cells and 3,360 triangles a cell
-// measures about 26 distances instead of 3,360 and the build takes 0.67 ms
-// instead of 10.1 (VALU-bound; 0.98 with the wave's bound alone).
+// measures about 26 distances instead of 3,360 and the search takes 0.64 ms
+// where the pass over all takes 10.1 (VALU-bound; 0.98 with the wave's bound alone).
 // ---------------------------------------------------------------------------
 // The closest point of triangle t (normal, v0, v1, v2) to p.  EXACT adds the
 // region of the edge v1-v2 that closestPtOnTriangle leaves out.
